@@ -191,6 +191,12 @@ int k3k_gemv_f32(float *y, const float *x, const float *W, int in, int out, int 
                  void *stream);
 int k3k_gemv_bf16(float *y, const float *x, const uint16_t *W, int in, int out, int ntok,
                   int ldy, void *stream);
+/* The same for two tokens and more on the matrix cores (k3_tok.hip): W bf16 (bf16 1) or fp32,
+ * where k3k_tok_ok holds (in % 8 == 0, x and W 16-byte aligned). k3k_gemv_* send their calls
+ * there. */
+int k3k_tok_ok(const float *x, const void *W, int in, int ntok);
+int k3k_tok_gemm(float *y, const float *x, const void *W, int bf16, int in, int out, int ntok, int ldy,
+                 void *stream);
 int k3k_gemv_q8(float *y, const float *x, const void *W, int in, int out, int ntok, int ldy,
                 void *stream);
 

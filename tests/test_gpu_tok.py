@@ -1,0 +1,62 @@
+# SPDX-License-Identifier: Apache-2.0
+"""Products of several tokens on the matrix cores, fp32-accurate (csrc/k3_tok.hip), at the
+edges of their tiles: against numpy's fp64 product of the same values. The 2-norm error of
+fp32 sums of exact products is 2e-7 to 4e-7 at these widths; activations cut to two bf16
+terms would show 2.6e-6, so 1e-6 tells a lost term."""
+import numpy as np
+import pytest
+
+from test_gpu_dense import dev_matmul, say
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("bf16", [True, False])
+@pytest.mark.parametrize("T,inn,out", [(2, 8, 1), (3, 7168, 12288), (16, 24, 17), (17, 64, 16), (33, 1000, 129), (37, 7168, 3584),
+                                       (64, 104, 4100), (65, 264, 300), (130, 2056, 1031), (256, 512, 4099),
+                                       (700, 96, 70)])
+def test_tok_matmul_edges(gpu, k3, bf16, T, inn, out):
+    say(f"case: {T} tokens {inn} -> {out} bf16={bf16}")
+    Wb = k3.gen_bf16_normal(inn * out, 5 + T, 0.0, 0.02).reshape(out, inn)
+    W = (Wb.astype(np.uint32) << 16).view(np.float32)
+    if not bf16:
+        W = (W * np.float32(1.0 + 2.0**-13)).astype(np.float32)
+    X = k3.gen_normal(T * inn, 6 + T).reshape(T, inn) * (np.float32(10.0) ** (np.arange(T) % 7 - 3))[:, None].astype(np.float32)
+    Y = dev_matmul(gpu, X, Wb if bf16 else W, bf16=bf16).astype(np.float64)
+    want = X.astype(np.float64) @ W.astype(np.float64).T
+    for t in range(T):
+        assert np.linalg.norm(Y[t] - want[t]) <= 1e-6 * np.linalg.norm(np.abs(X[t].astype(np.float64)) @ np.abs(W.T.astype(np.float64))), t
+    rel = np.linalg.norm(Y - want, axis=1) / np.linalg.norm(want, axis=1)
+    if out >= 16:
+        assert rel.max() <= 1e-6
+
+
+@pytest.mark.parametrize("bf16", [True, False])
+def test_tok_matmul_nonfinite(gpu, k3, bf16):
+    """Infinities and NaN in x and W, the largest finite x, subnormal x: what plain products
+    and sums give, element by element."""
+    T, inn, out = 20, 136, 40
+    say(f"case: non-finite operands bf16={bf16}")
+    Wb = k3.gen_bf16_normal(inn * out, 91, 0.0, 1.0).reshape(out, inn)
+    Wb[3, 7], Wb[4, 9], Wb[5, 100] = 0x7F80, 0xFF80, 0x7FC0          # +inf, -inf, NaN
+    Wb[6, :] = 0
+    W = (Wb.astype(np.uint32) << 16).view(np.float32)
+    X = k3.gen_normal(T * inn, 92).reshape(T, inn)
+    X[:, 7], X[:, 9] = 2.0, 0.0                                      # inf * 2 (one term only), inf * 0
+    X[1, 11], X[2, 13], X[3, 15] = np.inf, -np.inf, np.nan
+    X[4, 17] = np.finfo(np.float32).max
+    X[5, :] = np.float32(1e-41)
+    W[:, 17] = np.where(np.isfinite(W[:, 17]), np.clip(W[:, 17], -0.5, 0.5), W[:, 17])
+    Wb[:, 17] = (W[:, 17].view(np.uint32) >> 16).astype(np.uint16)
+    W = (Wb.astype(np.uint32) << 16).view(np.float32)
+    Y = dev_matmul(gpu, X, Wb if bf16 else W, bf16=bf16)
+    with np.errstate(invalid="ignore"):
+        want = np.array([[np.sum(X[t].astype(np.float64) * W[o].astype(np.float64)) for o in range(out)] for t in range(T)])
+    assert np.array_equal(np.isnan(Y), np.isnan(want))
+    inf = np.isinf(want)
+    assert np.array_equal(Y[inf], want[inf].astype(np.float32)) and not np.isinf(Y[~inf]).any()
+    fin = np.isfinite(want)
+    bound = np.abs(np.nan_to_num(X, posinf=0, neginf=0)).astype(np.float64) @ np.abs(np.nan_to_num(W, posinf=0, neginf=0)).astype(np.float64).T
+    # the cut's last term ends at 2^-133; fp32 products of subnormals at 2^-149
+    tiny = 2.0**-133 * np.abs(np.nan_to_num(W, posinf=0, neginf=0)).astype(np.float64).sum(1)[None, :] + inn * 2.0**-149
+    assert (np.abs(Y - want)[fin] <= (1e-6 * bound + tiny)[fin]).all()
