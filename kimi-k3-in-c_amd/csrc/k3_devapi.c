@@ -337,44 +337,57 @@ typedef struct {
 } MoeWs;
 
 /* Tokens per expert pass. The LDS-staged expert kernels need both matrix widths to be
- * multiples of 512: passes of 8 tokens, or of 32 (two MFMA column blocks) when the
- * activations are single bf16 terms and the batch averages at least 8 tokens per expert
- * (prefill). Other shapes run the register-fed kernel (16, row-major bank only). */
-/* One-term (prefill) activations at 8-32 tokens per expert on average on a tiled bank: two
- * pass lists (below). */
-static int moe_two_lists(int T, int n_experts, int topk, int prec, int layout)
+ * multiples of 512: passes of 8 tokens, or more (moe_pass_tok) for larger batches. Other shapes
+ * run the register-fed kernel (16, row-major bank only).
+ *
+ * Two pass lists on a tiled bank: one-term (prefill) activations at 8-32 tokens per expert on
+ * average, two-term ones from 5. There 7 % of the experts of a uniform routing hold more than
+ * 8 tokens and would stream their weights again; with fewer tokens the second list's two
+ * launches and its fork, about 15 us, cost more than they save (64 tokens of the 128-expert
+ * layer, 4 per expert: 266 us with one list, 282 with two). The prefill kernel addresses both
+ * activation terms from one base, below 2 GiB. */
+static int moe_two_lists(int T, int hidden, int inter, int n_experts, int topk, int prec, int layout)
 {
-    return prec == 1 && layout == K3D_LAYOUT_TILED && (long)T * topk >= 8L * n_experts &&
-           (long)T * topk < 32L * n_experts;
+    const long N = (long)T * topk;
+    if (layout != K3D_LAYOUT_TILED || hidden % 512 || inter % 512) return 0;
+    if (prec == 1) return N >= 8L * n_experts && N < 32L * n_experts;
+    return N >= 5L * n_experts && ((long long)N * inter + 256) * 4 < 0x7fff0000ll &&
+           ((long long)T * hidden + 256) * 4 < 0x7fff0000ll;
 }
 
-/* Tokens per expert pass. 8 for decode (fp32-accurate, weight streaming), 16 when the
- * widths are not multiples of 512; one-term (prefill) activations take, for a tiled bank, 8
- * from 8 tokens per expert on average (with the second list), 48 from 32 and 96 from 64;
- * for a row-major bank 32 from 8. Sizing: a row-major bank's first list has at most N / 32
- * passes beyond one per expert; a tiled bank's at most N / 8 where there is no second list,
- * and one per expert where there is (its experts hold at most 8 assignments). */
+/* Tokens per expert pass (of the first list). 8 for decode (fp32-accurate, weight streaming)
+ * and where there is a second list, 16 when the widths are not multiples of 512; one-term
+ * (prefill) activations take, for a tiled bank, 48 from 32 tokens per expert on average and 96
+ * from 64; for a row-major bank 32 from 8. Sizing: a row-major bank's first list has at most
+ * N / 32 (or N / 8) passes beyond one per expert; a tiled bank's at most N / 8 where there is
+ * no second list, and one per expert where there is (its experts hold at most 8 assignments). */
 static int moe_pass_tok(int T, int hidden, int inter, int n_experts, int topk, int prec, int layout)
 {
     if (hidden % 512 || inter % 512) return 16;
     if (prec == 1 && layout == K3D_LAYOUT_TILED && (long)T * topk >= 64L * n_experts) return 96;
     if (prec == 1 && layout == K3D_LAYOUT_TILED && (long)T * topk >= 32L * n_experts) return 48;
-    if (moe_two_lists(T, n_experts, topk, prec, layout)) return 8;
+    if (moe_two_lists(T, hidden, inter, n_experts, topk, prec, layout)) return 8;
     if (prec == 1 && (long)T * topk >= 8L * n_experts) return 32;
     return 8;
 }
 
 /* The second pass list: where moe_two_lists holds, the experts holding more than pass_tok
  * (8) assignments -- all but the coldest, and the hot ones of a skewed routing -- take the
- * prefill kernel's 96-token passes, so their weights stream once per 96 tokens, and the
- * rest one 8-token pass each on the streaming kernel. (Config 4, 512 tokens with skewed
- * routing: 309 experts of at most 32 assignments in 32-token passes and 21 hot ones in the
- * second list took 1.47 ms for gate/up + down; 282 experts of at most 8 in 8-token passes
- * and 48 in the second list take 1.40 ms.) */
-#define MOE_PASS_TOK2 96
-static int moe_pass_tok2(int T, int n_experts, int topk, int prec, int layout)
+ * prefill kernel's passes of 96 tokens, so their weights stream once per pass, and the rest one
+ * 8-token pass each on the streaming kernel. With two activation terms the passes are of 48
+ * tokens, or of 32 below 16 tokens per expert on average, where few passes fill a longer one
+ * and the shorter one's double stages keep twice the weights in flight (512 tokens of the
+ * 384-expert layer, skewed: 1.82 ms with 48, 1.70 with 32; 333 tokens through k3_moe_prefill
+ * at 896 experts: 4.48 and 4.31). 16-token streaming passes for the first list instead were
+ * slower (512 tokens of 896 experts 3.35 against 3.15 ms). (Config 4, 512
+ * tokens with skewed routing: 309 experts of at most 32 assignments in 32-token passes and 21
+ * hot ones in the second list took 1.47 ms for gate/up + down; 282 experts of at most 8 in
+ * 8-token passes and 48 in the second list take 1.40 ms.) */
+static int moe_pass_tok2(int T, int hidden, int inter, int n_experts, int topk, int prec, int layout)
 {
-    return moe_two_lists(T, n_experts, topk, prec, layout) ? MOE_PASS_TOK2 : 0;
+    if (!moe_two_lists(T, hidden, inter, n_experts, topk, prec, layout)) return 0;
+    if (prec == 1) return 96;
+    return (long)T * topk < 16L * n_experts ? 32 : 48;
 }
 
 /* The decode path (k3k_mx_decode): at most 16 assignments, widths multiples of 512 up to
@@ -392,7 +405,7 @@ static size_t moe_layout(Carve *c, MoeWs *w, int T, int hidden, int inter, int n
     const int maxjobs = (int)(N < (size_t)n_experts ? N : (size_t)n_experts);
     w->max_passes = maxjobs + (int)(N / (size_t)moe_pass_tok(T, hidden, inter, n_experts, topk, prec,
                                                                 K3D_LAYOUT_ROWS)) + 1;
-    if (!moe_two_lists(T, n_experts, topk, prec, K3D_LAYOUT_TILED)) {
+    if (!moe_two_lists(T, hidden, inter, n_experts, topk, prec, K3D_LAYOUT_TILED)) {
         const int pt = moe_pass_tok(T, hidden, inter, n_experts, topk, prec, K3D_LAYOUT_TILED);
         const int mp = maxjobs + (int)(N / (size_t)pt) + 1;
         if (mp > w->max_passes) w->max_passes = mp;
@@ -408,11 +421,12 @@ static size_t moe_layout(Carve *c, MoeWs *w, int T, int hidden, int inter, int n
     w->job_cnt = (int *)take(c, (size_t)maxjobs * 4);
     w->pass_job = (int *)take(c, (size_t)w->max_passes * 4);
     w->pass_tp = (int *)take(c, (size_t)w->max_passes * 4);
-    /* second list (one-term activations): experts of more than 8 assignments, each pass of
-     * up to 96 tokens -- at most N / 96 full passes plus one per such expert */
-    w->max_passes2 = prec == 1 ? (int)(N / MOE_PASS_TOK2 + N / 9 + 2) : 0;
-    w->pass_job2 = prec == 1 ? (int *)take(c, (size_t)w->max_passes2 * 4) : NULL;
-    w->pass_tp2 = prec == 1 ? (int *)take(c, (size_t)w->max_passes2 * 4) : NULL;
+    /* second list: experts of more than 8 assignments, each pass of up to 96 (48, 32) tokens -- at
+     * most N / that full passes plus one per such expert */
+    const int pt2 = moe_pass_tok2(T, hidden, inter, n_experts, topk, prec, K3D_LAYOUT_TILED);
+    w->max_passes2 = pt2 ? (int)(N / (size_t)pt2 + N / 9 + 2) : 0;
+    w->pass_job2 = pt2 ? (int *)take(c, (size_t)w->max_passes2 * 4) : NULL;
+    w->pass_tp2 = pt2 ? (int *)take(c, (size_t)w->max_passes2 * 4) : NULL;
     w->counts = (int *)take(c, (size_t)(4 + K3K_QUEUE_INTS) * 4);
     {
         const size_t gs = k3k_gather_scratch(T, topk, n_experts);
@@ -552,7 +566,7 @@ static int moe_experts_ws(float *out, const int *idx, const float *wt, const flo
     }
     /* (the routed layer runs the split beside its router, on the side stream) */
     if (!x_split && k3k_split_bf16(w->xhi, w->xlo, x, (size_t)T * hidden, stream)) return fail("split");
-    const int pass_tok2 = moe_pass_tok2(T, n_experts, topk, prec, layout);
+    const int pass_tok2 = moe_pass_tok2(T, hidden, inter, n_experts, topk, prec, layout);
     /* (gathered: the router's final kernel has run the gather) */
     if (!gathered &&
         k3k_gather(offsets, perm, w->job_expert, w->job_off, w->job_cnt, w->pass_job, w->pass_tp,
@@ -599,7 +613,7 @@ static int moe_experts_ws(float *out, const int *idx, const float *wt, const flo
     a.queue = w->counts + 4;
     a2.queue = w->counts + 4 + 2 * K3K_NXCD_Q;
     if (k3k_mx_gemm(K3K_MX_GATEUP, &a, stream)) return fail("mx_gemm gateup");
-    if (pass_tok2 && k3k_mx_gemm(K3K_MX_GATEUP, &a2, side)) return fail("mx_gemm gateup (96)");
+    if (pass_tok2 && k3k_mx_gemm(K3K_MX_GATEUP, &a2, side)) return fail("mx_gemm gateup (second list)");
     k3k_prof_mark(stream, K3D_STAGE_GATEUP);
     /* down: K = inter, rows = hidden, activations are the assignments */
     a.xhi = w->ahi;
@@ -618,7 +632,7 @@ static int moe_experts_ws(float *out, const int *idx, const float *wt, const flo
         a2.K = a.K;
         a2.n_xrows = a.n_xrows;
         a2.queue = w->counts + 4 + 3 * K3K_NXCD_Q;
-        if (k3k_mx_gemm(K3K_MX_DOWN, &a2, side)) return fail("mx_gemm down (96)");
+        if (k3k_mx_gemm(K3K_MX_DOWN, &a2, side)) return fail("mx_gemm down (second list)");
         if (k3k_join(stream)) return fail("join");
     }
     k3k_prof_mark(stream, K3D_STAGE_DOWN);
@@ -709,7 +723,7 @@ int k3d_moe_routed(float *out, int *idx, float *wt, const float *x, int T, const
         ga.bank = bank;
         ga.topk = topk;
         ga.pass_tok = pass_tok;
-        ga.pass_tok2 = moe_pass_tok2(T, n_experts, topk, prec, layout);
+        ga.pass_tok2 = moe_pass_tok2(T, hidden, inter, n_experts, topk, prec, layout);
         ga.ctr = r.ctr;
     }
     rc = router_run(idx, wt, x, T, router_w, bias, hidden, n_experts, topk, renorm, routed_scale,

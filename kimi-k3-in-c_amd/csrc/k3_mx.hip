@@ -1433,12 +1433,19 @@ int launch_moe(const K3kMxArgs *a, int grid, hipStream_t st)
     return 0;
 }
 
-/* ---- prefill: large token passes, one-term activations --------------------------------
- * mx_prefill_kernel: GATEUP / DOWN for passes of up to 16*NB tokens with the activations
- * as single bf16 terms (the prefill precision), weights in the tiled MXFP4 layout. An item
- * is (pass, row block); a wave owns MT tiles of 16 weight rows and all the pass's tokens,
- * so every dequantized weight fragment feeds NB MFMAs and each weight byte is read once per
- * pass. K is staged 128 * SPC columns at a time: the pass's activations for a stage are
+/* ---- prefill: large token passes -------------------------------------------------------
+ * mx_prefill_kernel: GATEUP / DOWN for passes of many tokens, weights in the tiled MXFP4
+ * layout: up to 16*NB tokens with the activations as single bf16 terms (NS 1, the prefill
+ * precision), 8*NB with two (NS 2, fp32-accurate). An item is (pass, row block); a wave owns
+ * MT tiles of 16 weight rows and all the pass's tokens, so every dequantized weight fragment
+ * feeds NB MFMAs and each weight byte is read once per pass. With two terms the NB matrix
+ * column blocks are the pass's token blocks twice, hi terms then lo terms (fewer blocks of
+ * each for a shorter pass), and the two sums of a token meet in the epilogue. (Experts of more
+ * than 8 tokens used to take one 8-token streaming pass after another at this precision: 512
+ * tokens of the 384-expert layer 2.70 ms, of the 128-expert one 0.96 ms, 333 tokens over 896
+ * experts of 3584 x 3072 3.28 ms of expert kernels; so: 1.79, 0.51 and 2.8 ms, the bits the
+ * same.)
+ * K is staged 128 * SPC columns at a time: the pass's activations for a stage are
  * copied into LDS by the buffer unit (buffer_load ... lds: no registers, no LDS store
  * instructions), double-buffered with one barrier per stage, and shared by the NW waves.
  *
@@ -1473,14 +1480,15 @@ __device__ __forceinline__ uint32_t k3_bload4s(k3_rsrc r, uint32_t voff, uint32_
     return __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0);
 }
 
-template <int MODE, int MT, int NB, int SPC, int NW>
+template <int MODE, int MT, int NB, int SPC, int NW, int NS>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 8)))
 void mx_prefill_kernel(K3kMxArgs a)
 {
-    constexpr int KC = 128 * SPC, PT = 16 * NB, PR = KC / 8;
+    static_assert(NB % NS == 0, "column blocks: NS terms of NB / NS token blocks");
+    constexpr int KC = 128 * SPC, PT = 16 * NB / NS, PR = KC / 8;
     constexpr int RT = (MODE == K3K_MX_GATEUP) ? MT / 2 : MT;
     constexpr int PRP = PR + 1;                               /* slots per token row */
-    constexpr int DPW = (PT * PRP + 64 * NW - 1) / (64 * NW); /* DMA instructions per wave */
+    constexpr int DPW = (16 * NB * PRP + 64 * NW - 1) / (64 * NW); /* DMA instructions per wave */
     constexpr int NSL = DPW * 64 * NW;                        /* 16-byte slots per stage */
     constexpr int NU = 4 * SPC;                               /* 32-column sub-steps per stage */
     /* s_waitcnt operand: vmcnt <= one stage's weight and scale loads (MT (SPC + 1)), the
@@ -1577,15 +1585,20 @@ void mx_prefill_kernel(K3kMxArgs a)
             stile[m] = k3_tile_idx(t, 0, nchunk) * 256u;
         }
         /* DMA sources: instruction i of this wave fills slots 64 (wv + NW i) + lane */
-        const uint32_t xbytes = (uint32_t)a.n_xrows * (uint32_t)K * 2u;
+        /* (two terms: one descriptor over both arrays, xlo after xhi; column p is token
+         * p % (16 tbu) of term p / (16 tbu), tbu the pass's token blocks) */
+        const uint32_t lo_off = NS == 2 ? (uint32_t)((const char *)a.xlo - (const char *)a.xhi) : 0u;
+        const uint32_t xbytes = lo_off + (uint32_t)a.n_xrows * (uint32_t)K * 2u;
         const k3_rsrc rx = k3_make_rsrc(a.xhi, xbytes);
+        const int ptok = NS == 2 ? (ntok + 15) & ~15 : PT;
         uint32_t gsrc[DPW];
 #pragma unroll
         for (int i = 0; i < DPW; i++) {
             const int s = 64 * (wv + NW * i) + lane, p = s / PRP, o = (s % PRP) % PR;
-            const int ar = a.perm[off + tok0 + (p < ntok ? p : 0)];
+            const int pt = NS == 2 && p >= ptok ? p - ptok : p;
+            const int ar = a.perm[off + tok0 + (pt < ntok ? pt : 0)];
             const int xr = (MODE == K3K_MX_GATEUP) ? ar / a.topk : ar;
-            gsrc[i] = ((uint32_t)xr * (uint32_t)K + (uint32_t)o * 8u) * 2u;
+            gsrc[i] = ((uint32_t)xr * (uint32_t)K + (uint32_t)o * 8u) * 2u + (NS == 2 && p >= ptok ? lo_off : 0u);
         }
 
         k3_f32x4 acc[MT][NB];
@@ -1726,24 +1739,54 @@ void mx_prefill_kernel(K3kMxArgs a)
                 stage(c, P0{});
                 stage(c + 1, P1{});
             }
+            if constexpr (NS == 2)                        /* hi + lo */
+#pragma unroll
+                for (int m = 0; m < MT; m++)
+#pragma unroll
+                    for (int nb = 0; nb < NBU / 2; nb++) acc[m][nb] += acc[m][nb + NBU / 2];
         };
-        switch ((ntok + 15) >> 4) {
+        if constexpr (NS == 2) {
+            switch ((ntok + 15) >> 4) {
+                case 1: run(std::integral_constant<int, 2>{}); break;
+                case 2: run(std::integral_constant<int, (NB >= 4 ? 4 : NB)>{}); break;
+                default: run(std::integral_constant<int, NB>{}); break;
+            }
+        } else {
+            switch ((ntok + 15) >> 4) {
             case 1: if (NB >= 1) run(std::integral_constant<int, (NB >= 1 ? 1 : NB)>{}); break;
             case 2: if (NB >= 2) run(std::integral_constant<int, (NB >= 2 ? 2 : NB)>{}); break;
             case 3: if (NB >= 3) run(std::integral_constant<int, (NB >= 3 ? 3 : NB)>{}); break;
             case 4: if (NB >= 4) run(std::integral_constant<int, (NB >= 4 ? 4 : NB)>{}); break;
             case 5: if (NB >= 5) run(std::integral_constant<int, (NB >= 5 ? 5 : NB)>{}); break;
             default: run(std::integral_constant<int, NB>{}); break;
+            }
         }
 
 #pragma unroll
-        for (int nb = 0; nb < NB; nb++) {
+        for (int nb = 0; nb < NB / NS; nb++) {
             const int tk = nb * 16 + r16;
             if (tk >= ntok) continue;
             const int orow = orow_sh[tk];
             for (int m = 0; m < RT; m++) {
                 const int base = rb * rpg + wv * rpw + 16 * m + 4 * g;
-                if (MODE == K3K_MX_GATEUP) {
+                if (MODE == K3K_MX_GATEUP && NS == 2) {
+                    uint16_t h[4], l[4];
+#pragma unroll
+                    for (int jj = 0; jj < 4; jj++)
+                        k3_split2(k3_act_pair(acc[m][nb][jj], acc[m + RT][nb][jj], a.act, a.b1, a.b2), h[jj], l[jj]);
+                    uint16_t *oh = a.ahi + (size_t)orow * rows + base, *ol = a.alo + (size_t)orow * rows + base;
+                    if (base + 3 < rows && (rows & 3) == 0) {
+                        *reinterpret_cast<uint2 *>(oh) = make_uint2(h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16));
+                        *reinterpret_cast<uint2 *>(ol) = make_uint2(l[0] | ((uint32_t)l[1] << 16), l[2] | ((uint32_t)l[3] << 16));
+                    } else {
+                        for (int jj = 0; jj < 4; jj++)
+                            if (base + jj < rows) {
+                                oh[jj] = h[jj];
+                                ol[jj] = l[jj];
+                            }
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                } else if (MODE == K3K_MX_GATEUP) {
                     /* the activation is rounded to bf16: its fast form suffices */
                     uint16_t h[4];
 #pragma unroll
@@ -1776,12 +1819,12 @@ void mx_prefill_kernel(K3kMxArgs a)
     }
 }
 
-template <int MODE, int MT, int NB, int SPC, int NW>
+template <int MODE, int MT, int NB, int SPC, int NW, int NS = 1>
 int launch_prefill(const K3kMxArgs *a, int grid, hipStream_t st)
 {
     K3kMxArgs b = *a;
     b.stamps = k3k_stamps_take(MODE == K3K_MX_GATEUP ? 3 : 4, grid);
-    hipLaunchKernelGGL((mx_prefill_kernel<MODE, MT, NB, SPC, NW>), dim3(grid), dim3(64 * NW), 0, st, b);
+    hipLaunchKernelGGL((mx_prefill_kernel<MODE, MT, NB, SPC, NW, NS>), dim3(grid), dim3(64 * NW), 0, st, b);
     K3K_LAUNCH_CHECK("mx_prefill launch");
     return 0;
 }
@@ -1913,14 +1956,19 @@ extern "C" int k3k_mx_gemm(int mode, const K3kMxArgs *a, void *stream)
         if (a->nsplit == 2) return launch_mx<K3K_MX_PLAIN, 1, 1, 2, 2, 16>(a, kw, grid, st);
         return launch_mx<K3K_MX_PLAIN, 1, 1, 1, 2, 16>(a, kw, grid, st);
     }
-    if (a->pass_tok == 48 || a->pass_tok == 96) {
+    if (a->pass_tok == 48 || a->pass_tok == 96 || (a->pass_tok == 32 && a->nsplit == 2)) {
         /* large prefill batches on a tiled bank: 48-token passes (K staged 256 columns at a
          * time) or 96-token passes (128 columns at a time, so the pass fits in LDS twice
          * per CU); weights two stages ahead; each dequantized weight fragment feeds 3 or 6
-         * MFMA column blocks */
-        if (a->K % 512 || a->nsplit != 1 || a->layout != 1)
-            return k3k_fail("mx_moe: 48/96-token passes need K % 512 == 0, bf16 activations and "
-                            "a tiled bank", hipErrorInvalidValue);
+         * MFMA column blocks. Two activation terms: 48-token passes of 6 column blocks, or 32-token
+         * ones of 4 with K staged 256 columns at a time (twice the weights in flight) */
+        if (a->K % 512 || (a->nsplit != 1 && a->pass_tok == 96) || a->layout != 1)
+            return k3k_fail("mx_moe: 48/96-token passes need K % 512 == 0, bf16 activations (96) "
+                            "and a tiled bank", hipErrorInvalidValue);
+        if (a->nsplit == 2 &&
+            (a->xlo < a->xhi || (uint64_t)((const char *)a->xlo - (const char *)a->xhi) +
+                                        (uint64_t)a->n_xrows * a->K * 2 >= 0x80000000u))
+            return k3k_fail("mx_moe: two-term activations beyond 2 GiB", hipErrorInvalidValue);
         const bool gu = mode == K3K_MX_GATEUP;
         /* 8 waves per workgroup (one workgroup per CU at two waves per SIMD): twice the rows
          * per staged copy of the pass's activations of 4 waves, half the activation reads */
@@ -1930,6 +1978,12 @@ extern "C" int k3k_mx_gemm(int mode, const K3kMxArgs *a, void *stream)
         if (a->pass_tok == 96)
             return gu ? launch_prefill<K3K_MX_GATEUP, 4, 6, 1, 8>(a, grid, st)
                       : launch_prefill<K3K_MX_DOWN, 4, 6, 1, 8>(a, grid, st);
+        if (a->nsplit == 2 && a->pass_tok == 32)
+            return gu ? launch_prefill<K3K_MX_GATEUP, 4, 4, 2, 8, 2>(a, grid, st)
+                      : launch_prefill<K3K_MX_DOWN, 4, 4, 2, 8, 2>(a, grid, st);
+        if (a->nsplit == 2)
+            return gu ? launch_prefill<K3K_MX_GATEUP, 4, 6, 1, 8, 2>(a, grid, st)
+                      : launch_prefill<K3K_MX_DOWN, 4, 6, 1, 8, 2>(a, grid, st);
         return gu ? launch_prefill<K3K_MX_GATEUP, 4, 3, 2, 8>(a, grid, st)
                   : launch_prefill<K3K_MX_DOWN, 4, 3, 2, 8>(a, grid, st);
     }
