@@ -48,6 +48,11 @@ struct K3DevBank {
     uint64_t *used_at, clock;
     uint64_t *pin, epoch;       /* pin[s] == epoch while a MoE call holds the slot */
     int in_call;
+    /* device copy of the slots' pointers, [n_layers][n_experts] (NULL pointers: not resident),
+     * made on first use; a layer's part is rewritten when its slots have changed */
+    K3ExpertQ *table;
+    unsigned char *stale;       /* [n_layers] */
+    int *nres;                  /* [n_layers] experts resident */
     K3DevBankStats st;
 };
 
@@ -84,6 +89,15 @@ static void fill_q(const K3DevBank *b, int slot, K3ExpertQ *q)
     q->s3 = base + b->off[3];
     q->p2 = base + b->off[4];
     q->s2 = base + b->off[5];
+}
+
+/* The slot of a key changes (slot -1: it leaves the bank). */
+static void set_slot(K3DevBank *b, int key, int slot)
+{
+    const int layer = key / b->n_experts;
+    b->nres[layer] += (slot >= 0) - (b->slot_of[key] >= 0);
+    b->stale[layer] = 1;
+    b->slot_of[key] = slot;
 }
 
 static int key_ok(const K3DevBank *b, int layer, int expert)
@@ -124,7 +138,7 @@ static int admit(K3DevBank *b, int key, const void *const host[6])
     }
     void *stream = k3h_stream();
     if (b->key_of[slot] >= 0) {
-        b->slot_of[b->key_of[slot]] = -1;
+        set_slot(b, b->key_of[slot], -1);
         b->key_of[slot] = -1;
         b->st.evictions++;
     }
@@ -148,7 +162,7 @@ static int admit(K3DevBank *b, int key, const void *const host[6])
     /* the host bytes may be recycled by the upstream source's next get() */
     if (k3k_sync(stream)) return bank_error("k3_devbank: upload: %s", k3k_error());
     b->key_of[slot] = key;
-    b->slot_of[key] = slot;
+    set_slot(b, key, slot);
     b->st.misses++;
     touch(b, slot);
     return slot;
@@ -289,10 +303,13 @@ K3DevBank *k3_devbank_create(int n_layers, int n_experts, int width, int inter, 
     b->key_of = (int *)malloc((size_t)slots * sizeof(int));
     b->used_at = (uint64_t *)calloc((size_t)slots, sizeof(uint64_t));
     b->pin = (uint64_t *)calloc((size_t)slots, sizeof(uint64_t));
-    if (!b->slot_of || !b->key_of || !b->used_at || !b->pin) {
+    b->stale = (unsigned char *)malloc((size_t)n_layers);
+    b->nres = (int *)calloc((size_t)n_layers, sizeof(int));
+    if (!b->slot_of || !b->key_of || !b->used_at || !b->pin || !b->stale || !b->nres) {
         bank_error("k3_devbank_create: %s", "out of host memory");
         goto fail;
     }
+    memset(b->stale, 1, (size_t)n_layers);
     for (size_t k = 0; k < nkey; k++) b->slot_of[k] = -1;
     for (int s = 0; s < slots; s++) b->key_of[s] = -1;
     b->arena = (char *)k3k_malloc((size_t)slots * b->slot_bytes);
@@ -325,6 +342,8 @@ fail:
         free(b->key_of);
         free(b->used_at);
         free(b->pin);
+        free(b->stale);
+        free(b->nres);
         free(b);
     }
     b = NULL;
@@ -356,7 +375,7 @@ int k3_devbank_put_run(K3DevBank *b, int layer, int expert, const void *run, siz
         const int key = layer * b->n_experts + expert;
         if (b->slot_of[key] >= 0) {            /* replace in place */
             const int s = b->slot_of[key];
-            b->slot_of[key] = -1;
+            set_slot(b, key, -1);
             b->key_of[s] = -1;
         }
         rc = admit(b, key, host) < 0 ? -1 : 0;
@@ -388,6 +407,9 @@ void k3_devbank_destroy(K3DevBank *b)
     free(b->key_of);
     free(b->used_at);
     free(b->pin);
+    free(b->stale);
+    free(b->nres);
+    k3k_free(b->table);
     free(b);
     k3h_unlock();
 }
@@ -416,4 +438,31 @@ void k3_bank_call(K3ExpertSrc *src, int begin)
     K3DevBank *b = (K3DevBank *)src->ctx;
     if (begin) b->epoch++;
     b->in_call = begin;
+}
+
+const void *k3_bank_table(const K3ExpertSrc *src, int layer, int n_experts, int *all)
+{
+    *all = 0;
+    if (!src || src->get != src_get) return NULL;
+    K3DevBank *b = (K3DevBank *)src->ctx;
+    if (layer < 0 || layer >= b->n_layers || n_experts != b->n_experts) return NULL;
+    const size_t row = (size_t)n_experts * sizeof(K3ExpertQ);
+    if (!b->table) {
+        b->table = (K3ExpertQ *)k3k_malloc((size_t)b->n_layers * row);
+        if (!b->table) return NULL;
+    }
+    char *dev = (char *)b->table + (size_t)layer * row;
+    if (b->stale[layer]) {
+        K3ExpertQ *h = (K3ExpertQ *)calloc((size_t)n_experts, sizeof(K3ExpertQ));
+        if (!h) return NULL;
+        const int *slot = b->slot_of + (size_t)layer * n_experts;
+        for (int e = 0; e < n_experts; e++)
+            if (slot[e] >= 0) fill_q(b, slot[e], &h[e]);
+        const int rc = k3k_h2d(dev, h, row, k3h_stream()) || k3k_sync(k3h_stream());
+        free(h);
+        if (rc) return NULL;
+        b->stale[layer] = 0;
+    }
+    *all = b->nres[layer] == n_experts;
+    return dev;
 }

@@ -609,7 +609,7 @@ static int moe_experts_ws(float *out, const int *idx, const float *wt, const flo
     a2.max_passes = w->max_passes2;
     /* the second list's gate/up and down run on a side stream beside the first's */
     void *side = NULL;
-    if (pass_tok2 && k3k_fork(stream, &side)) return fail("fork");
+    if (pass_tok2 && k3k_fork(stream, 0, &side)) return fail("fork");
     a.queue = w->counts + 4;
     a2.queue = w->counts + 4 + 2 * K3K_NXCD_Q;
     if (k3k_mx_gemm(K3K_MX_GATEUP, &a, stream)) return fail("mx_gemm gateup");
@@ -633,7 +633,7 @@ static int moe_experts_ws(float *out, const int *idx, const float *wt, const flo
         a2.n_xrows = a.n_xrows;
         a2.queue = w->counts + 4 + 3 * K3K_NXCD_Q;
         if (k3k_mx_gemm(K3K_MX_DOWN, &a2, side)) return fail("mx_gemm down (second list)");
-        if (k3k_join(stream)) return fail("join");
+        if (k3k_join(stream, 0)) return fail("join");
     }
     k3k_prof_mark(stream, K3D_STAGE_DOWN);
     if (k3k_combine(out, w->contrib, wt, idx, bank, n_experts, T, topk, hidden, stream)) return fail("combine");
@@ -701,7 +701,7 @@ int k3d_moe_routed(float *out, int *idx, float *wt, const float *x, int T, const
     const int split_side = split && (size_t)T * hidden >= ((size_t)1 << 22);
     if (split) {
         void *side = stream;
-        if (split_side && k3k_fork(stream, &side)) return fail("fork");
+        if (split_side && k3k_fork(stream, 0, &side)) return fail("fork");
         if (k3k_split_bf16(w.xhi, w.xlo, x, (size_t)T * hidden, side)) return fail("split");
     }
     /* the expert-major gather runs in the router's final kernel when it can (a launch and its
@@ -729,7 +729,7 @@ int k3d_moe_routed(float *out, int *idx, float *wt, const float *x, int T, const
     rc = router_run(idx, wt, x, T, router_w, bias, hidden, n_experts, topk, renorm, routed_scale,
                     &r, gathered ? &ga : NULL, stream);
     if (rc) return rc;
-    if (split_side && k3k_join(stream)) return fail("join");
+    if (split_side && k3k_join(stream, 0)) return fail("join");
     k3k_prof_mark(stream, K3D_STAGE_ROUTER);
     return moe_experts_ws(out, idx, wt, x, T, bank, layout, hidden, inter, n_experts, topk, act,
                           b1, b2, prec, &w, perm_out, offsets_out, drops_out, NULL, split, gathered,

@@ -147,6 +147,88 @@ static void *pinned(size_t bytes)
     return g_pin;
 }
 
+/* x and the output of the MoE block through pinned staging: copy kernels move them between the
+ * staging and the device (k3k_pin_copy; 9.5 MB, 333 tokens of 7168, in 0.19 ms), and a few
+ * threads between the staging and the caller's memory, chunk by chunk beside the transfers. As
+ * pageable copies the two took 0.45 and 0.85 ms: one thread moved about 12 GB/s. */
+#define STAGE_MAX ((size_t)32 << 20)    /* the most staging kept, and bytes per round */
+#define STAGE_CHUNKS 4
+#define STAGE_THREADS 4
+static char *g_stage = NULL;
+static size_t g_stage_cap = 0;
+static void *g_stage_ev[STAGE_CHUNKS];
+
+static char *staging(size_t bytes)
+{
+    if (bytes > STAGE_MAX) bytes = STAGE_MAX;
+    if (g_stage_cap < bytes) {
+        check(k3k_sync(NULL), "synchronize before staging growth");
+        k3k_host_free(g_stage);
+        g_stage_cap = bytes + bytes / 4 < STAGE_MAX ? bytes + bytes / 4 : STAGE_MAX;
+        g_stage = (char *)k3k_host_alloc(g_stage_cap);
+        if (!g_stage) fatal("pinned host allocation");
+    }
+    for (int i = 0; i < STAGE_CHUNKS; i++)
+        if (!g_stage_ev[i] && !(g_stage_ev[i] = k3k_event_create())) fatal("event creation");
+    return g_stage;
+}
+
+static void host_copy(char *dst, const char *src, size_t bytes)
+{
+    if (bytes < ((size_t)256 << 10)) {
+        memcpy(dst, src, bytes);
+        return;
+    }
+    const size_t part = (bytes / STAGE_THREADS + 4095u) & ~(size_t)4095u;
+#pragma omp parallel for num_threads(STAGE_THREADS) schedule(static, 1)
+    for (int i = 0; i < STAGE_THREADS; i++) {
+        const size_t a = (size_t)i * part < bytes ? (size_t)i * part : bytes;
+        const size_t b = a + part < bytes ? a + part : bytes;
+        memcpy(dst + a, src + a, b - a);
+    }
+}
+
+static size_t stage_chunk(size_t bytes)
+{
+    const size_t c = (bytes / STAGE_CHUNKS + 4095u) & ~(size_t)4095u;
+    return c > ((size_t)1 << 20) ? c : (size_t)1 << 20;
+}
+
+static void *upload_staged(int slot, const void *h, size_t bytes)
+{
+    char *d = (char *)buf(slot, bytes), *st = staging(bytes);
+    for (size_t r0 = 0; r0 < bytes; r0 += STAGE_MAX) {
+        const size_t n = bytes - r0 < STAGE_MAX ? bytes - r0 : STAGE_MAX, c = stage_chunk(n);
+        if (r0) check(k3k_sync(g_stream), "synchronize");       /* the staging is free again */
+        for (size_t o = 0; o < n; o += c) {
+            const size_t k = n - o < c ? n - o : c;
+            host_copy(st + o, (const char *)h + r0 + o, k);
+            check(k3k_pin_copy(d + r0 + o, st + o, NULL, k, g_stream), "host to device copy");
+        }
+    }
+    return d;
+}
+
+/* h = d, or d + add */
+static void download_staged(float *h, const float *d, const float *add, size_t bytes)
+{
+    char *st = staging(bytes);
+    for (size_t r0 = 0; r0 < bytes; r0 += STAGE_MAX) {
+        const size_t n = bytes - r0 < STAGE_MAX ? bytes - r0 : STAGE_MAX, c = stage_chunk(n);
+        int i = 0;
+        for (size_t o = 0; o < n; o += c, i++) {
+            check(k3k_pin_copy(st + o, (const char *)d + r0 + o, add ? add + (r0 + o) / 4 : NULL,
+                               n - o < c ? n - o : c, g_stream), "device to host copy");
+            check(k3k_event_record(g_stage_ev[i], g_stream), "event");
+        }
+        i = 0;
+        for (size_t o = 0; o < n; o += c, i++) {
+            check(k3k_event_sync(g_stage_ev[i]), "device to host copy");
+            host_copy((char *)h + r0 + o, st + o, n - o < c ? n - o : c);
+        }
+    }
+}
+
 /* ---------------------------------------------------------------- registry ---- */
 typedef struct {
     const unsigned char *host;
@@ -463,14 +545,16 @@ static void experts_generic(float *out_d, const int *idx, const float *wt_d, con
           "combine");
 }
 
-/* Runs the expert half for a device bank already resolved into `bank` (host array of
- * device pointers, NULL where absent): out_d[T][hidden] = sum_j wt * expert(x). */
+/* Enqueues the expert half for a device bank already resolved into `bank` (host array of
+ * device pointers, NULL where absent), or already on the device in `table`:
+ * out_d[T][hidden] = sum_j wt * expert(x). */
 static void run_bank(float *out_d, const int *idx, const int *idx_d, const float *wt_d,
                      const float *x_d, int T, const QPtr *bank, int hidden, int inter,
-                     int n_experts, int topk, int act, float b1, float b2, int prec, int layout)
+                     int n_experts, int topk, int act, float b1, float b2, int prec, int layout,
+                     const void *table)
 {
     if ((hidden % 32) == 0 && (inter % 32) == 0) {
-        void *bank_d = upload(B_BANK, bank, (size_t)n_experts * sizeof(QPtr));
+        const void *bank_d = table ? table : upload(B_BANK, bank, (size_t)n_experts * sizeof(QPtr));
         const size_t wsb = k3d_moe_ws(T, hidden, inter, n_experts, topk, prec);
         check(k3d_moe_experts(out_d, idx_d, wt_d, x_d, T, bank_d, layout, hidden, inter,
                               n_experts, topk, act, b1, b2, prec, buf(B_WS, wsb), wsb, NULL, NULL,
@@ -480,7 +564,6 @@ static void run_bank(float *out_d, const int *idx, const int *idx_d, const float
         experts_generic(out_d, idx, wt_d, idx_d, x_d, T, bank, hidden, inter, n_experts, topk, act,
                         b1, b2);
     }
-    check(k3k_sync(g_stream), "synchronize");
 }
 
 /* Resolves the experts selected in idx (host) from a host bank and runs them. */
@@ -507,7 +590,8 @@ static void run_experts_mxfp4(float *out_d, const int *idx, const int *idx_d, co
     for (int e = 0; e < n_experts; e++)
         if (sel[e] && expert_ok(&hbank[e])) resolve_expert(&bank[e], &hbank[e], hidden, inter, arena, &off);
     run_bank(out_d, idx, idx_d, wt_d, x_d, T, bank, hidden, inter, n_experts, topk, act, b1, b2, prec,
-             K3D_LAYOUT_ROWS);
+             K3D_LAYOUT_ROWS, NULL);
+    check(k3k_sync(g_stream), "synchronize");
     free(bank);
     free(sel);
 }
@@ -587,16 +671,25 @@ static size_t wbytes(int wdt, int in, int out)
     return (size_t)in * out * 4;
 }
 
-/* y[t*ldy + o] = W x[t] for a tagged weight matrix (k3_mmw, reference k3.h:289-295). Up to
- * four tokens stream the weights through the vector-unit GEMV; more bf16 tokens go to the
- * matrix-core GEMM with the activations split into two bf16 terms (fp32-accurate). */
+/* Whether a bf16 product of ntok tokens has 128 x 64 tiles for three fifths of the CUs, so that
+ * the matrix-core GEMM (k3_gemm.hip, two activation terms) is the faster one. Below, and for one
+ * token, it streams through k3k_gemv_bf16, whose several-token kernel takes the fp32 activations
+ * as they are (7168 -> 3584: 37 tokens 21 us against 78 for the split and the GEMM, 256 tokens
+ * (112 tiles) 55 against 78, 333 tokens (168) 96 against 78). */
+static int mmw_gemm(int wdt, int ntok, int in, int out)
+{
+    return wdt == K3_WBF16 && in % 64 == 0 &&
+           (long)((out + 127) / 128) * ((ntok + 63) / 64) * 5 >= (long)k3k_cu_count() * 3 &&
+           (unsigned long long)out * in * 2 < 0x80000000ull && (unsigned long long)ntok * in * 2 < 0x80000000ull;
+}
+
+/* y[t*ldy + o] = W x[t] for a tagged weight matrix (k3_mmw, reference k3.h:289-295). */
 static void mmw_on(float *y_d, const float *x_d, int ntok, const void *W, int wdt, int in, int out,
                    int ldy, int slot, int xs_slot, void *stream)
 {
     const void *dw = weights(slot, W, wbytes(wdt, in, out));
     int rc;
-    if (wdt == K3_WBF16 && ntok > 4 && in % 64 == 0 &&
-        (unsigned long long)out * in * 2 < 0x80000000ull && (unsigned long long)ntok * in * 2 < 0x80000000ull) {
+    if (ntok > 1 && mmw_gemm(wdt, ntok, in, out)) {
         uint16_t *xs = (uint16_t *)buf(xs_slot, (size_t)ntok * in * 4);
         uint16_t *xl = xs + (size_t)ntok * in;
         check(k3k_split_bf16(xs, xl, x_d, (size_t)ntok * in, stream), "activation split");
@@ -670,19 +763,24 @@ static void run_fetched(Fetch *f)
     }
     if (!any && f->passes > 0) return;
     float *dst = f->passes == 0 ? f->dacc : (float *)buf(B_SDN, (size_t)T * L * 4);
-    check(k3k_h2d(f->di, f->pidx, TK * 4, g_stream), "host to device copy");
-    check(k3k_h2d(f->dwt, f->hwt, TK * 4, g_stream), "host to device copy");
+    /* the router's own idx and weights are still there: sent again only where a slot fell out
+     * or the weights were renormalised */
+    const int resent = f->passes > 0 || f->w->cache_only || memcmp(f->pidx, f->hidx, TK * 4);
+    if (resent) {
+        check(k3k_h2d(f->di, f->pidx, TK * 4, g_stream), "host to device copy");
+        check(k3k_h2d(f->dwt, f->hwt, TK * 4, g_stream), "host to device copy");
+    }
+    int all;
+    const void *table = f->bank_layout >= 0 ? k3_bank_table(f->w->src, f->w->layer, f->N, &all) : NULL;
     const int layout = f->bank_layout >= 0 ? f->bank_layout : K3D_LAYOUT_ROWS;
     for (int b0 = 0; b0 < T; b0 += MOE_DEV_BLOCK) {
         const int nb = T - b0 < MOE_DEV_BLOCK ? T - b0 : MOE_DEV_BLOCK;
         const size_t o = (size_t)b0 * K;
         run_bank(dst + (size_t)b0 * L, f->pidx + o, f->di + o, f->dwt + o, f->dz + (size_t)b0 * L, nb,
-                 f->bank, L, f->I, f->N, K, K3_ACT_SITU, f->b1, f->b2, 0, layout);
+                 f->bank, L, f->I, f->N, K, K3_ACT_SITU, f->b1, f->b2, 0, layout, table);
     }
-    if (f->passes > 0) {
-        check(k3k_axpy_rows(f->dacc, dst, (size_t)T * L, g_stream), "aggregate");
-        check(k3k_sync(g_stream), "synchronize");
-    }
+    if (f->passes > 0) check(k3k_axpy_rows(f->dacc, dst, (size_t)T * L, g_stream), "aggregate");
+    if (resent || !table) check(k3k_sync(g_stream), "synchronize");    /* host arrays the copies read */
     f->passes++;
 }
 
@@ -697,6 +795,7 @@ static int fetch(Fetch *f, int e, int via_resident)
      * so it never needs more than topk + 1 slots; k3_cache.c:305) */
     if (!via_resident && f->bank_layout >= 0 && k3_bank_full(s, f->w->layer, e)) {
         run_fetched(f);
+        check(k3k_sync(g_stream), "synchronize");       /* its slots are computed */
         k3_bank_call(s, 0);
         k3_bank_call(s, 1);
         memset(f->bank, 0, (size_t)f->N * sizeof(QPtr));
@@ -777,6 +876,61 @@ static void fetch_chunk(Fetch *f, int t0, int n, int *uniq, unsigned char *seen)
     }
 }
 
+/* The shared expert's sum sdn [T][E] on `stream`; its weights are on the device, or uploaded one
+ * matrix at a time. */
+static float *shared_on(const float *dx, const K3MoeW *w, const K3Cfg *c, int T, void *stream)
+{
+    const int E = c->hidden, SI = c->moe_inter * c->n_shared;
+    float *sdn = (float *)buf(B_SSDN, (size_t)T * E * 4);
+    const uint16_t *w1 = (const uint16_t *)k3_dev_lookup(w->sh1), *w3 = (const uint16_t *)k3_dev_lookup(w->sh3);
+    if (T > 1 && w1 && w3 && E % 64 == 0 && SI % 64 == 0 && mmw_gemm(w->wdt, T, E, SI) &&
+        mmw_gemm(w->wdt, T, SI, E)) {
+        /* many tokens: gate, up and the activation in one GEMM, its result as bf16 terms */
+        uint16_t *xs = (uint16_t *)buf(B_SXS, (size_t)T * E * 4), *as = (uint16_t *)buf(B_SACT, (size_t)T * SI * 4);
+        check(k3k_split_bf16(xs, xs + (size_t)T * E, dx, (size_t)T * E, stream), "activation split");
+        check(k3k_dense_gateup(as, as + (size_t)T * SI, w1, w3, xs, xs + (size_t)T * E, SI, T, E, K3_ACT_SITU,
+                               c->situ_b1, c->situ_b2, NULL, 0, stream),
+              "shared gate/up");
+        check(k3k_dense_gemm(sdn, E, 0, (const uint16_t *)weights(B_P, w->sh2, wbytes(w->wdt, SI, E)), as,
+                             as + (size_t)T * SI, E, T, SI, NULL, 0, stream),
+              "shared down");
+        return sdn;
+    }
+    float *sact = (float *)buf(B_SACT, (size_t)T * SI * 4);
+    if (T == 1 && w1 && w3 && w->wdt != K3_WI8 && E % 8 == 0 && aligned16(w1) && aligned16(w3)) {
+        /* one token: gate, up and the activation in one launch */
+        check(k3k_gemv_glu(sact, dx, w1, w3, w->wdt == K3_WBF16, E, SI, K3_ACT_SITU, c->situ_b1, c->situ_b2, stream),
+              "shared gate/up");
+        mmw_on(sdn, sact, T, w->sh2, w->wdt, SI, E, E, B_P, B_SXS, stream);
+        return sdn;
+    }
+    float *sgu = (float *)buf(B_SGU, (size_t)T * 2 * SI * 4);
+    mmw_on(sgu, dx, T, w->sh1, w->wdt, E, SI, 2 * SI, B_P, B_SXS, stream);
+    mmw_on(sgu + SI, dx, T, w->sh3, w->wdt, E, SI, 2 * SI, B_P, B_SXS, stream);
+    check(k3k_act(sact, sgu, SI, T, K3_ACT_SITU, c->situ_b1, c->situ_b2, stream), "shared act");
+    mmw_on(sdn, sact, T, w->sh2, w->wdt, SI, E, E, B_P, B_SXS, stream);
+    return sdn;
+}
+
+/* The block after the routed experts: the aggregate's norm and up-projection into dout. Returns
+ * the shared expert's sum, to be added to it on the way out (sdn, when it is already on its way
+ * on the side stream), or NULL. */
+static const float *moe_tail(float *dout, float *dacc, const float *dx, const K3MoeW *w, const K3Cfg *c, int T,
+                             int shared, const float *sdn)
+{
+    const int E = c->hidden, L = c->latent;
+    /* 4. RMSNorm of the aggregate, 5. up-project */
+    if (c->latent_norm) {
+        const float *dn = (const float *)weights(B_T1, w->latent_norm, (size_t)L * 4);
+        check(k3k_rmsnorm(dacc, dacc, dn, L, T, c->rms_eps, g_stream), "latent rmsnorm");
+    }
+    mmw_dev(dout, dacc, T, w->up, w->wdt, L, E, E, B_P);
+    /* 6. shared expert on the original input, added unweighted */
+    if (sdn) check(k3k_join(g_stream, 1), "join");
+    else if (shared) sdn = shared_on(dx, w, c, T, g_stream);
+    return sdn;
+}
+
 /* Stable LatentMoE over T tokens (reference k3_ops.c:556-656), batched on the device:
  * route all tokens, down-project, run the selected experts expert-major, sum in slot
  * order, RMSNorm the aggregate, up-project, add the unweighted shared expert. The
@@ -805,54 +959,64 @@ static void moe_latent(float *out, const float *x, const K3MoeW *w, const K3Cfg 
         abort();
     }
     /* 1. route on the full width */
-    const float *dx = (const float *)upload(B_X, x, (size_t)T * E * 4);
+    const float *dx = (const float *)upload_staged(B_X, x, (size_t)T * E * 4);
     const float *dW = (const float *)weights(B_RW, w->gate, (size_t)N * E * 4);
     const float *db = w->bias ? (const float *)weights(B_BIAS, w->bias, (size_t)N * 4) : NULL;
-    int *di = (int *)buf(B_IDX, TK * 4);
-    float *dwt = (float *)buf(B_WT, TK * 4);
+    const size_t TKp = (TK + 63) & ~(size_t)63;            /* idx, then the weights */
+    int *di = (int *)buf(B_IDX, (TKp + TK) * 4);
+    float *dwt = (float *)(di + TKp);
+    /* 6. (ahead) the shared expert depends on x alone: with its weights resident it runs on a
+     * side stream and is joined before its sum is added. One token: from the start, beside the
+     * router and the down-projection, which leave the HBM idle; more: beside the routed experts,
+     * which leave the matrix cores idle (beside the router of 333 tokens it made that and the
+     * down-projection 0.23 ms longer). */
+    const int shared = SI > 0 && w->sh1 && w->sh3 && w->sh2;
+    const int shared_side = shared && k3_dev_lookup(w->sh1) && k3_dev_lookup(w->sh3) &&
+                            k3_dev_lookup(w->sh2) && wbytes(w->wdt, E, SI) > 0;
+    void *side = NULL;
     {
         const size_t wsb = k3d_router_ws(T, E, N);
-        check(k3d_router(di, dwt, dx, T, dW, db, E, N, K, c->moe_renorm, c->routed_scale,
-                         buf(B_WS, wsb), wsb, g_stream),
+        void *ws = buf(B_WS, wsb);
+        if (shared_side && T == 1) check(k3k_fork(g_stream, 1, &side), "fork");
+        check(k3d_router(di, dwt, dx, T, dW, db, E, N, K, c->moe_renorm, c->routed_scale, ws, wsb, g_stream),
               "k3_moe router");
     }
+    float *sdn = NULL;
     /* the routing comes back through pinned memory; the host waits for it alone, while the
-     * device goes on with the down-projection */
-    {
-        char *pin = (char *)pinned(TK * 8);
-        check(k3k_d2h(pin, di, TK * 4, g_stream), "device to host copy");
-        check(k3k_d2h(pin + TK * 4, dwt, TK * 4, g_stream), "device to host copy");
-        check(k3k_event_record(g_pin_ev, g_stream), "event");
-    }
+     * device goes on */
+    check(k3k_pin_copy(pinned((TKp + TK) * 4), di, NULL, (TKp + TK) * 4, g_stream), "device to host copy");
+    check(k3k_event_record(g_pin_ev, g_stream), "event");
     /* 2. down-project into the latent space */
     float *dz = (float *)buf(B_Z, (size_t)T * L * 4);
     mmw_dev(dz, dx, T, w->down, w->wdt, E, L, L, B_P);
-    /* 6. (ahead) the shared expert depends on x alone: with its weights resident it runs on
-     * the library stream's side stream, forked after the routing and the down-projection
-     * (the critical path), beside the routed experts, and joined before its sum is added */
-    const size_t wsh = wbytes(w->wdt, E, SI);
-    const int shared = SI > 0 && w->sh1 && w->sh3 && w->sh2;
-    const int shared_side = shared && k3_dev_lookup(w->sh1) && k3_dev_lookup(w->sh3) &&
-                            k3_dev_lookup(w->sh2) && wsh > 0;
-    float *sdn = NULL;
-    if (shared_side) {
-        void *side = NULL;
-        check(k3k_fork(g_stream, &side), "fork");
-        float *sgu = (float *)buf(B_SGU, (size_t)T * 2 * SI * 4);
-        float *sact = (float *)buf(B_SACT, (size_t)T * SI * 4);
-        sdn = (float *)buf(B_SSDN, (size_t)T * E * 4);
-        mmw_on(sgu, dx, T, w->sh1, w->wdt, E, SI, 2 * SI, B_P, B_SXS, side);
-        mmw_on(sgu + SI, dx, T, w->sh3, w->wdt, E, SI, 2 * SI, B_P, B_SXS, side);
-        check(k3k_act(sact, sgu, SI, T, K3_ACT_SITU, c->situ_b1, c->situ_b2, side), "shared act");
-        mmw_on(sdn, sact, T, w->sh2, w->wdt, SI, E, E, B_P, B_SXS, side);
+    if (shared_side && T == 1) sdn = shared_on(dx, w, c, T, side);
+    else if (shared_side) check(k3k_fork(g_stream, 1, &side), "fork");
+    float *dacc = (float *)buf(B_ACC, (size_t)T * L * 4);
+    float *dout = (float *)buf(B_OUT, (size_t)T * E * 4);
+    /* With every expert of the layer in this library's HBM bank, no fetch can be needed: the
+     * experts run from the bank's own device table on the routing as the router wrote it, and
+     * the host follows with the bank's bookkeeping (the same get / getmany calls, all hits)
+     * while the block runs, instead of between the two. */
+    int all = 0;
+    const void *table = w->src && !w->cache_only && L % 32 == 0 && I % 32 == 0 &&
+                                k3_bank_layout(w->src, L, I) >= 0
+                            ? k3_bank_table(w->src, w->layer, N, &all) : NULL;
+    if (all) {
+        for (int b0 = 0; b0 < T; b0 += MOE_DEV_BLOCK) {
+            const int nb = T - b0 < MOE_DEV_BLOCK ? T - b0 : MOE_DEV_BLOCK;
+            const size_t o = (size_t)b0 * K;
+            run_bank(dacc + (size_t)b0 * L, NULL, di + o, dwt + o, dz + (size_t)b0 * L, nb, NULL, L, I, N, K,
+                     K3_ACT_SITU, c->situ_b1, c->situ_b2, 0, k3_bank_layout(w->src, L, I), table);
+        }
     }
+    if (shared_side && !sdn) sdn = shared_on(dx, w, c, T, side);
+    const float *add = all ? moe_tail(dout, dacc, dx, w, c, T, shared, sdn) : NULL;
 
     check(k3k_event_sync(g_pin_ev), "routing copy");
     memcpy(hidx, g_pin, TK * 4);
-    memcpy(hwt, (char *)g_pin + TK * 4, TK * 4);
+    memcpy(hwt, (char *)g_pin + TKp * 4, TK * 4);
 
     /* 3. routed experts, weighted sum in slot order */
-    float *dacc = (float *)buf(B_ACC, (size_t)T * L * 4);
     int wrote_last = 0;
     if (w->src) {
         Fetch f;
@@ -916,7 +1080,7 @@ static void moe_latent(float *out, const float *x, const K3MoeW *w, const K3Cfg 
         }
         /* the assignments not computed yet, on the routing the device uses: kept slots,
          * renormalised weights */
-        run_fetched(&f);
+        if (!all) run_fetched(&f);
         k3_bank_call(w->src, 0);
         free(f.bank);
         free(f.done);
@@ -948,29 +1112,8 @@ static void moe_latent(float *out, const float *x, const K3MoeW *w, const K3Cfg 
         wrote_last = 1;
     }
 
-    /* 4. RMSNorm of the aggregate, 5. up-project */
-    if (c->latent_norm) {
-        const float *dn = (const float *)weights(B_T1, w->latent_norm, (size_t)L * 4);
-        check(k3k_rmsnorm(dacc, dacc, dn, L, T, c->rms_eps, g_stream), "latent rmsnorm");
-    }
-    float *dout = (float *)buf(B_OUT, (size_t)T * E * 4);
-    mmw_dev(dout, dacc, T, w->up, w->wdt, L, E, E, B_P);
-
-    /* 6. shared expert on the original input, added unweighted */
-    if (shared_side) {
-        check(k3k_join(g_stream), "join");
-        check(k3k_axpy_rows(dout, sdn, (size_t)T * E, g_stream), "shared add");
-    } else if (shared) {
-        float *sgu = (float *)buf(B_SGU, (size_t)T * 2 * SI * 4);
-        float *sact = (float *)buf(B_SACT, (size_t)T * SI * 4);
-        sdn = (float *)buf(B_SSDN, (size_t)T * E * 4);
-        mmw_dev(sgu, dx, T, w->sh1, w->wdt, E, SI, 2 * SI, B_P);
-        mmw_dev(sgu + SI, dx, T, w->sh3, w->wdt, E, SI, 2 * SI, B_P);
-        check(k3k_act(sact, sgu, SI, T, K3_ACT_SITU, c->situ_b1, c->situ_b2, g_stream), "shared act");
-        mmw_dev(sdn, sact, T, w->sh2, w->wdt, SI, E, E, B_P);
-        check(k3k_axpy_rows(dout, sdn, (size_t)T * E, g_stream), "shared add");
-    }
-    download(out, dout, (size_t)T * E * 4);
+    if (!all) add = moe_tail(dout, dacc, dx, w, c, T, shared, sdn);
+    download_staged(out, dout, add, (size_t)T * E * 4);
     if (wrote_last) {
         if (idx_last) memcpy(idx_last, hidx + (size_t)(T - 1) * K, (size_t)K * sizeof(int));
         if (wt_last) memcpy(wt_last, hwt + (size_t)(T - 1) * K, (size_t)K * sizeof(float));

@@ -97,6 +97,31 @@ extern "C" int k3k_d2d(void *dst, const void *src, size_t bytes, void *stream)
 }
 
 namespace {
+/* Words between device memory and pinned host memory (either way), 16 bytes a lane. Between
+ * kernels of one stream a copy by the DMA engine costs far more than its bytes: the kernel
+ * behind it waited 160 us for a 42 KB copy to signal, and copies with an event between them
+ * started 240 us apart; a kernel moves 47-50 GB/s and costs a launch. */
+__global__ __launch_bounds__(256) void pin_copy_kernel(uint4 *d, const uint4 *s, const float *add, size_t n16, int ntail)
+{
+    uint32_t *dw = reinterpret_cast<uint32_t *>(d);
+    const uint32_t *sw = reinterpret_cast<const uint32_t *>(s);
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n16; i += (size_t)gridDim.x * 256) {
+        uint4 v = s[i];
+        if (add) {
+            const float4 a = reinterpret_cast<const float4 *>(add)[i];
+            v.x = __float_as_uint(__uint_as_float(v.x) + a.x);
+            v.y = __float_as_uint(__uint_as_float(v.y) + a.y);
+            v.z = __float_as_uint(__uint_as_float(v.z) + a.z);
+            v.w = __float_as_uint(__uint_as_float(v.w) + a.w);
+        }
+        d[i] = v;
+    }
+    if (blockIdx.x == 0 && (int)threadIdx.x < ntail) {
+        const size_t i = 4 * n16 + threadIdx.x;
+        dw[i] = add ? __float_as_uint(__uint_as_float(sw[i]) + add[i]) : sw[i];
+    }
+}
+
 __global__ void zero_kernel(uint32_t *p, size_t nwords, uint8_t *tail, size_t ntail)
 {
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < nwords;
@@ -105,6 +130,20 @@ __global__ void zero_kernel(uint32_t *p, size_t nwords, uint8_t *tail, size_t nt
     if (blockIdx.x == 0 && threadIdx.x < ntail) tail[threadIdx.x] = 0;
 }
 }  // namespace
+
+extern "C" int k3k_pin_copy(void *dst, const void *src, const float *add, size_t bytes, void *stream)
+{
+    if (!bytes) return 0;
+    if (bytes % 4 || (((uintptr_t)dst | (uintptr_t)src | (uintptr_t)add) & 15)) return k3k_fail("pin_copy alignment", hipErrorInvalidValue);
+    const size_t n16 = bytes / 16;
+    size_t blocks = (n16 + 255) / 256;
+    if (blocks < 1) blocks = 1;
+    if (blocks > 1024) blocks = 1024;
+    hipLaunchKernelGGL(pin_copy_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, (uint4 *)dst,
+                       (const uint4 *)src, add, n16, (int)(bytes % 16 / 4));
+    K3K_LAUNCH_CHECK("pin_copy launch");
+    return 0;
+}
 
 /* A fill kernel rather than hipMemsetAsync, so that a caller may capture it in a graph. */
 extern "C" int k3k_zero(void *dst, size_t bytes, void *stream)
@@ -168,7 +207,8 @@ extern "C" int k3k_sync(void *stream)
 
 /* ---- side streams --------------------------------------------------------------------
  * Work that may run beside the caller's (the activation split beside the router, the hot
- * experts' pass list) goes to a side stream of the caller's stream: one per caller stream,
+ * experts' pass list; in the host entry points also the shared expert, on the second one)
+ * goes to a side stream of the caller's stream: two per caller stream,
  * created with the default priority, non-blocking, with its own fork and join events.
  * Work is forked after what is already queued on the caller's stream and joined back into
  * it; both are event waits, so a stream being captured into a graph captures the side work
@@ -178,8 +218,8 @@ extern "C" int k3k_sync(void *stream)
  * stream's entry. */
 #define K3_SIDE_MAX 256
 struct K3Side {
-    hipStream_t caller, side;
-    hipEvent_t fork, join;
+    hipStream_t caller, side[2];
+    hipEvent_t fork[2], join[2];
 };
 static K3Side g_side[K3_SIDE_MAX];
 static int g_nside = 0;
@@ -199,18 +239,24 @@ static K3Side *side_of(hipStream_t s)
         if (g_nside == K3_SIDE_MAX) {
             k3k_fail("side stream: more than 256 caller streams", hipErrorInvalidValue);
         } else {
-            K3Side n = {s, nullptr, nullptr, nullptr};
-            hipError_t e = hipStreamCreateWithFlags(&n.side, hipStreamNonBlocking);
-            if (e == hipSuccess) e = hipEventCreateWithFlags(&n.fork, hipEventDisableTiming);
-            if (e == hipSuccess) e = hipEventCreateWithFlags(&n.join, hipEventDisableTiming);
+            K3Side n = {};
+            n.caller = s;
+            hipError_t e = hipSuccess;
+            for (int k = 0; k < 2; k++) {
+                if (e == hipSuccess) e = hipStreamCreateWithFlags(&n.side[k], hipStreamNonBlocking);
+                if (e == hipSuccess) e = hipEventCreateWithFlags(&n.fork[k], hipEventDisableTiming);
+                if (e == hipSuccess) e = hipEventCreateWithFlags(&n.join[k], hipEventDisableTiming);
+            }
             if (e == hipSuccess) {
                 g_side[g_nside] = n;
                 r = &g_side[g_nside++];
             } else {
                 k3k_fail("side stream: create", e);
-                if (n.join) (void)hipEventDestroy(n.join);
-                if (n.fork) (void)hipEventDestroy(n.fork);
-                if (n.side) (void)hipStreamDestroy(n.side);
+                for (int k = 0; k < 2; k++) {
+                    if (n.join[k]) (void)hipEventDestroy(n.join[k]);
+                    if (n.fork[k]) (void)hipEventDestroy(n.fork[k]);
+                    if (n.side[k]) (void)hipStreamDestroy(n.side[k]);
+                }
             }
         }
     }
@@ -224,23 +270,23 @@ extern "C" int k3k_side_init(void)
     return side_of(nullptr) ? 0 : -1;
 }
 
-extern "C" int k3k_fork(void *stream, void **side)
+extern "C" int k3k_fork(void *stream, int which, void **side)
 {
     K3Side *sd = side_of((hipStream_t)stream);
     if (!sd) return -1;
-    hipError_t e = hipEventRecord(sd->fork, (hipStream_t)stream);
-    if (e == hipSuccess) e = hipStreamWaitEvent(sd->side, sd->fork, 0);
+    hipError_t e = hipEventRecord(sd->fork[which], (hipStream_t)stream);
+    if (e == hipSuccess) e = hipStreamWaitEvent(sd->side[which], sd->fork[which], 0);
     if (e != hipSuccess) return k3k_fail("fork", e);
-    *side = sd->side;
+    *side = sd->side[which];
     return 0;
 }
 
-extern "C" int k3k_join(void *stream)
+extern "C" int k3k_join(void *stream, int which)
 {
     K3Side *sd = side_of((hipStream_t)stream);
     if (!sd) return -1;
-    hipError_t e = hipEventRecord(sd->join, sd->side);
-    if (e == hipSuccess) e = hipStreamWaitEvent((hipStream_t)stream, sd->join, 0);
+    hipError_t e = hipEventRecord(sd->join[which], sd->side[which]);
+    if (e == hipSuccess) e = hipStreamWaitEvent((hipStream_t)stream, sd->join[which], 0);
     return e == hipSuccess ? 0 : k3k_fail("join", e);
 }
 
@@ -265,10 +311,12 @@ extern "C" int k3k_stream_destroy(void *stream)
     pthread_mutex_lock(&g_side_mu);
     for (int i = 0; i < g_nside; i++)
         if (g_side[i].caller == (hipStream_t)stream) {
-            (void)hipStreamSynchronize(g_side[i].side);
-            (void)hipEventDestroy(g_side[i].fork);
-            (void)hipEventDestroy(g_side[i].join);
-            (void)hipStreamDestroy(g_side[i].side);
+            for (int k = 0; k < 2; k++) {
+                (void)hipStreamSynchronize(g_side[i].side[k]);
+                (void)hipEventDestroy(g_side[i].fork[k]);
+                (void)hipEventDestroy(g_side[i].join[k]);
+                (void)hipStreamDestroy(g_side[i].side[k]);
+            }
             g_side[i] = g_side[--g_nside];
             break;
         }

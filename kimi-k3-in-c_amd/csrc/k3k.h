@@ -32,17 +32,21 @@ void *k3k_stream_create(void);
 int k3k_stream_destroy(void *stream);
 int k3k_cu_count(void);
 /* Graph capture of the work enqueued on `stream` (a created stream, not NULL). */
-/* k3k_fork: *side = a second stream that first waits for the work queued on stream;
- * k3k_join: stream waits for the work queued on the side stream since. */
+/* k3k_fork: *side = a second stream that first waits for the work queued on stream (which 0:
+ * used inside the device entry points; 1: the host entry points' own, so that the two can be
+ * open at once); k3k_join: stream waits for the work queued on that side stream since. */
 /* pinned host memory and events (host-side waits for part of a stream's work) */
 void *k3k_host_alloc(size_t bytes);
 void k3k_host_free(void *p);
+/* a copy kernel between device memory and k3k_host_alloc memory, either way: whole words, all
+ * 16-byte aligned; with add, dst = src + add as floats */
+int k3k_pin_copy(void *dst, const void *src, const float *add, size_t bytes, void *stream);
 void *k3k_event_create(void);
 int k3k_event_record(void *ev, void *stream);
 int k3k_event_sync(void *ev);
 int k3k_side_init(void);
-int k3k_fork(void *stream, void **side);
-int k3k_join(void *stream);
+int k3k_fork(void *stream, int which, void **side);
+int k3k_join(void *stream, int which);
 int k3k_graph_begin(void *stream);
 int k3k_graph_end(void *stream, void **exec);
 int k3k_graph_launch(void *exec, void *stream);
@@ -191,7 +195,11 @@ int k3k_gemv_f32(float *y, const float *x, const float *W, int in, int out, int 
                  void *stream);
 int k3k_gemv_bf16(float *y, const float *x, const uint16_t *W, int in, int out, int ntok,
                   int ldy, void *stream);
-/* The same for two tokens and more on the matrix cores (k3_tok.hip): W bf16 (bf16 1) or fp32,
+/* One token: y[o] = act(Wg[o][:] . x, Wu[o][:] . x), o < out, with the sums k3k_gemv_* form and
+ * k3k_act's activation; in % 8 == 0, all 16-byte aligned. */
+int k3k_gemv_glu(float *y, const float *x, const void *Wg, const void *Wu, int bf16, int in, int out, int act,
+                 float b1, float b2, void *stream);
+/* k3k_gemv_f32 / _bf16 for two tokens and more on the matrix cores (k3_tok.hip): W bf16 (bf16 1) or fp32,
  * where k3k_tok_ok holds (in % 8 == 0, x and W 16-byte aligned). k3k_gemv_* send their calls
  * there. */
 int k3k_tok_ok(const float *x, const void *W, int in, int ntok);

@@ -1,0 +1,60 @@
+# SPDX-License-Identifier: Apache-2.0
+"""k3_moe / k3_moe_prefill with every expert of the layer in the HBM bank (the experts then run
+from the bank's device table before the routing is back on the host) against the same calls with
+one expert missing from the bank until it is fetched, whose experts wait for the host: outputs,
+routing and the bank's counters."""
+import numpy as np
+import pytest
+
+from test_gpu_dense import say
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("T", [1, 2, 5, 70, 600])
+def test_resident_bank_same_as_fetched(gpu, wl, T):
+    say(f"case: resident bank T={T}")
+    cfg, W, ex = wl.latent_layer(1024, 512, 512, 24, 4, n_shared=1, tag="host.resident")
+    runs = {e: wl.expert_run(ex[e]) for e in ex}
+    x = wl.tokens(T, 1024, tag=f"host.resident.{T}")
+    keep = {}
+
+    @gpu.GETFN
+    def get(self, layer, e, out):
+        t = ex[e].t
+        keep[e] = t
+        q = out.contents
+        q.p1, q.s1, q.p3, q.s3, q.p2, q.s2 = [a.ctypes.data for a in t]
+        return 0
+
+    up = gpu.K3ExpertSrc(get, gpu.GETMANYFN(), gpu.GETFN(), None)
+    import ctypes as C
+    full = gpu.HbmBank(1, 24, 512, 512, 24)
+    part = gpu.HbmBank(1, 24, 512, 512, 24, upstream_ptr=C.addressof(up))
+    try:
+        for e in range(24):
+            full.put_run(0, e, runs[e])
+        for e in range(23):
+            part.put_run(0, e, runs[e])          # the last one comes from upstream when routed
+        for a in ("gate", "down", "up", "sh1", "sh3", "sh2"):
+            gpu.dev_register(W[a])
+        want = gpu.moe(x, cfg, W, 1, part.src, int(T > 1))
+        h0 = full.stats()
+        got = gpu.moe(x, cfg, W, 1, full.src, int(T > 1))
+        h1 = full.stats()
+        again = gpu.moe(x, cfg, W, 1, full.src, int(T > 1))
+        assert np.array_equal(got[0], want[0]) and np.array_equal(again[0], want[0])
+        assert np.array_equal(got[1], want[1]) and np.array_equal(got[2], want[2], equal_nan=True)
+        assert got[3] == want[3] == 0 and h1["misses"] == h0["misses"] and h1["hits"] > h0["hits"]
+        # the table follows the bank: another expert's bytes under id 3, then the right ones again
+        if T == 70:
+            full.put_run(0, 3, runs[7])
+            other = gpu.moe(x, cfg, W, 1, full.src, 1)
+            assert not np.array_equal(other[0], want[0])
+            full.put_run(0, 3, runs[3])
+            assert np.array_equal(gpu.moe(x, cfg, W, 1, full.src, 1)[0], want[0])
+    finally:
+        for a in ("gate", "down", "up", "sh1", "sh3", "sh2"):
+            gpu.dev_unregister(W[a])
+        full.destroy()
+        part.destroy()
