@@ -340,8 +340,8 @@ typedef struct {
  * multiples of 512: passes of 8 tokens, or more (moe_pass_tok) for larger batches. Other shapes
  * run the register-fed kernel (16, row-major bank only).
  *
- * Two pass lists on a tiled bank: one-term (prefill) activations at 8-32 tokens per expert on
- * average, two-term ones from 5. There 7 % of the experts of a uniform routing hold more than
+ * Two pass lists: one-term (prefill) activations at 8-32 tokens per expert on average (a tiled
+ * bank), two-term ones from 5. There 7 % of the experts of a uniform routing hold more than
  * 8 tokens and would stream their weights again; with fewer tokens the second list's two
  * launches and its fork, about 15 us, cost more than they save (64 tokens of the 128-expert
  * layer, 4 per expert: 266 us with one list, 282 with two). The prefill kernel addresses both
@@ -349,25 +349,26 @@ typedef struct {
 static int moe_two_lists(int T, int hidden, int inter, int n_experts, int topk, int prec, int layout)
 {
     const long N = (long)T * topk;
-    if (layout != K3D_LAYOUT_TILED || hidden % 512 || inter % 512) return 0;
-    if (prec == 1) return N >= 8L * n_experts && N < 32L * n_experts;
+    if (hidden % 512 || inter % 512) return 0;
+    if (prec == 1) return layout == K3D_LAYOUT_TILED && N >= 8L * n_experts && N < 32L * n_experts;
     return N >= 5L * n_experts && ((long long)N * inter + 256) * 4 < 0x7fff0000ll &&
            ((long long)T * hidden + 256) * 4 < 0x7fff0000ll;
 }
 
 /* Tokens per expert pass (of the first list). 8 for decode (fp32-accurate, weight streaming)
  * and where there is a second list, 16 when the widths are not multiples of 512; one-term
- * (prefill) activations take, for a tiled bank, 48 from 32 tokens per expert on average and 96
- * from 64; for a row-major bank 32 from 8. Sizing: a row-major bank's first list has at most
- * N / 32 (or N / 8) passes beyond one per expert; a tiled bank's at most N / 8 where there is
- * no second list, and one per expert where there is (its experts hold at most 8 assignments). */
+ * (prefill) activations take 48 from 32 tokens per expert on average and 96 from 64 (a row-major
+ * bank 96 from 32, and from 8 the streaming kernel's 32-token passes: there the prefill kernel's
+ * loads, a line per lane, cost more than the shorter passes, 512 tokens of 384 experts 2.51
+ * against 2.00 ms; from 32 on it is the faster one, 4096 tokens 5.74 against 6.07, 2048 tokens
+ * of 896 experts 5.46 against 6.34, 1000 of 128 experts 0.63 against 0.78). */
 static int moe_pass_tok(int T, int hidden, int inter, int n_experts, int topk, int prec, int layout)
 {
+    const long N = (long)T * topk;
     if (hidden % 512 || inter % 512) return 16;
-    if (prec == 1 && layout == K3D_LAYOUT_TILED && (long)T * topk >= 64L * n_experts) return 96;
-    if (prec == 1 && layout == K3D_LAYOUT_TILED && (long)T * topk >= 32L * n_experts) return 48;
-    if (moe_two_lists(T, hidden, inter, n_experts, topk, prec, layout)) return 8;
-    if (prec == 1 && (long)T * topk >= 8L * n_experts) return 32;
+    if (prec == 1 && N >= (layout == K3D_LAYOUT_TILED ? 64L : 32L) * n_experts) return 96;
+    if (prec == 1 && N >= 32L * n_experts) return 48;
+    if (prec == 1 && N >= 8L * n_experts && layout == K3D_LAYOUT_ROWS) return 32;
     return 8;
 }
 
@@ -379,15 +380,15 @@ static int moe_pass_tok(int T, int hidden, int inter, int n_experts, int topk, i
  * and the shorter one's double stages keep twice the weights in flight (512 tokens of the
  * 384-expert layer, skewed: 1.82 ms with 48, 1.70 with 32; 333 tokens through k3_moe_prefill
  * at 896 experts: 4.48 and 4.31). 16-token streaming passes for the first list instead were
- * slower (512 tokens of 896 experts 3.35 against 3.15 ms). (Config 4, 512
- * tokens with skewed routing: 309 experts of at most 32 assignments in 32-token passes and 21
- * hot ones in the second list took 1.47 ms for gate/up + down; 282 experts of at most 8 in
- * 8-token passes and 48 in the second list take 1.40 ms.) */
+ * slower (512 tokens of 896 experts 3.35 against 3.15 ms). (512 tokens with skewed routing,
+ * one term: 309 experts of at most 32 assignments in 32-token passes and 21 hot ones in the
+ * second list took 1.47 ms for gate/up + down; 282 experts of at most 8 in 8-token passes and
+ * 48 in the second list take 1.40 ms.) */
 static int moe_pass_tok2(int T, int hidden, int inter, int n_experts, int topk, int prec, int layout)
 {
     if (!moe_two_lists(T, hidden, inter, n_experts, topk, prec, layout)) return 0;
     if (prec == 1) return 96;
-    return (long)T * topk < 16L * n_experts ? 32 : 48;
+    return layout == K3D_LAYOUT_TILED && (long)T * topk < 16L * n_experts ? 32 : 48;
 }
 
 /* The decode path (k3k_mx_decode): at most 16 assignments, widths multiples of 512 up to
@@ -403,13 +404,12 @@ static size_t moe_layout(Carve *c, MoeWs *w, int T, int hidden, int inter, int n
 {
     const size_t N = (size_t)T * topk;
     const int maxjobs = (int)(N < (size_t)n_experts ? N : (size_t)n_experts);
-    w->max_passes = maxjobs + (int)(N / (size_t)moe_pass_tok(T, hidden, inter, n_experts, topk, prec,
-                                                                K3D_LAYOUT_ROWS)) + 1;
-    if (!moe_two_lists(T, hidden, inter, n_experts, topk, prec, K3D_LAYOUT_TILED)) {
-        const int pt = moe_pass_tok(T, hidden, inter, n_experts, topk, prec, K3D_LAYOUT_TILED);
-        const int mp = maxjobs + (int)(N / (size_t)pt) + 1;
-        if (mp > w->max_passes) w->max_passes = mp;
-    }
+    /* first list: one pass per expert beside a second list, else up to N / pass_tok full ones more */
+    const int pt[2] = {moe_pass_tok(T, hidden, inter, n_experts, topk, prec, K3D_LAYOUT_ROWS),
+                       moe_pass_tok(T, hidden, inter, n_experts, topk, prec, K3D_LAYOUT_TILED)};
+    w->max_passes = maxjobs;
+    if (!moe_two_lists(T, hidden, inter, n_experts, topk, prec, K3D_LAYOUT_ROWS))
+        w->max_passes += (int)(N / (size_t)(pt[0] < pt[1] ? pt[0] : pt[1])) + 1;
     w->xhi = (uint16_t *)take(c, (size_t)T * hidden * 2);
     w->xlo = prec == 0 ? (uint16_t *)take(c, (size_t)T * hidden * 2) : NULL;
     w->ahi = (uint16_t *)take(c, N * inter * 2);

@@ -1120,9 +1120,12 @@ __global__ __launch_bounds__(1024) void mx_decode_combine_kernel(K3kMxArgs a)
  * blocks = 4 steps of 128). K order inside a chunk: at step d, lane group g (lanes
  * 16g..16g+15) holds MX block 4d+g of its row (the MFMA's K permutation is free as long
  * as A and B agree). Weights come in one of two layouts:
- *   LAYOUT 0, row-major (the reference's): per step a lane loads its block's 16 bytes
- *     (a wave: 16 rows x 64 contiguous bytes), per chunk one 16-byte load of the row's
- *     16 scale bytes, of which it uses one per step;
+ *   LAYOUT 0, row-major (the reference's): a load of a wave takes 8 rows x 128 contiguous
+ *     bytes (consecutive lanes of a row), two loads a tile's next two steps, which pass
+ *     through a small LDS buffer of the wave to the lanes of their rows; the scale bytes of a
+ *     tile's chunk come in one 4-byte load per lane the same way. (Each lane loading its own
+ *     row's 16 bytes, neighbouring lanes in different rows, the L1 works a line per lane:
+ *     23 tokens of 896 experts 1181 us, 888 so.)
  *   LAYOUT 1, tiled (mx_tile_kernel, k3_tile_idx): the bytes of a 16-row tile's chunk
  *     stored in lane order, so a wave's load is 1 KB contiguous and a lane's four scale
  *     bytes of the chunk are one 4-byte load; the four tiles of a group lie side by side
@@ -1145,11 +1148,16 @@ void mx_moe_kernel(K3kMxArgs a)
     constexpr bool PACK = NS == 2 && PT <= 8 && NB == 1;     /* hi and lo in one column block */
     constexpr int RT = (MODE == K3K_MX_GATEUP) ? MT / 2 : MT;
     constexpr int KC = 512, SPC = 4, LDT = KC + 8;           /* LDS row: 16-byte pad */
-    /* tiled MXFP4 weights are streamed once per pass and non-temporal; row-major ones keep
-     * the default policy (a 128-byte line is consumed by two steps' loads) */
-    constexpr int WPOL = LAYOUT == 1 ? K3_LD_NT : K3_LD_DEFAULT;
+    /* MXFP4 codes are streamed once per pass, non-temporal (row-major scale bytes are not: a line
+     * of them serves eight chunks; with both non-temporal 23 tokens of 896 experts took 1049 us,
+     * with neither 969, with the codes 888) */
+    constexpr int WPOL = K3_LD_NT;
     constexpr int NRH = PT * NS;                             /* staged row-halves per chunk */
     constexpr int PPW = (NRH + NW - 1) / NW;                 /* row-halves per wave */
+    /* LAYOUT 0: a wave's transposition buffers, two of 16 rows x 128 bytes of codes, and a chunk's
+     * scale bytes of its tiles */
+    __shared__ uint4 tcode[LAYOUT == 0 ? NW : 1][LAYOUT == 0 ? 2 : 1][LAYOUT == 0 ? 128 : 1];
+    __shared__ __attribute__((aligned(16))) uint32_t tscale[LAYOUT == 0 ? NW : 1][LAYOUT == 0 ? MT * 64 : 1];
     /* row PT of each buffer/half stays zero: the B operand of absent token columns */
     __shared__ __attribute__((aligned(16))) uint16_t bsh[2][NS][PT + 1][LDT];
 
@@ -1201,9 +1209,10 @@ void mx_moe_kernel(K3kMxArgs a)
         for (int m = 0; m < MT; m++) {
             const int mt = (MODE == K3K_MX_GATEUP) ? (m % RT) : m;
             if (LAYOUT == 0) {
-                const int r = min(rb * rpg + wv * rpw + 16 * mt + r16, rows - 1);
-                poff[m] = (uint32_t)r * rstride + (uint32_t)g * 16u;
-                soff[m] = (uint32_t)r * (uint32_t)nblk;
+                /* (rows past the end lie beyond the buffers: zeros) */
+                const uint32_t r = (uint32_t)(rb * rpg + wv * rpw + 16 * mt);
+                poff[m] = (r + (uint32_t)(lane >> 3)) * rstride + (uint32_t)(lane & 7) * 16u;
+                soff[m] = (r + (uint32_t)(lane >> 2)) * (uint32_t)nblk + (uint32_t)(lane & 3) * 4u;
             } else {
                 const int t = min((rb * rpg + wv * rpw) / 16 + mt, ntile - 1);
                 poff[m] = k3_tile_idx(t, 0, nchunk) * 4096u + (uint32_t)lane * 16u;
@@ -1246,7 +1255,7 @@ void mx_moe_kernel(K3kMxArgs a)
          * c has consumed it. DEPTH 2: chunks alternate between two slots and step d of
          * chunk c+2 is loaded into chunk c's slot. Scales follow one chunk behind. */
         constexpr int NSLOT = DEPTH == 2 ? 2 : 1;
-        constexpr int SQN = MT * (LAYOUT == 0 ? 4 : 1);
+        constexpr int SQN = MT;
         uint4 qa[NSLOT][SPC][MT];
         uint32_t sq[SQN], sqn[SQN], sqnn[SQN];
         uint4 bst[PPW];
@@ -1272,7 +1281,7 @@ void mx_moe_kernel(K3kMxArgs a)
         };
         auto load_step = [&](int c, int d, auto slot) {
             constexpr int S = decltype(slot)::value;
-            const uint32_t bo = LAYOUT == 0 ? (uint32_t)c * 256u + (uint32_t)d * 64u
+            const uint32_t bo = LAYOUT == 0 ? (uint32_t)c * 256u + (uint32_t)(d >> 1) * 128u + (uint32_t)(d & 1) * 8u * rstride
                                             : (uint32_t)c * K3_TILE_CSTRIDE + (uint32_t)d * 1024u;
 #pragma unroll
             for (int m = 0; m < MT; m++)
@@ -1283,12 +1292,7 @@ void mx_moe_kernel(K3kMxArgs a)
 #pragma unroll
             for (int m = 0; m < MT; m++) {
                 const k3_rsrc rs = m < RT || MODE != K3K_MX_GATEUP ? rs0 : rs1;
-                if (LAYOUT == 0) {
-                    const uint4 v = k3_bload16<WPOL>(rs, c < nchunk ? soff[m] + (uint32_t)c * 16u : OOB);
-                    ss[4 * m] = v.x; ss[4 * m + 1] = v.y; ss[4 * m + 2] = v.z; ss[4 * m + 3] = v.w;
-                } else {
-                    ss[m] = k3_bload4<WPOL>(rs, c < nchunk ? soff[m] + (uint32_t)c * K3_TILE_SCSTRIDE : OOB);
-                }
+                ss[m] = k3_bload4<LAYOUT == 0 ? K3_LD_DEFAULT : WPOL>(rs, c < nchunk ? soff[m] + (uint32_t)c * (LAYOUT == 0 ? 16u : K3_TILE_SCSTRIDE) : OOB);
             }
         };
 
@@ -1317,8 +1321,40 @@ void mx_moe_kernel(K3kMxArgs a)
             load_b(c + 1);
             load_scales(c + DEPTH, DEPTH == 2 ? sqnn : sqn);
             if constexpr (PT <= 8) __builtin_amdgcn_sched_barrier(0);
+            uint4 sqv[LAYOUT == 0 ? MT : 1];               /* LAYOUT 0: row r16's 16 scale bytes */
+            uint4 frag[LAYOUT == 0 ? 2 : 1][LAYOUT == 0 ? MT : 1];
+            if constexpr (LAYOUT == 0) {
+#pragma unroll
+                for (int m = 0; m < MT; m++) tscale[wv][64 * m + lane] = sq[m];
+#pragma unroll
+                for (int m = 0; m < MT; m++) sqv[m] = *reinterpret_cast<const uint4 *>(&tscale[wv][64 * m + 4 * r16]);
+            }
 #pragma unroll
             for (int d = 0; d < SPC; d++) {
+                if constexpr (LAYOUT == 0) {
+                    /* two steps at once, tile after tile: the loaded words (lane l: row l / 8 of
+                     * the tile's half, 16-byte piece l % 8 of 128 bytes) into the buffer, a row's
+                     * piece p at p ^ (row / 2 % 8), and the fragments of both steps (lane (g, r16):
+                     * pieces g and 4 + g of row r16) back from it; LDS operations of one wave
+                     * complete in order. The registers take chunk c + DEPTH. */
+                    if ((d & 1) == 0) {
+#pragma unroll
+                        for (int m = 0; m < MT; m++) {
+                            uint4 *tb = tcode[wv][m & 1];
+#pragma unroll
+                            for (int h = 0; h < 2; h++) {
+                                const int row = 8 * h + (lane >> 3);
+                                tb[row * 8 + ((lane & 7) ^ ((row >> 1) & 7))] = qa[S][d + h][m];
+                            }
+                            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                            for (int h = 0; h < 2; h++) frag[h][m] = tb[r16 * 8 + ((4 * h + g) ^ ((r16 >> 1) & 7))];
+                            __builtin_amdgcn_wave_barrier();
+                        }
+                        load_step(c + DEPTH, d, slot);
+                        load_step(c + DEPTH, d + 1, slot);
+                    }
+                }
                 /* B operand: token columns (or the zero row), block 4d+g of the chunk */
                 uint4 bh[NB][4], bl[NB][4];
 #pragma unroll
@@ -1335,12 +1371,16 @@ void mx_moe_kernel(K3kMxArgs a)
                 float so[MT];
 #pragma unroll
                 for (int m = 0; m < MT; m++) {
-                    const uint32_t sraw = LAYOUT == 0 ? (sq[4 * m + d] >> (8 * g)) & 0xFFu
-                                                      : (sq[m] >> (8 * d)) & 0xFFu;
+                    uint32_t sraw;
+                    if constexpr (LAYOUT == 0)
+                        sraw = ((d == 0 ? sqv[m].x : d == 1 ? sqv[m].y : d == 2 ? sqv[m].z : sqv[m].w) >> (8 * g)) & 0xFFu;
+                    else
+                        sraw = (sq[m] >> (8 * d)) & 0xFFu;
                     /* NaN byte: the block is 0 (a tiled bank stores it as zeros, scale 127) */
                     const bool nanb = LAYOUT == 0 && sraw == 255u;
                     const uint32_t keep = nanb ? 0u : ~0u;       /* a mask, not a branch */
-                    qq[m] = qa[S][d][m];
+                    if constexpr (LAYOUT == 0) qq[m] = frag[d & 1][m];
+                    else qq[m] = qa[S][d][m];
                     qq[m].x &= keep;
                     qq[m].y &= keep;
                     qq[m].z &= keep;
@@ -1360,7 +1400,7 @@ void mx_moe_kernel(K3kMxArgs a)
                                 acc[m][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, k3_as_bf16x8(bl[nb][pp]), acc[m][nb], 0, 0, 0);
                         }
                     }
-                load_step(c + DEPTH, d, slot);
+                if (LAYOUT != 0) load_step(c + DEPTH, d, slot);
             }
             if (more) store_b(buf ^ 1);
 #pragma unroll
@@ -1435,7 +1475,7 @@ int launch_moe(const K3kMxArgs *a, int grid, hipStream_t st)
 
 /* ---- prefill: large token passes -------------------------------------------------------
  * mx_prefill_kernel: GATEUP / DOWN for passes of many tokens, weights in the tiled MXFP4
- * layout: up to 16*NB tokens with the activations as single bf16 terms (NS 1, the prefill
+ * layout (LAYOUT 1) or the reference's rows (LAYOUT 0: each lane loads its own row's bytes): up to 16*NB tokens with the activations as single bf16 terms (NS 1, the prefill
  * precision), 8*NB with two (NS 2, fp32-accurate). An item is (pass, row block); a wave owns
  * MT tiles of 16 weight rows and all the pass's tokens, so every dequantized weight fragment
  * feeds NB MFMAs and each weight byte is read once per pass. With two terms the NB matrix
@@ -1480,11 +1520,12 @@ __device__ __forceinline__ uint32_t k3_bload4s(k3_rsrc r, uint32_t voff, uint32_
     return __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0);
 }
 
-template <int MODE, int MT, int NB, int SPC, int NW, int NS>
+template <int MODE, int MT, int NB, int SPC, int NW, int NS, int LAYOUT>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 8)))
 void mx_prefill_kernel(K3kMxArgs a)
 {
     static_assert(NB % NS == 0, "column blocks: NS terms of NB / NS token blocks");
+    static_assert(LAYOUT == 1 || SPC == 1, "row-major: one dword of scales per stage");
     constexpr int KC = 128 * SPC, PT = 16 * NB / NS, PR = KC / 8;
     constexpr int RT = (MODE == K3K_MX_GATEUP) ? MT / 2 : MT;
     constexpr int PRP = PR + 1;                               /* slots per token row */
@@ -1524,7 +1565,8 @@ void mx_prefill_kernel(K3kMxArgs a)
     /* lane's B fragment slot: token r16 (+16 per block), piece 16 (u / 4) + 4 g + u % 4 of
      * the stage (the 8 columns matching the weight codes it holds) */
     const int lrd = r16 * PRP + 4 * g;
-    const uint32_t lvoff = (uint32_t)lane * 16u, lsoff = (uint32_t)lane * 4u;
+    const uint32_t lvoff = LAYOUT == 1 ? (uint32_t)lane * 16u : (uint32_t)r16 * rstride + (uint32_t)g * 16u;
+    const uint32_t lsoff = LAYOUT == 1 ? (uint32_t)lane * 4u : (uint32_t)r16 * (uint32_t)nblk;
     /* Prefetches past the last stage are issued too, so that every wait counts exactly the
      * loads issued after the one it waits for: DOWN's at a per-lane offset of 2^31, beyond
      * every buffer (zeros, no data moved); GATEUP's re-read the last stage, because the
@@ -1563,7 +1605,7 @@ void mx_prefill_kernel(K3kMxArgs a)
         const int tok0 = a.pass_tp[pass] * PT;
         const int ntok = __builtin_amdgcn_readfirstlane(min(PT, a.job_cnt[j] - tok0));
         const ExpertQDev q = reinterpret_cast<const ExpertQDev *>(a.bank)[e];
-        const uint32_t prow = k3_tile_prows(rows);
+        const uint32_t prow = LAYOUT == 1 ? k3_tile_prows(rows) : (uint32_t)rows;
         const uint32_t pbytes = prow * rstride;
         const uint32_t sbytes = prow * nblk;
         k3_rsrc rp0, rp1, rs0, rs1;
@@ -1581,8 +1623,8 @@ void mx_prefill_kernel(K3kMxArgs a)
         for (int m = 0; m < MT; m++) {
             const int mt = (MODE == K3K_MX_GATEUP) ? (m % RT) : m;
             const int t = min((rb * rpg + wv * rpw) / 16 + mt, ntile - 1);
-            ptile[m] = k3_tile_idx(t, 0, nchunk) * 4096u;
-            stile[m] = k3_tile_idx(t, 0, nchunk) * 256u;
+            ptile[m] = LAYOUT == 1 ? k3_tile_idx(t, 0, nchunk) * 4096u : (uint32_t)t * 16u * rstride;
+            stile[m] = LAYOUT == 1 ? k3_tile_idx(t, 0, nchunk) * 256u : (uint32_t)t * 16u * (uint32_t)nblk;
         }
         /* DMA sources: instruction i of this wave fills slots 64 (wv + NW i) + lane */
         /* (two terms: one descriptor over both arrays, xlo after xhi; column p is token
@@ -1615,7 +1657,7 @@ void mx_prefill_kernel(K3kMxArgs a)
             constexpr int S = decltype(slot)::value;
             /* the 128-column step s of the tile: chunk s / 4, step s % 4 */
             const uint32_t s = (uint32_t)min(c * SPC + d, nstage * SPC - 1);
-            const uint32_t bo = (s >> 2) * K3_TILE_CSTRIDE + (s & 3u) * 1024u;
+            const uint32_t bo = LAYOUT == 1 ? (s >> 2) * K3_TILE_CSTRIDE + (s & 3u) * 1024u : s * 64u;
             const uint32_t vo = (MODE == K3K_MX_GATEUP || c < nstage) ? lvoff : OOB;
 #pragma unroll
             for (int m = 0; m < MT; m++)
@@ -1625,7 +1667,8 @@ void mx_prefill_kernel(K3kMxArgs a)
          * (c clamped: past the end re-reads the last stage) */
         auto load_scales = [&](int c, auto slot) {
             constexpr int S = decltype(slot)::value;
-            const uint32_t so = (uint32_t)(min(c, nstage - 1) * SPC >> 2) * K3_TILE_SCSTRIDE;
+            const uint32_t so = LAYOUT == 1 ? (uint32_t)(min(c, nstage - 1) * SPC >> 2) * K3_TILE_SCSTRIDE
+                                            : (uint32_t)min(c, nstage - 1) * 4u;
             const uint32_t vo = (MODE == K3K_MX_GATEUP || c < nstage) ? lsoff : OOB;
 #pragma unroll
             for (int m = 0; m < MT; m++)
@@ -1640,9 +1683,13 @@ void mx_prefill_kernel(K3kMxArgs a)
 #pragma unroll
             for (int m = 0; m < MT; m++) {
                 /* a NaN-scale block is stored as zero codes with scale 127 in the tiled bank */
-                const uint32_t sraw = (sw[m] >> (8 * ((c * SPC + (u >> 2)) & 3))) & 0xFFu;
+                uint32_t sraw = (sw[m] >> (LAYOUT == 1 ? 8 * ((c * SPC + (u >> 2)) & 3) : 8 * g)) & 0xFFu;
                 const uint4 qv = qs[u >> 2][m];
-                const uint32_t codes = (u & 3) == 0 ? qv.x : (u & 3) == 1 ? qv.y : (u & 3) == 2 ? qv.z : qv.w;
+                uint32_t codes = (u & 3) == 0 ? qv.x : (u & 3) == 1 ? qv.y : (u & 3) == 2 ? qv.z : qv.w;
+                if (LAYOUT == 0) {                         /* NaN byte: the block is 0 */
+                    codes = sraw == 255u ? 0u : codes;
+                    sraw = sraw == 255u ? 127u : sraw;
+                }
                 dst[m] = k3_dequant8_bf16(codes, k3_e8m0_operand(sraw));
             }
         };
@@ -1819,12 +1866,12 @@ void mx_prefill_kernel(K3kMxArgs a)
     }
 }
 
-template <int MODE, int MT, int NB, int SPC, int NW, int NS = 1>
+template <int MODE, int MT, int NB, int SPC, int NW, int NS = 1, int LAYOUT = 1>
 int launch_prefill(const K3kMxArgs *a, int grid, hipStream_t st)
 {
     K3kMxArgs b = *a;
     b.stamps = k3k_stamps_take(MODE == K3K_MX_GATEUP ? 3 : 4, grid);
-    hipLaunchKernelGGL((mx_prefill_kernel<MODE, MT, NB, SPC, NW, NS>), dim3(grid), dim3(64 * NW), 0, st, b);
+    hipLaunchKernelGGL((mx_prefill_kernel<MODE, MT, NB, SPC, NW, NS, LAYOUT>), dim3(grid), dim3(64 * NW), 0, st, b);
     K3K_LAUNCH_CHECK("mx_prefill launch");
     return 0;
 }
@@ -1962,9 +2009,12 @@ extern "C" int k3k_mx_gemm(int mode, const K3kMxArgs *a, void *stream)
          * per CU); weights two stages ahead; each dequantized weight fragment feeds 3 or 6
          * MFMA column blocks. Two activation terms: 48-token passes of 6 column blocks, or 32-token
          * ones of 4 with K staged 256 columns at a time (twice the weights in flight) */
-        if (a->K % 512 || (a->nsplit != 1 && a->pass_tok == 96) || a->layout != 1)
-            return k3k_fail("mx_moe: 48/96-token passes need K % 512 == 0, bf16 activations (96) "
-                            "and a tiled bank", hipErrorInvalidValue);
+        const bool tiled = a->layout == 1;
+        const bool one = a->nsplit == 1;
+        if (a->K % 512 || (a->pass_tok == 96 && !one) || (a->pass_tok == 32 && (one || !tiled)) ||
+            (a->pass_tok == 48 && one && !tiled))
+            return k3k_fail("mx_moe: passes of 96 tokens need one activation term, of 32 two and a tiled bank, of 48 "
+                            "two or a tiled bank, and K % 512 == 0", hipErrorInvalidValue);
         if (a->nsplit == 2 &&
             (a->xlo < a->xhi || (uint64_t)((const char *)a->xlo - (const char *)a->xhi) +
                                         (uint64_t)a->n_xrows * a->K * 2 >= 0x80000000u))
@@ -1975,9 +2025,15 @@ extern "C" int k3k_mx_gemm(int mode, const K3kMxArgs *a, void *stream)
         const int rpg = gu ? 256 : 512;
         const long items = (long)a->max_passes * ((a->rows + rpg - 1) / rpg);
         const int grid = (int)(items < (long)cus ? (items > 0 ? items : 1) : (long)cus);
+        if (a->pass_tok == 96 && !tiled)
+            return gu ? launch_prefill<K3K_MX_GATEUP, 4, 6, 1, 8, 1, 0>(a, grid, st)
+                      : launch_prefill<K3K_MX_DOWN, 4, 6, 1, 8, 1, 0>(a, grid, st);
         if (a->pass_tok == 96)
             return gu ? launch_prefill<K3K_MX_GATEUP, 4, 6, 1, 8>(a, grid, st)
                       : launch_prefill<K3K_MX_DOWN, 4, 6, 1, 8>(a, grid, st);
+        if (!one && !tiled)
+            return gu ? launch_prefill<K3K_MX_GATEUP, 4, 6, 1, 8, 2, 0>(a, grid, st)
+                      : launch_prefill<K3K_MX_DOWN, 4, 6, 1, 8, 2, 0>(a, grid, st);
         if (a->nsplit == 2 && a->pass_tok == 32)
             return gu ? launch_prefill<K3K_MX_GATEUP, 4, 4, 2, 8, 2>(a, grid, st)
                       : launch_prefill<K3K_MX_DOWN, 4, 4, 2, 8, 2>(a, grid, st);
@@ -1988,21 +2044,16 @@ extern "C" int k3k_mx_gemm(int mode, const K3kMxArgs *a, void *stream)
                   : launch_prefill<K3K_MX_DOWN, 4, 3, 2, 8>(a, grid, st);
     }
     if (a->pass_tok == 32) {
-        /* prefill: 32-token passes, two MFMA column blocks per weight fragment, activations
-         * as one bf16 term (the bf16-MFMA prefill precision) */
-        if (a->K % 512 || a->nsplit != 1)
-            return k3k_fail("mx_moe: 32-token passes need K % 512 == 0 and bf16 activations",
+        /* a row-major bank's moderate prefill batches: two MFMA column blocks per weight fragment */
+        if (a->K % 512 || a->layout != 0)
+            return k3k_fail("mx_moe: 32-token passes of one term need K % 512 == 0 and a row-major bank",
                             hipErrorInvalidValue);
         const bool gu = mode == K3K_MX_GATEUP;
         const int rpg = gu ? 128 : 256;
         const long items = (long)a->max_passes * ((a->rows + rpg - 1) / rpg);
         const int grid = (int)(items < (long)cus * 4 ? (items > 0 ? items : 1) : (long)cus * 4);
-        const bool tiled = a->layout == 1;
-        if (gu)
-            return tiled ? launch_moe<K3K_MX_GATEUP, 4, 1, 32, 4, 2, 1, 1, 2>(a, grid, st)
-                         : launch_moe<K3K_MX_GATEUP, 4, 1, 32, 4, 2, 0, 1, 2>(a, grid, st);
-        return tiled ? launch_moe<K3K_MX_DOWN, 4, 1, 32, 4, 2, 1, 1, 2>(a, grid, st)
-                     : launch_moe<K3K_MX_DOWN, 4, 1, 32, 4, 2, 0, 1, 2>(a, grid, st);
+        return gu ? launch_moe<K3K_MX_GATEUP, 4, 1, 32, 4, 1, 0, 1, 2>(a, grid, st)
+                  : launch_moe<K3K_MX_DOWN, 4, 1, 32, 4, 1, 0, 1, 2>(a, grid, st);
     }
     if (a->pass_tok == 8) {
         /* LDS-staged expert kernel: K % 512 == 0. Items are 4 waves x MT tiles of 16 rows;
