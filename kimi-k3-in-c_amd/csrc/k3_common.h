@@ -165,6 +165,11 @@ __device__ __forceinline__ uint32_t k3_bload4(k3_rsrc r, uint32_t off)
 {
     return __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, POL);
 }
+template <int POL = K3_LD_DEFAULT>
+__device__ __forceinline__ uint32_t k3_bload1(k3_rsrc r, uint32_t off)
+{
+    return __builtin_amdgcn_raw_buffer_load_b8(r, off, 0, POL);
+}
 
 /* 16 bytes per lane from a buffer straight into LDS (buffer_load_dwordx4 ... lds): lane L
  * writes lds_row + 16 L, where lds_row is wave-uniform; counts against vmcnt. The builtin

@@ -17,6 +17,13 @@
  *     (Two rounded terms, as the expert kernels use, would lose 7 bits.) bf16 ends at 2^-133,
  *     so bits of x below that are dropped: only an |x| under 2^-109 has any.
  *   fp32 weights: v_mfma_f32_16x16x4_f32 on the values as they are.
+ *   MXFP4 weights (k3_matmul_mxfp4 of the reference for three tokens and more): the codes are
+ *     exact in bf16 under their block's scale; x comes as two rounded bf16 terms, the entry
+ *     point's precision. The expert streaming kernel, which reads the weights once per 16 or 32
+ *     tokens through a register ring, took 16 / 39 / 273 us for 7168 -> 2048 at 8 / 64 / 512
+ *     tokens and 3575 at 512 of 12288 -> 16384; here 11.5 / 22 / 54 and 635. K of any multiple
+ *     of 32: the scales come a byte at a time, since a row's start is at no multiple of 4 (dwords
+ *     where K % 128 == 0: 11.1 / 21 / 52 and 617, not worth a second kernel).
  *
  * A workgroup owns MT tiles of 16 rows x N8 groups of 8 tokens; its KW waves split K, and no
  * barrier joins them until their sums meet in LDS (added in wave order, so the result does
@@ -65,11 +72,18 @@ __device__ __forceinline__ void k3_tok_for(F &&f)
 
 typedef uint32_t k3_u32x4 __attribute__((ext_vector_type(4)));
 
+enum { TOK_F32 = 0, TOK_BF16 = 1, TOK_MX = 2 };       /* weights */
+
 struct TokArgs {
     float *y;
-    const float *x;
-    const void *W;
-    int in, out, ntok, ldy;
+    const float *x;                       /* fp32 activations, or */
+    const uint16_t *xhi;                  /* their two bf16 terms, lo_off bytes apart */
+    uint32_t lo_off;
+    const void *W, *W2;                   /* W2: GLU's up matrix */
+    const uint8_t *scales;                /* MX */
+    int in, out, ntok, ldy, accumulate;
+    int act, rpt;                         /* GLU: activation, rows of each matrix per workgroup */
+    float b1, b2;
     int ntt, items, per_xcd;              /* token blocks, workgroups with work, per XCD */
 };
 
@@ -106,37 +120,54 @@ __device__ __forceinline__ void tok_cut(k3_u32x4 a, k3_u32x4 b, uint4 &h, uint4 
     l = make_uint4(up(q[0], q[1]), up(q[2], q[3]), up(q[4], q[5]), up(q[6], q[7]));
 }
 
-/* BF: bf16 weights, else fp32. Stages of 32 columns. */
-template <int BF, int MT, int N8, int KW, int ST>
+/* Stages of 32 columns. WT: the weights' type; XT 0: fp32 activations, 1: two bf16 terms.
+ * GLU: tiles 0 and 1 are rpt rows of W and the same rows of W2, y = act(tile 0, tile 1).
+ * WT MX: the codes come 128 columns at a time (a piece is a block of 32) into buffers of their
+ * own, one chunk ahead, and their scale bytes into registers (lane: row r16, block g; a permute
+ * hands a stage's to its rows' lanes); lane group g takes dword g of the block a stage
+ * multiplies, which is columns 8g .. 8g+7. */
+template <int WT, int XT, int GLU, int MT, int N8, int KW, int ST>
 __global__ __launch_bounds__(64 * KW) void tok_gemm_kernel(TokArgs a)
 {
     constexpr int NB = (N8 + 1) / 2;               /* matrix column blocks of 16 tokens */
-    constexpr int ES = BF ? 2 : 4;                 /* bytes per weight */
+    constexpr int BF = WT != TOK_F32, MX = WT == TOK_MX;
+    constexpr int ES = WT == TOK_F32 ? 4 : 2;      /* bytes per weight (not MX) */
     constexpr int PRW = 2 * ES, PRX = 8;           /* 16-byte pieces per row and stage */
     constexpr int RLW = 16 / PRW, RLX = 2;         /* rows to 256 bytes of LDS */
-    constexpr int SLW = 16 * PRW;                  /* slots per row tile (64 per token group) */
+    constexpr int SLW = MX ? 0 : 16 * PRW;         /* slots per row tile (64 per token group) */
     constexpr int WSL = MT * SLW + N8 * 64;        /* slots per wave and stage */
     constexpr int ND = WSL / 64;                   /* copy instructions per wave and stage */
     constexpr uint32_t OOB = 0x80000000u;
     static_assert(ST >= 2 && ST <= 4 && ND * (ST - 1) < 64, "stages, vmcnt field");
-    static_assert((KW - 1) * MT * NB * 64 <= KW * WSL, "the sums fit stage array 0");
+    static_assert(!MX || ST != 3, "eight stages to a loop");
+    static_assert(!GLU || (MT == 2 && !MX), "gate and up tiles");
+    constexpr int RED = (KW - 1) * MT * NB * 64;   /* the waves' sums, in stage array 0 */
+    constexpr int B0 = RED > KW * WSL ? RED : KW * WSL;
     /* an array per stage of a plain vector type, read at one integer index: the compiler then
      * tells a copy into one array from reads of another (through longer pointer chains it does
      * not, and waits for every copy in flight before each read) */
-    __shared__ __attribute__((aligned(1024))) k3_u32x4 b0[KW * WSL], b1[KW * WSL];
+    __shared__ __attribute__((aligned(1024))) k3_u32x4 b0[B0], b1[KW * WSL];
     __shared__ __attribute__((aligned(1024))) k3_u32x4 b2[ST > 2 ? KW * WSL : 1], b3[ST > 3 ? KW * WSL : 1];
+    __shared__ __attribute__((aligned(1024))) uint32_t w0[MX ? KW * MT * 256 : 1], w1[MX ? KW * MT * 256 : 1];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r16 = lane & 15, g = lane >> 4;
     const int item = (blockIdx.x % K3_NXCD) * a.per_xcd + (int)blockIdx.x / K3_NXCD;
     if (item >= a.items) return;
     const int tb = item % a.ntt, rb = item / a.ntt;
-    const int row0 = rb * 16 * MT, tok0 = tb * 8 * N8;
-    const int nrow = min(a.out - row0, 16 * MT), ntok = min(a.ntok - tok0, 8 * N8);
-    const k3_rsrc rw = k3_make_rsrc((const char *)a.W + (size_t)row0 * a.in * ES, (uint32_t)nrow * (uint32_t)a.in * ES);
-    const k3_rsrc rx = k3_make_rsrc(a.x + (size_t)tok0 * a.in, (uint32_t)ntok * (uint32_t)a.in * 4u);
+    const int row0 = rb * (GLU ? a.rpt : 16 * MT), tok0 = tb * 8 * N8;
+    const int nrow = min(a.out - row0, GLU ? a.rpt : 16 * MT), ntok = min(a.ntok - tok0, 8 * N8);
+    const size_t wrow = MX ? (size_t)a.in / 2 : (size_t)a.in * ES;       /* bytes per weight row */
+    const k3_rsrc rw = k3_make_rsrc((const char *)a.W + row0 * wrow, (uint32_t)(nrow * wrow));
+    const k3_rsrc rw2 = k3_make_rsrc(GLU ? (const char *)a.W2 + row0 * wrow : (const char *)a.W, GLU ? (uint32_t)(nrow * wrow) : 0u);
+    const k3_rsrc rs = k3_make_rsrc(MX ? a.scales + (size_t)row0 * (a.in / 32) : nullptr, MX ? (uint32_t)nrow * (uint32_t)(a.in / 32) : 0u);
+    const k3_rsrc rx = XT ? k3_make_rsrc(a.xhi + (size_t)tok0 * a.in, a.lo_off + (uint32_t)ntok * (uint32_t)a.in * 2u)
+                          : k3_make_rsrc(a.x + (size_t)tok0 * a.in, (uint32_t)ntok * (uint32_t)a.in * 4u);
+    /* the wave's share, whole chunks of MX codes */
+    constexpr int U = MX ? 4 : 1;
     const int nst = (a.in + 31) / 32;
-    const int s0 = wv * nst / KW, s1 = (wv + 1) * nst / KW;
+    const int nch = (nst + U - 1) / U;
+    const int s0 = wv * nch / KW * U, s1 = min((wv + 1) * nch / KW * U, nst);
     /* copy instruction i fills slots 64 i + lane: its lane's source row and piece. Rows and
      * tokens past the end, pieces past K and stages past the share read at 2^31 and more,
      * beyond the buffer: zeros, no data moved. */
@@ -147,9 +178,34 @@ __global__ __launch_bounds__(64 * KW) void tok_gemm_kernel(TokArgs a)
         const int sl = 64 * i + lane - (isw ? 0 : MT * SLW);
         const int pr = isw ? PRW : PRX, row = sl / pr;
         const int p = (sl % pr) ^ ((row / (isw ? RLW : RLX)) & (pr - 1));
-        voff[i] = row < (isw ? nrow : ntok) ? (uint32_t)row * (uint32_t)a.in * (isw ? ES : 4) + 16u * p : OOB;
-        col[i] = p * (isw ? 16 / ES : 4);
+        const int wr = GLU ? row & 15 : row;
+        if (isw) {
+            voff[i] = wr < nrow ? (uint32_t)wr * (uint32_t)a.in * ES + 16u * p : OOB;
+            col[i] = p * (16 / ES);
+        } else if (XT) {                           /* pieces 0-3: hi, 4-7: lo */
+            voff[i] = row < ntok ? (uint32_t)row * (uint32_t)a.in * 2u + 16u * (p & 3) + (p >> 2) * a.lo_off : OOB;
+            col[i] = (p & 3) * 8;
+        } else {
+            voff[i] = row < ntok ? (uint32_t)row * (uint32_t)a.in * 4u + 16u * p : OOB;
+            col[i] = p * 4;
+        }
     }
+    /* MX: a tile's chunk copy (slot lane: row lane / 4, block mb = (lane % 4) ^ (row / 4 % 4)) */
+    const int mb = (lane & 3) ^ ((lane >> 4) & 3);
+    const uint32_t mo = (uint32_t)(lane >> 2) * (uint32_t)(a.in / 2) + 16u * mb;
+    const uint32_t so = (uint32_t)r16 * (uint32_t)(a.in / 32) + g;
+    uint32_t sc[2][MT];
+    auto copy_w = [&](int c, auto slot) {
+        constexpr int S = decltype(slot)::value;
+        const bool inw = 4 * c + mb < s1, ins = 4 * c + g < s1;
+#pragma unroll
+        for (int m = 0; m < MT; m++) {
+            const uint32_t ro = 16u * m;
+            uint32_t *d = S ? w1 : w0;
+            k3_dma16(rw, &d[(wv * MT + m) * 256], inw && ro + (lane >> 2) < (uint32_t)nrow ? mo + ro * (uint32_t)(a.in / 2) + 64u * c : OOB, 0);
+            sc[S][m] = k3_bload1(rs, ins && ro + r16 < (uint32_t)nrow ? so + ro * (uint32_t)(a.in / 32) + 4u * c : OOB);
+        }
+    };
     auto buf = [&](auto slot) -> k3_u32x4 * {
         constexpr int S = decltype(slot)::value;
         if constexpr (S == 0) return b0;
@@ -163,8 +219,9 @@ __global__ __launch_bounds__(64 * KW) void tok_gemm_kernel(TokArgs a)
         const uint32_t ss = (uint32_t)min(s, nst - 1);
 #pragma unroll
         for (int i = 0; i < ND; i++) {
-            const bool isw = i < MT * SLW / 64;
-            k3_dma16(isw ? rw : rx, &d[wv * WSL + 64 * i], col[i] < left ? voff[i] : OOB, ss * (32u * (isw ? ES : 4)));
+            const bool isw = i < MT * SLW / 64, up = GLU && i >= SLW / 64;
+            k3_dma16(isw ? (up ? rw2 : rw) : rx, &d[wv * WSL + 64 * i], col[i] < left ? voff[i] : OOB,
+                     ss * (32u * (isw ? ES : XT ? 2 : 4)));
         }
     };
     /* Sums in two levels, so that rounding grows with the square root of K's parts: bf16, the
@@ -181,30 +238,58 @@ __global__ __launch_bounds__(64 * KW) void tok_gemm_kernel(TokArgs a)
         for (int b = 0; b < NB; b++) acc[m][b] = zero;
     /* the slots of this lane's pieces in row tile 0 and token block 0 */
     constexpr int NPW = BF ? 1 : 2;
-    int iw[NPW], ix[2], il[2];
+    int iw[MX ? 4 : NPW], ix[2], il[2];
+    if constexpr (MX) {
 #pragma unroll
-    for (int h = 0; h < NPW; h++) iw[h] = wv * WSL + r16 * PRW + ((NPW * g + h) ^ ((r16 / RLW) & (PRW - 1)));
+        for (int q = 0; q < 4; q++) iw[q] = wv * MT * 256 + (r16 * 4 + (q ^ (r16 >> 2))) * 4 + g;
+    } else {
+#pragma unroll
+        for (int h = 0; h < NPW; h++) iw[h] = wv * WSL + r16 * PRW + ((NPW * g + h) ^ ((r16 / RLW) & (PRW - 1)));
+    }
 #pragma unroll
     for (int h = 0; h < 2; h++) {
-        ix[h] = wv * WSL + MT * SLW + r16 * PRX + ((2 * g + h) ^ ((r16 / RLX) & (PRX - 1)));
+        ix[h] = wv * WSL + MT * SLW + r16 * PRX + ((XT ? 4 * h + g : 2 * g + h) ^ ((r16 / RLX) & (PRX - 1)));
         /* the last block of an odd N8 holds 8 tokens: columns 8..15 read some of its slots
          * again (a result column depends on its own operand column only, and these go unused) */
         il[h] = N8 & 1 ? ix[h] - (r16 & 8) * PRX : ix[h];
     }
-    auto comp = [&](auto slot) {
-        constexpr int S = decltype(slot)::value;
+    auto comp = [&](auto slot, auto step) {
+        constexpr int S = decltype(step)::value;       /* of the unrolled loop */
         const k3_u32x4 *d = buf(slot);
         k3_u32x4 w[MT][NPW];
 #pragma unroll
-        for (int m = 0; m < MT; m++)
+        for (int m = 0; m < MT; m++) {
+            if constexpr (MX) {
+                const uint32_t *wd = (S >> 2) & 1 ? w1 : w0;
+                uint32_t codes = wd[iw[S & 3] + m * 256], ss = (uint32_t)__builtin_amdgcn_ds_bpermute((16 * (S & 3) + r16) * 4, (int)sc[(S >> 2) & 1][m]);
+                codes = ss == 255u ? 0u : codes;       /* NaN byte: the block is 0 */
+                ss = ss == 255u ? 127u : ss;
+                w[m][0] = __builtin_bit_cast(k3_u32x4, k3_dequant8_bf16(codes, k3_e8m0_operand(ss)));
+            } else {
 #pragma unroll
-            for (int h = 0; h < NPW; h++) w[m][h] = d[iw[h] + m * SLW];
+                for (int h = 0; h < NPW; h++) w[m][h] = d[iw[h] + m * SLW];
+            }
+        }
         k3_u32x4 xv[NB][2];
 #pragma unroll
         for (int b = 0; b < NB; b++)
 #pragma unroll
             for (int h = 0; h < 2; h++) xv[b][h] = d[(b + 1 < NB ? ix[h] : il[h]) + b * 128];
-        if constexpr (BF) {
+        if constexpr (BF && XT) {
+#pragma unroll
+            for (int b = 0; b < NB; b++) {
+#pragma unroll
+                for (int k = 1; k >= 0; k--)
+#pragma unroll
+                    for (int m = 0; m < MT; m++)
+                        seg[m][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(k3_bf16x8, w[m][0]),
+                                                                            __builtin_bit_cast(k3_bf16x8, xv[b][k]),
+                                                                            S % SEG == 0 && k == 1 ? zero : seg[m][b], 0, 0, 0);
+                if (S % SEG == SEG - 1)
+#pragma unroll
+                    for (int m = 0; m < MT; m++) acc[m][b] += seg[m][b];
+            }
+        } else if constexpr (BF) {
             uint4 t[2][3];
             tok_cut(xv[0][0], xv[0][1], t[0][0], t[0][1], t[0][2]);
 #pragma unroll
@@ -243,16 +328,21 @@ __global__ __launch_bounds__(64 * KW) void tok_gemm_kernel(TokArgs a)
     constexpr int NW = ND * (ST - 1);
     constexpr int WAIT_STAGE = (NW & 15) | (7 << 4) | (15 << 8) | ((NW >> 4) << 14);
     constexpr int WAIT_LDS = 15 | (7 << 4) | (3 << 14);
+    /* MX: the chunk copies lie between stage copies, so a stage's wait lets fewer stages be in
+     * flight, never more; a chunk's were issued before its first stage's. */
+    constexpr int UN = MX ? 8 : ST;                /* stages per loop */
+    if constexpr (MX) copy_w(s0 / 4, std::integral_constant<int, 0>{});
     k3_tok_for<ST - 1>([&](auto sl) { copy(s0 + decltype(sl)::value, sl); });
-    for (int s = s0; s < s1; s += ST)              /* a stage past the share multiplies zeros */
-        k3_tok_for<ST>([&](auto sl) {
-            constexpr int S = decltype(sl)::value;
+    for (int s = s0; s < s1; s += UN)              /* a stage past the share multiplies zeros */
+        k3_tok_for<UN>([&](auto st) {
+            constexpr int S = decltype(st)::value;
             __builtin_amdgcn_s_waitcnt(WAIT_LDS);
             __builtin_amdgcn_sched_barrier(0);
+            if constexpr (MX && S % 4 == 0) copy_w((s + S) / 4 + 1, std::integral_constant<int, (S / 4 + 1) & 1>{});
             copy(s + S + ST - 1, std::integral_constant<int, (S + ST - 1) % ST>{});
             __builtin_amdgcn_s_waitcnt(WAIT_STAGE);
             __builtin_amdgcn_sched_barrier(0);
-            comp(sl);
+            comp(std::integral_constant<int, S % ST>{}, st);
         });
     /* the waves' sums, in wave order */
     __builtin_amdgcn_s_waitcnt(0);
@@ -267,63 +357,79 @@ __global__ __launch_bounds__(64 * KW) void tok_gemm_kernel(TokArgs a)
     if (wv > 0) return;
     const bool vec = ((a.ldy | a.out) & 3) == 0 && ((uintptr_t)a.y & 15) == 0;
 #pragma unroll
-    for (int m = 0; m < MT; m++)
+    for (int m = 0; m < (GLU ? 1 : MT); m++)
 #pragma unroll
         for (int b = 0; b < NB; b++) {
-            k3_f32x4 v = acc[m][b];
+            const int t = tok0 + 16 * b + r16, lr = 16 * m + 4 * g, r = row0 + lr;
+            k3_f32x4 v[GLU ? 2 : 1];
 #pragma unroll
-            for (int k = 0; k < KW - 1; k++) v += red[(k * MT * NB + m * NB + b) * 64 + lane];
-            const int t = tok0 + 16 * b + r16, r = row0 + 16 * m + 4 * g;
-            if (t >= a.ntok || 16 * b + r16 >= 8 * N8 || r >= a.out) continue;
+            for (int h = 0; h < (GLU ? 2 : 1); h++) {
+                v[h] = acc[m + h][b];
 #pragma unroll
-            for (int e = 0; e < 4; e++)
-                if (v[e] != v[e] && r + e < a.out)
-                    v[e] = tok_plain_dot<BF>(a.W, a.x + (size_t)t * a.in, (size_t)(r + e), a.in);
+                for (int k = 0; k < KW - 1; k++) v[h] += red[(k * MT * NB + (m + h) * NB + b) * 64 + lane];
+            }
+            if (t >= a.ntok || 16 * b + r16 >= 8 * N8 || lr >= nrow) continue;
+            if constexpr (!MX && !XT) {
+#pragma unroll
+                for (int h = 0; h < (GLU ? 2 : 1); h++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        if (v[h][e] != v[h][e] && lr + e < nrow)
+                            v[h][e] = tok_plain_dot<BF>(h ? a.W2 : a.W, a.x + (size_t)t * a.in, (size_t)(r + e), a.in);
+            }
+            if constexpr (GLU)
+#pragma unroll
+                for (int e = 0; e < 4; e++) v[0][e] = k3_act_pair(v[0][e], v[1][e], a.act, a.b1, a.b2);
             float *o = a.y + (size_t)t * a.ldy + r;
             if (vec) {
-                *reinterpret_cast<float4 *>(o) = make_float4(v[0], v[1], v[2], v[3]);
+                if (a.accumulate) v[0] = *reinterpret_cast<const k3_f32x4 *>(o) + v[0];
+                *reinterpret_cast<k3_f32x4 *>(o) = v[0];
             } else {
 #pragma unroll
                 for (int e = 0; e < 4; e++)
-                    if (r + e < a.out) o[e] = v[e];
+                    if (lr + e < nrow) o[e] = a.accumulate ? o[e] + v[0][e] : v[0][e];
             }
         }
 }
 
-template <int BF, int MT, int N8>
+template <int WT, int XT, int GLU, int MT, int N8>
 int launch_tok(TokArgs a, hipStream_t st)
 {
-    /* eight waves where two stages of theirs fit 160 KB of LDS, else four; up to four stages */
-    constexpr int SKB = MT * (BF ? 1 : 2) + N8, KW = SKB <= 10 ? 8 : 4;
-    constexpr int ST = 160 / (KW * SKB) > 4 ? 4 : 160 / (KW * SKB);
-    const int nrb = (a.out + 16 * MT - 1) / (16 * MT);
+    /* eight waves where two stages of theirs fit 160 KB of LDS, else four; up to four stages (MX: two
+     * or four, beside two chunks of codes) */
+    constexpr int MX = WT == TOK_MX;
+    constexpr int SKB = MX ? N8 : MT * (WT == TOK_F32 ? 2 : 1) + N8, CKB = MX ? 2 * MT : 0;
+    constexpr int KW = 8 * (2 * SKB + CKB) <= 160 ? 8 : 4;
+    constexpr int RKB = (KW - 1) * MT * ((N8 + 1) / 2) - KW * SKB;       /* the sums beyond buffer 0 */
+    constexpr int S4 = (160 - (RKB > 0 ? RKB : 0) - KW * CKB) / (KW * SKB), ST = S4 >= 4 ? 4 : MX ? 2 : S4;
+    const int rows = GLU ? a.rpt : 16 * MT;
     a.ntt = (a.ntok + 8 * N8 - 1) / (8 * N8);
-    a.items = nrb * a.ntt;
+    a.items = (a.out + rows - 1) / rows * a.ntt;
     a.per_xcd = (a.items + K3_NXCD - 1) / K3_NXCD;
-    hipLaunchKernelGGL((tok_gemm_kernel<BF, MT, N8, KW, ST>), dim3((unsigned)(a.per_xcd * K3_NXCD)), dim3(64 * KW), 0,
-                       st, a);
+    hipLaunchKernelGGL((tok_gemm_kernel<WT, XT, GLU, MT, N8, KW, ST>), dim3((unsigned)(a.per_xcd * K3_NXCD)), dim3(64 * KW),
+                       0, st, a);
     K3K_LAUNCH_CHECK("tok gemm launch");
     return 0;
 }
 
 /* Cycles for the workgroups that fall to the busiest CU: per workgroup, K columns of cutting x
- * (bf16), moving the operands (50 bytes per cycle) and multiplying, of which the largest counts
- * whole and the others by 0.4 (measured, how far they overlap), and about 4 us (9600 cycles) to
- * start, fill the stages and add up. */
-float tok_cost(int bf, int mt, int n8, int out, int ntok, int in, int cus)
+ * (fp32 activations against bf16 weights), moving the operands (50 bytes per cycle) and
+ * multiplying, of which the largest counts whole and the others by 0.4 (measured, how far they
+ * overlap), and about 4 us (9600 cycles) to start, fill the stages and add up. */
+float tok_cost(int wt, int xt, int mt, int n8, int out, int ntok, int in, int cus)
 {
     const long wgs = (long)((out + 16 * mt - 1) / (16 * mt)) * ((ntok + 8 * n8 - 1) / (8 * n8));
     const int nb = (n8 + 1) / 2;
-    const float cut = bf ? 16.f * nb * 5.5f / 64.f : 0.f;
-    const float bytes = (16.f * mt * (bf ? 2 : 4) + 8.f * n8 * 4) / 50.f;
-    const float mfma = mt * nb * 512.f * (bf ? 3.f / 4096.f : 1.f / 256.f);
+    const float cut = xt ? 0.f : wt == TOK_BF16 ? 16.f * nb * 5.5f / 64.f : 0.f;
+    const float bytes = (16.f * mt * (wt == TOK_F32 ? 4.f : wt == TOK_BF16 ? 2.f : 0.6f) + 8.f * n8 * 4) / 50.f;
+    const float mfma = mt * nb * 512.f * (wt == TOK_F32 ? 1.f / 256.f : (xt ? 2.f : 3.f) / 4096.f);
     float c = cut > bytes ? cut : bytes;
     if (mfma > c) c = mfma;
     c += 0.4f * (cut + bytes + mfma - c);
     return (c * in + 9600.f) * (float)((wgs + cus - 1) / cus);
 }
 
-template <int BF>
+template <int WT, int XT>
 int dispatch_tok(const TokArgs &a, hipStream_t st)
 {
     static const int shapes[][2] = {{1, 1}, {1, 2}, {1, 3}, {1, 4}, {1, 5}, {1, 6}, {1, 8},
@@ -332,31 +438,31 @@ int dispatch_tok(const TokArgs &a, hipStream_t st)
     int best = 0;
     float bc = 0;
     for (int i = 0; i < (int)(sizeof shapes / sizeof shapes[0]); i++) {
-        const float c = tok_cost(BF, shapes[i][0], shapes[i][1], a.out, a.ntok, a.in, k3k_cu_count());
+        const float c = tok_cost(WT, XT, shapes[i][0], shapes[i][1], a.out, a.ntok, a.in, k3k_cu_count());
         if (i == 0 || c < bc) {
             best = i;
             bc = c;
         }
     }
     switch (best) {
-    case 0: return launch_tok<BF, 1, 1>(a, st);
-    case 1: return launch_tok<BF, 1, 2>(a, st);
-    case 2: return launch_tok<BF, 1, 3>(a, st);
-    case 3: return launch_tok<BF, 1, 4>(a, st);
-    case 4: return launch_tok<BF, 1, 5>(a, st);
-    case 5: return launch_tok<BF, 1, 6>(a, st);
-    case 6: return launch_tok<BF, 1, 8>(a, st);
-    case 7: return launch_tok<BF, 2, 1>(a, st);
-    case 8: return launch_tok<BF, 2, 2>(a, st);
-    case 9: return launch_tok<BF, 2, 4>(a, st);
-    case 10: return launch_tok<BF, 2, 8>(a, st);
-    case 11: return launch_tok<BF, 3, 1>(a, st);
-    case 12: return launch_tok<BF, 3, 2>(a, st);
-    case 13: return launch_tok<BF, 3, 4>(a, st);
-    case 14: return launch_tok<BF, 4, 1>(a, st);
-    case 15: return launch_tok<BF, 4, 2>(a, st);
-    case 16: return launch_tok<BF, 4, 4>(a, st);
-    default: return launch_tok<BF, 4, 8>(a, st);
+    case 0: return launch_tok<WT, XT, 0, 1, 1>(a, st);
+    case 1: return launch_tok<WT, XT, 0, 1, 2>(a, st);
+    case 2: return launch_tok<WT, XT, 0, 1, 3>(a, st);
+    case 3: return launch_tok<WT, XT, 0, 1, 4>(a, st);
+    case 4: return launch_tok<WT, XT, 0, 1, 5>(a, st);
+    case 5: return launch_tok<WT, XT, 0, 1, 6>(a, st);
+    case 6: return launch_tok<WT, XT, 0, 1, 8>(a, st);
+    case 7: return launch_tok<WT, XT, 0, 2, 1>(a, st);
+    case 8: return launch_tok<WT, XT, 0, 2, 2>(a, st);
+    case 9: return launch_tok<WT, XT, 0, 2, 4>(a, st);
+    case 10: return launch_tok<WT, XT, 0, 2, 8>(a, st);
+    case 11: return launch_tok<WT, XT, 0, 3, 1>(a, st);
+    case 12: return launch_tok<WT, XT, 0, 3, 2>(a, st);
+    case 13: return launch_tok<WT, XT, 0, 3, 4>(a, st);
+    case 14: return launch_tok<WT, XT, 0, 4, 1>(a, st);
+    case 15: return launch_tok<WT, XT, 0, 4, 2>(a, st);
+    case 16: return launch_tok<WT, XT, 0, 4, 4>(a, st);
+    default: return launch_tok<WT, XT, 0, 4, 8>(a, st);
     }
 }
 
@@ -383,5 +489,39 @@ extern "C" int k3k_tok_gemm(float *y, const float *x, const void *W, int bf16, i
     a.out = out;
     a.ntok = ntok;
     a.ldy = ldy;
-    return bf16 ? dispatch_tok<1>(a, (hipStream_t)stream) : dispatch_tok<0>(a, (hipStream_t)stream);
+    return bf16 ? dispatch_tok<TOK_BF16, 0>(a, (hipStream_t)stream) : dispatch_tok<TOK_F32, 0>(a, (hipStream_t)stream);
+}
+
+/* both terms reachable from xhi with 32-bit offsets */
+static int terms_ok(const uint16_t *xhi, const uint16_t *xlo, int in, int ntok, uint32_t *lo_off)
+{
+    const uint64_t d = (uint64_t)((const char *)xlo - (const char *)xhi);
+    if (xlo < xhi || d + (uint64_t)ntok * in * 2 >= 0x80000000u || (((uintptr_t)xhi | (uintptr_t)xlo) & 15)) return 0;
+    *lo_off = (uint32_t)d;
+    return 1;
+}
+
+extern "C" int k3k_tok_mx_ok(const uint16_t *xhi, const uint16_t *xlo, const void *packed, int in, int ntok)
+{
+    uint32_t lo;
+    return ntok > 2 && in % 32 == 0 && in < (1 << 22) && ((uintptr_t)packed & 15) == 0 &&
+           terms_ok(xhi, xlo, in, ntok, &lo);
+}
+
+extern "C" int k3k_tok_mx(float *y, const uint16_t *xhi, const uint16_t *xlo, const void *packed, const uint8_t *scales,
+                          int in, int out, int ntok, int ldy, void *stream)
+{
+    if (!k3k_tok_mx_ok(xhi, xlo, packed, in, ntok)) return k3k_fail("tok mx shape", hipErrorInvalidValue);
+    if (out <= 0) return 0;
+    TokArgs a = {};
+    a.y = y;
+    a.xhi = xhi;
+    (void)terms_ok(xhi, xlo, in, ntok, &a.lo_off);
+    a.W = packed;
+    a.scales = scales;
+    a.in = in;
+    a.out = out;
+    a.ntok = ntok;
+    a.ldy = ldy;
+    return dispatch_tok<TOK_MX, 1>(a, (hipStream_t)stream);
 }

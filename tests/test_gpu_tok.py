@@ -60,3 +60,33 @@ def test_tok_matmul_nonfinite(gpu, k3, bf16):
     # the cut's last term ends at 2^-133; fp32 products of subnormals at 2^-149
     tiny = 2.0**-133 * np.abs(np.nan_to_num(W, posinf=0, neginf=0)).astype(np.float64).sum(1)[None, :] + inn * 2.0**-149
     assert (np.abs(Y - want)[fin] <= (1e-6 * bound + tiny)[fin]).all()
+
+
+@pytest.mark.parametrize("T,inn,rows", [(3, 128, 1), (3, 7168, 2048), (8, 256, 17), (9, 384, 48), (17, 1152, 130), (33, 3584, 4097),
+                                        (64, 896, 300), (65, 512, 4100), (130, 2176, 71), (257, 128, 1031),
+                                        (3, 32, 5), (19, 224, 100), (40, 1504, 515), (100, 4128, 70)])
+def test_tok_mxfp4_edges(gpu, k3, T, inn, rows):
+    """k3d_matmul_mxfp4 from three tokens: the activations are two bf16 terms, off by at most
+    2^-17 of each (8 bits a term, rounded, and a sign), and a block whose scale is NaN is 0."""
+    say(f"case: mxfp4 {T} tokens {inn} -> {rows}")
+    rng = np.random.default_rng(T)
+    codes = rng.integers(0, 256, (rows, inn // 2), dtype=np.uint8)
+    scales = rng.integers(118, 127, (rows, inn // 32), dtype=np.uint8)
+    scales[rows // 2, inn // 64] = 255
+    X = k3.gen_normal(T * inn, 7 + T).reshape(T, inn) * (np.float32(10.0) ** (np.arange(T) % 7 - 3))[:, None].astype(np.float32)
+    val = np.array([0, .5, 1, 1.5, 2, 3, 4, 6, -0., -.5, -1, -1.5, -2, -3, -4, -6])
+    W = np.stack([val[codes & 15], val[codes >> 4]], axis=2).reshape(rows, inn)
+    W *= np.repeat(np.where(scales == 255, 0.0, 2.0 ** (scales.astype(np.float64) - 127)), 32, axis=1)
+    want, bound = X.astype(np.float64) @ W.T, np.abs(X.astype(np.float64)) @ np.abs(W.T)
+    L = gpu.lib()
+    bufs = [gpu.DevBuf(a.nbytes).upload(np.ascontiguousarray(a)) for a in (X, codes, scales)]
+    bufs += [gpu.DevBuf(max(L.k3d_matmul_mxfp4_ws(T, inn), 16)), gpu.DevBuf(T * rows * 4)]
+    dx, dp, ds, ws, dy = bufs
+    try:
+        for prec in (0, 1):
+            gpu.check(L.k3d_matmul_mxfp4(dy.ptr, dx.ptr, T, dp.ptr, ds.ptr, inn, rows, prec, ws.ptr, ws.nbytes, None), "mxfp4")
+            Y = dy.download(np.empty((T, rows), np.float32))
+            assert (np.abs(Y - want) <= (2.0**-17 + 1e-6) * bound).all(), prec
+    finally:
+        for b in bufs:
+            b.free()
