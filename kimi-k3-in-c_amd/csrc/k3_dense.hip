@@ -268,7 +268,7 @@ extern "C" int k3k_gemv_f32(float *y, const float *x, const float *W, int in, in
                             int ldy, void *stream)
 {
     if (out <= 0 || ntok <= 0) return 0;
-    if (k3k_tok_ok(x, W, in, ntok)) return k3k_tok_gemm(y, x, W, 0, in, out, ntok, ldy, stream);
+    if (k3k_tok_ok(x, W, in, ntok)) return k3k_tok_gemm(y, x, W, 0, in, out, ntok, ldy, 0, stream);
     const int vec = (in % 8 == 0) && aligned16(x) && aligned16(W);
     if (vec && in > 0 && ntok == 1) launch_gemv<float>(y, x, W, in, out, (hipStream_t)stream);
     else hipLaunchKernelGGL(gemv_kernel<float>, dim3((out + 3) / 4, ntok), dim3(256), 0,
@@ -281,7 +281,7 @@ extern "C" int k3k_gemv_bf16(float *y, const float *x, const uint16_t *W, int in
                              int ntok, int ldy, void *stream)
 {
     if (out <= 0 || ntok <= 0) return 0;
-    if (k3k_tok_ok(x, W, in, ntok)) return k3k_tok_gemm(y, x, W, 1, in, out, ntok, ldy, stream);
+    if (k3k_tok_ok(x, W, in, ntok)) return k3k_tok_gemm(y, x, W, 1, in, out, ntok, ldy, 0, stream);
     const int vec = (in % 8 == 0) && aligned16(x) && aligned16(W);
     if (vec && in > 0 && ntok == 1) launch_gemv<uint16_t>(y, x, W, in, out, (hipStream_t)stream);
     else hipLaunchKernelGGL(gemv_kernel<uint16_t>, dim3((out + 3) / 4, ntok), dim3(256), 0,

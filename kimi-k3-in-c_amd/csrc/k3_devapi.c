@@ -762,8 +762,8 @@ int k3d_mxfp4_tile(uint8_t *tpacked, uint8_t *tscales, const uint8_t *packed,
 }
 
 /* ---- dense (bf16) shared expert ------------------------------------------------------------
- * Two launches of the dense GEMM kernel (k3_gemm.hip) after the activation split: gate and up
- * in one pass over x with the activation and its bf16 split in the epilogue, then down,
+ * Two launches of the dense GEMM kernel (k3_gemm.hip) after the activation split (few tokens: of
+ * the several-token kernel, k3_tok.hip, without it): gate and up in one pass over x with the activation and its bf16 split in the epilogue, then down,
  * written or added onto y (one fp32 add of the finished sum, the reference's
  * `ot[i] += sdn[i]`, k3_ops.c:654). */
 typedef struct {
@@ -803,13 +803,34 @@ int k3d_shared_expert(float *y, int accumulate, const float *x, int T, const uin
     Carve c = {(char *)ws, 0};
     ShWs w;
     shared_layout(&c, &w, T, hidden, inter, prec);
+    /* Few tokens: gate, up and the activation in one launch of the several-token kernel and down
+     * in another, on fp32 activations (act takes the terms' place in the workspace), instead of a
+     * split, two GEMMs and two slice sums. Better while the gate and up rows make one round of
+     * workgroups and x, padded to the kernel's blocks of 8, 16 and 32 tokens, is short against
+     * them: of 7168 columns 8 / 16 / 32 tokens of 2048 rows 30.2 -> 21.3 / 31.2 -> 23.4 / 34.0 ->
+     * 33.5 us; of 4096 rows 47.2 -> 42.9 / 48.6 -> 48.2 / 52.9 -> 61.8; two rounds (6144 rows) 68
+     * -> 71 / 70 -> 80; of 4096 columns 32 tokens of 1024 rows 23.7 -> 20.0. */
+    const int Tp = T <= 8 ? 8 : T <= 16 ? 16 : 32;
+    if (T <= 32 && (long)Tp * hidden <= 131072 && inter <= 16 * k3k_cu_count() && ws_bytes >= (size_t)T * inter * 4 &&
+        k3k_tok_glu_ok(x, w1, w3, hidden) && k3k_tok_glu_ok(ws, w2, w2, inter)) {
+        float *a32 = (float *)ws;
+        if (k3k_tok_glu(a32, x, w1, w3, hidden, inter, T, act, b1, b2, stream)) return fail("shared gate/up");
+        if (k3k_tok_gemm(y, a32, w2, 1, inter, hidden, T, hidden, accumulate, stream)) return fail("shared down");
+        k3k_prof_mark(stream, K3D_STAGE_SHARED);
+        return 0;
+    }
     if (k3k_split_bf16(w.xhi, w.xlo, x, (size_t)T * hidden, stream)) return fail("split");
     if (k3k_dense_gateup(w.ahi, w.alo, w1, w3, w.xhi, w.xlo, inter, T, hidden, act, b1, b2, w.part,
                          w.part_bytes, stream))
         return fail("shared gate/up");
-    if (k3k_dense_gemm(y, hidden, accumulate, w2, w.ahi, w.alo, hidden, T, inter, w.part, w.part_bytes,
-                       stream))
+    /* a short K leaves the GEMM little to slice: the several-token kernel, while its tokens' terms
+     * are short too (7168 rows, 64 tokens: of 1024 / 2048 / 3072 columns the whole call 31.7 -> 28.1 /
+     * 39.3 -> 36.0 / 52.0 -> 52.1 us; 128 tokens of 2048 47.3 -> 47.1, 200 66 -> 76) */
+    if (prec == 0 && inter <= 2048 && (long)T * inter <= 131072 && k3k_tok_terms_ok(w.ahi, w.alo, w2, inter, T)) {
+        if (k3k_tok_terms(y, hidden, accumulate, w2, w.ahi, w.alo, inter, hidden, T, stream)) return fail("shared down");
+    } else if (k3k_dense_gemm(y, hidden, accumulate, w2, w.ahi, w.alo, hidden, T, inter, w.part, w.part_bytes, stream)) {
         return fail("shared down");
+    }
     k3k_prof_mark(stream, K3D_STAGE_SHARED);
     return 0;
 }

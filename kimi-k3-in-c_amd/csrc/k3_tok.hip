@@ -471,15 +471,20 @@ int dispatch_tok(const TokArgs &a, hipStream_t st)
 /* in % 8 == 0, x and W 16-byte aligned, and a row block's operand under 2 GiB. Up to four tokens
  * of fewer than 512 columns stay with the vector units: their waves would have one stage each
  * at most, and there is no weight stream to share (2 tokens of 256 -> 1024: 6.8 us either way). */
+static int shape_ok(const void *x, const void *W, int in)
+{
+    return in >= 8 && in % 8 == 0 && in < (1 << 22) && (((uintptr_t)x | (uintptr_t)W) & 15) == 0;
+}
+
 extern "C" int k3k_tok_ok(const float *x, const void *W, int in, int ntok)
 {
-    return ntok > 1 && (ntok > 4 || in >= 512) && in >= 8 && in % 8 == 0 && in < (1 << 22) && (((uintptr_t)x | (uintptr_t)W) & 15) == 0;
+    return ntok > 1 && (ntok > 4 || in >= 512) && shape_ok(x, W, in);
 }
 
 extern "C" int k3k_tok_gemm(float *y, const float *x, const void *W, int bf16, int in, int out, int ntok, int ldy,
-                            void *stream)
+                            int accumulate, void *stream)
 {
-    if (!k3k_tok_ok(x, W, in, ntok)) return k3k_fail("tok gemm shape", hipErrorInvalidValue);
+    if (!shape_ok(x, W, in)) return k3k_fail("tok gemm shape", hipErrorInvalidValue);
     if (out <= 0) return 0;
     TokArgs a = {};
     a.y = y;
@@ -489,7 +494,38 @@ extern "C" int k3k_tok_gemm(float *y, const float *x, const void *W, int bf16, i
     a.out = out;
     a.ntok = ntok;
     a.ldy = ldy;
+    a.accumulate = accumulate;
     return bf16 ? dispatch_tok<TOK_BF16, 0>(a, (hipStream_t)stream) : dispatch_tok<TOK_F32, 0>(a, (hipStream_t)stream);
+}
+
+extern "C" int k3k_tok_glu_ok(const void *x, const void *Wg, const void *Wu, int in)
+{
+    return shape_ok(x, Wg, in) && shape_ok(x, Wu, in);
+}
+
+extern "C" int k3k_tok_glu(float *y, const float *x, const uint16_t *Wg, const uint16_t *Wu, int in, int out, int ntok,
+                           int act, float b1, float b2, void *stream)
+{
+    if (!k3k_tok_glu_ok(x, Wg, Wu, in)) return k3k_fail("tok glu shape", hipErrorInvalidValue);
+    if (out <= 0) return 0;
+    TokArgs a = {};
+    a.y = y;
+    a.x = x;
+    a.W = Wg;
+    a.W2 = Wu;
+    a.in = in;
+    a.out = a.ldy = out;
+    a.ntok = ntok;
+    a.act = act;
+    a.b1 = b1;
+    a.b2 = b2;
+    /* half-filled tiles where those are still one round of workgroups (8 tokens of 7168 -> 3072, two
+     * rounds of them: 37.6 us with the down product, 38.7 on the GEMMs): the weight stream, not the
+     * products, is what takes the time */
+    a.rpt = (out + 7) / 8 <= k3k_cu_count() ? 8 : 16;
+    return ntok <= 8    ? launch_tok<TOK_BF16, 0, 1, 2, 1>(a, (hipStream_t)stream)
+           : ntok <= 16 ? launch_tok<TOK_BF16, 0, 1, 2, 2>(a, (hipStream_t)stream)
+                        : launch_tok<TOK_BF16, 0, 1, 2, 4>(a, (hipStream_t)stream);
 }
 
 /* both terms reachable from xhi with 32-bit offsets */
@@ -524,4 +560,28 @@ extern "C" int k3k_tok_mx(float *y, const uint16_t *xhi, const uint16_t *xlo, co
     a.ntok = ntok;
     a.ldy = ldy;
     return dispatch_tok<TOK_MX, 1>(a, (hipStream_t)stream);
+}
+
+extern "C" int k3k_tok_terms_ok(const uint16_t *xhi, const uint16_t *xlo, const uint16_t *W, int in, int ntok)
+{
+    uint32_t lo;
+    return shape_ok(W, W, in) && terms_ok(xhi, xlo, in, ntok, &lo);
+}
+
+extern "C" int k3k_tok_terms(float *y, int ldy, int accumulate, const uint16_t *W, const uint16_t *xhi, const uint16_t *xlo,
+                             int in, int out, int ntok, void *stream)
+{
+    if (!k3k_tok_terms_ok(xhi, xlo, W, in, ntok)) return k3k_fail("tok terms shape", hipErrorInvalidValue);
+    if (out <= 0) return 0;
+    TokArgs a = {};
+    a.y = y;
+    a.xhi = xhi;
+    (void)terms_ok(xhi, xlo, in, ntok, &a.lo_off);
+    a.W = W;
+    a.in = in;
+    a.out = out;
+    a.ntok = ntok;
+    a.ldy = ldy;
+    a.accumulate = accumulate;
+    return dispatch_tok<TOK_BF16, 1>(a, (hipStream_t)stream);
 }

@@ -203,8 +203,17 @@ int k3k_gemv_glu(float *y, const float *x, const void *Wg, const void *Wu, int b
  * where k3k_tok_ok holds (in % 8 == 0, x and W 16-byte aligned). k3k_gemv_* send their calls
  * there. */
 int k3k_tok_ok(const float *x, const void *W, int in, int ntok);
-int k3k_tok_gemm(float *y, const float *x, const void *W, int bf16, int in, int out, int ntok, int ldy,
+int k3k_tok_gemm(float *y, const float *x, const void *W, int bf16, int in, int out, int ntok, int ldy, int accumulate,
                  void *stream);
+/* y[t][r] = act(gate, up) of bf16 weights, fp32 x, where k3k_tok_glu_ok holds (as k3k_tok_gemm:
+ * in % 8 == 0, 16-byte aligned); k3k_tok_terms: y[t][r] (=, or +=) the products with x as two bf16 terms,
+ * where k3k_tok_terms_ok holds (in % 8 == 0, 16-byte aligned). */
+int k3k_tok_glu_ok(const void *x, const void *Wg, const void *Wu, int in);
+int k3k_tok_glu(float *y, const float *x, const uint16_t *Wg, const uint16_t *Wu, int in, int out, int ntok, int act,
+                float b1, float b2, void *stream);
+int k3k_tok_terms_ok(const uint16_t *xhi, const uint16_t *xlo, const uint16_t *W, int in, int ntok);
+int k3k_tok_terms(float *y, int ldy, int accumulate, const uint16_t *W, const uint16_t *xhi, const uint16_t *xlo, int in,
+                  int out, int ntok, void *stream);
 /* MXFP4 weights (row-major, group 32) times three tokens and more given as two bf16 terms, where
  * k3k_tok_mx_ok holds (in % 32 == 0, packed 16-byte aligned, the terms within 2 GiB of each other). */
 int k3k_tok_mx_ok(const uint16_t *xhi, const uint16_t *xlo, const void *packed, int in, int ntok);

@@ -90,3 +90,30 @@ def test_tok_mxfp4_edges(gpu, k3, T, inn, rows):
     finally:
         for b in bufs:
             b.free()
+
+
+@pytest.mark.parametrize("act", [0, 1])
+@pytest.mark.parametrize("T,hidden,inter", [(1, 64, 64), (2, 7168, 192), (8, 128, 4096), (9, 448, 4160), (16, 7168, 2048), (17, 7168, 64),
+                                            (32, 4096, 128), (33, 64, 2048), (64, 192, 2048), (65, 320, 1984), (128, 64, 1024)])
+def test_shared_expert_few_tokens(gpu, k3, act, T, hidden, inter):
+    """The shared expert where it takes this kernel (up to 32 tokens whole, its down product
+    up to 128), next to those bounds, written and added: 1e-4 of the largest result with fp32
+    or two-term activations, 2e-2 of the norm with one."""
+    say(f"case: shared expert {T} tokens {hidden} -> {inter} act={act}")
+    W = [k3.gen_bf16_normal(hidden * inter, 31 + i + T, 0.0, 0.03) for i in range(3)]
+    F = [(w.astype(np.uint32) << 16).view(np.float32).astype(np.float64) for w in W]
+    X = k3.gen_normal(T * hidden, 40 + T).reshape(T, hidden)
+    g, u = X.astype(np.float64) @ F[0].reshape(inter, hidden).T, X.astype(np.float64) @ F[1].reshape(inter, hidden).T
+    sg = g / (1.0 + np.exp(-g))
+    a = sg * u if act == 1 else 4.0 * np.tanh(g / 4.0) / (1.0 + np.exp(-g)) * 25.0 * np.tanh(u / 25.0)
+    want = a @ F[2].reshape(hidden, inter).T
+    y0 = k3.gen_normal(T * hidden, 41 + T).reshape(T, hidden)
+    for prec in (0, 1):
+        for add in (None, y0):
+            got = gpu.shared_expert_device(X, *[w.reshape(s) for w, s in zip(W, ((inter, hidden), (inter, hidden), (hidden, inter)))],
+                                           hidden, inter, act=act, prec=prec, y0=add)
+            ref = want if add is None else want + add
+            if prec == 0:
+                assert np.abs(got - ref).max() <= 1e-4 * np.abs(ref).max()
+            else:
+                assert np.linalg.norm(got - ref) <= 2e-2 * np.linalg.norm(ref)
