@@ -106,21 +106,25 @@ static int exc_table(const K3kExc **out)
                 if (m > mmax) mmax = m;
             }
             const uint32_t mwords = ((mmax - mmin) >> 5) + 1;
-            uint32_t *bits = (uint32_t *)calloc((size_t)2 * mwords, 4);
+            /* after it one bit per word: whether the word has any */
+            const size_t nw = (size_t)2 * mwords, ncw = (nw + 31) / 32;
+            uint32_t *bits = (uint32_t *)calloc(nw + ncw, 4);
             if (!bits) {
                 free(index);
                 return bad("router exception bitmap: out of host memory");
             }
             for (int j = 0; j < n; j++) {
                 const uint32_t key = k3_expf_exc[2 * j], bi = (key & 0x7fffffffu) - mmin;
-                bits[(size_t)(key >> 31) * mwords + (bi >> 5)] |= 1u << (bi & 31);
+                const size_t w = (size_t)(key >> 31) * mwords + (bi >> 5);
+                bits[w] |= 1u << (bi & 31);
+                bits[nw + (w >> 5)] |= 1u << (w & 31);
             }
             uint32_t *dp = (uint32_t *)k3k_malloc((size_t)2 * n * 4);
             uint32_t *di = (uint32_t *)k3k_malloc((size_t)(nb + 1) * 4);
-            uint32_t *db = (uint32_t *)k3k_malloc((size_t)2 * mwords * 4);
+            uint32_t *db = (uint32_t *)k3k_malloc((nw + ncw) * 4);
             int rc = !dp || !di || !db || k3k_h2d(dp, k3_expf_exc, (size_t)2 * n * 4, NULL) ||
                      k3k_h2d(di, index, (size_t)(nb + 1) * 4, NULL) ||
-                     k3k_h2d(db, bits, (size_t)2 * mwords * 4, NULL) || k3k_sync(NULL);
+                     k3k_h2d(db, bits, (nw + ncw) * 4, NULL) || k3k_sync(NULL);
             free(index);
             free(bits);
             if (rc) return fail("router exception table upload");
@@ -244,7 +248,7 @@ typedef struct {
 static size_t router_layout(Carve *c, RtWs *w, int T, int hidden, int n_experts)
 {
     const int c8 = k3k_router_i8_chunk(T, hidden, n_experts);
-    w->chunk = c8 ? c8 : k3k_router_chunk(T, hidden, n_experts);
+    w->chunk = c8 ? c8 : k3k_router_chunk(T, hidden, n_experts, NULL);
     const size_t ks = (size_t)((hidden + w->chunk - 1) / w->chunk);
     /* chunk partials, or (a few tokens) one 16-byte scored record per logit */
     w->part = (double *)take(c, (ks < 2 ? 2 : ks) * T * n_experts * 8);
@@ -255,11 +259,30 @@ static size_t router_layout(Carve *c, RtWs *w, int T, int hidden, int n_experts)
     return c->off;
 }
 
+/* What router_layout takes for any batch of up to T tokens: scratch sized for T tokens serves
+ * fewer, which may take the other partials, or more chunks. (The fp64 kernel's chunks: at most 12
+ * workgroups of 2048 logits per CU, and 28 of 256 columns of 7168; what it takes past that it takes
+ * for T tokens too.) The calls themselves ask for what they take. */
+static size_t router_size(Carve *c, int T, int hidden, int n_experts)
+{
+    const size_t start = c->off;
+    RtWs w;
+    router_layout(c, &w, T, hidden, n_experts);
+    if (T >= 128) {
+        const size_t tn = (size_t)T * n_experts, f64 = (size_t)12 * 2048 * (k3k_cu_count() > 0 ? k3k_cu_count() : 1);
+        const size_t all = (size_t)((hidden + 255) / 256) * tn, i8 = k3k_router_i8_ws(T, hidden, n_experts);
+        size_t any = (all < f64 ? all : f64) * 12;
+        if (any < i8) any = i8;
+        any += (size_t)T * 4 + 5 * 256;        /* nrecomp, ctr, the parts' rounding */
+        if (c->off - start < any) c->off = start + any;
+    }
+    return c->off;
+}
+
 size_t k3d_router_ws(int T, int hidden, int n_experts)
 {
     Carve c = {NULL, 0};
-    RtWs w;
-    return router_layout(&c, &w, T, hidden, n_experts);
+    return router_size(&c, T, hidden, n_experts);
 }
 
 /* gather (may be NULL): the router's final kernel also runs the expert-major gather */
@@ -326,10 +349,9 @@ int k3d_router(int *idx, float *wt, const float *x, int T, const float *W, const
     if (T <= 0) return 0;
     if (topk < 1 || topk > K3_MAX_TOPK) return bad("k3d_router: topk outside 1..64");
     if (n_experts < 1 || n_experts > 2048) return bad("k3d_router: n_experts outside 1..2048");
-    if (ws_bytes < k3d_router_ws(T, hidden, n_experts)) return bad("k3d_router: workspace too small");
     Carve c = {(char *)ws, 0};
     RtWs w;
-    router_layout(&c, &w, T, hidden, n_experts);
+    if (ws_bytes < router_layout(&c, &w, T, hidden, n_experts)) return bad("k3d_router: workspace too small");
     return router_run(idx, wt, x, T, W, bias, hidden, n_experts, topk, renorm, routed_scale, &w, NULL,
                       stream);
 }
@@ -450,10 +472,8 @@ size_t k3d_moe_ws(int T, int hidden, int inter, int n_experts, int topk, int pre
 {
     Carve c = {NULL, 0};
     MoeWs w;
-    RtWs r;
     moe_layout(&c, &w, T, hidden, inter, n_experts, topk, prec);
-    router_layout(&c, &r, T, hidden, n_experts);
-    return c.off;
+    return router_size(&c, T, hidden, n_experts);
 }
 
 static int moe_check(const char *fn, int hidden, int inter, int n_experts, int topk, int layout)
@@ -658,11 +678,11 @@ int k3d_moe_experts(float *out, const int *idx, const float *wt, const float *x,
     if (T <= 0) return 0;
     int rc = moe_check("k3d_moe_experts", hidden, inter, n_experts, topk, layout);
     if (rc) return rc;
-    if (ws_bytes < k3d_moe_ws(T, hidden, inter, n_experts, topk, prec))
-        return bad("k3d_moe_experts: workspace too small");
     Carve c = {(char *)ws, 0};
     MoeWs w;
+    RtWs r;
     moe_layout(&c, &w, T, hidden, inter, n_experts, topk, prec);
+    if (ws_bytes < router_layout(&c, &r, T, hidden, n_experts)) return bad("k3d_moe_experts: workspace too small");
     k3k_prof_mark(stream, K3D_STAGE_BEGIN);
     return moe_experts_ws(out, idx, wt, x, T, bank, layout, hidden, inter, n_experts, topk, act,
                           b1, b2, prec, &w, perm_out, offsets_out, drops_out, NULL, 0, 0, stream);
@@ -677,13 +697,11 @@ int k3d_moe_routed(float *out, int *idx, float *wt, const float *x, int T, const
     if (T <= 0) return 0;
     int rc = moe_check("k3d_moe_routed", hidden, inter, n_experts, topk, layout);
     if (rc) return rc;
-    if (ws_bytes < k3d_moe_ws(T, hidden, inter, n_experts, topk, prec))
-        return bad("k3d_moe_routed: workspace too small");
     Carve c = {(char *)ws, 0};
     MoeWs w;
     RtWs r;
     moe_layout(&c, &w, T, hidden, inter, n_experts, topk, prec);
-    router_layout(&c, &r, T, hidden, n_experts);
+    if (ws_bytes < router_layout(&c, &r, T, hidden, n_experts)) return bad("k3d_moe_routed: workspace too small");
     k3k_prof_mark(stream, K3D_STAGE_BEGIN);
     if (moe_decode_ok(T, hidden, inter, topk, x) && k3k_router_small(T, hidden) && n_experts <= 512 &&
         !perm_out && !offsets_out) {

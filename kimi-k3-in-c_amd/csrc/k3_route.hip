@@ -496,6 +496,11 @@ __device__ __forceinline__ void round_interval(float f, double &lo, double &hi)
  * choice, score + bias, is then certain too); otherwise scmax is the score of the largest
  * float the logit can be. Non-finite sums come from inf/NaN inputs and propagate alike in
  * any order (ok). fword = exc_word((float)Q, exc), loaded by the caller. */
+__device__ __forceinline__ double certify_bound(double Q, double bs)
+{
+    return 1.01 * 0x1p-53 * bs + 4.0 * 0x1p-53 * fabs(Q) + 0x1p-1060;
+}
+
 struct Certified {
     float sc, scmax;
     bool ok;
@@ -510,7 +515,7 @@ __device__ __forceinline__ Certified certify_score(double Q, double bs, const Ex
     r.scmax = r.sc;
     r.ok = true;
     if (fabs(Q) <= 0x1.fffffffffffffp+1023) {
-        const double B = 1.01 * 0x1p-53 * bs + 4.0 * 0x1p-53 * fabs(Q) + 0x1p-1060;
+        const double B = certify_bound(Q, bs);
         double mlo, mhi;
         round_interval(f, mlo, mhi);
         if (!((Q - B > mlo) && (Q + B < mhi))) {
@@ -785,7 +790,9 @@ __global__ __launch_bounds__(KB > 32 ? 512 : 1024) void router_final_kernel(int 
                     }
                 }
             }
-            const Certified cs = certify_score(Q, bs, exc, exc_word((float)Q, exc));
+            /* (few logits: one load after the other costs more than misses in the L2s do) */
+            const Certified cs = certify_score(Q, bs, exc, (long)T * n_experts < 131072 ? exc_word((float)Q, exc)
+                                                                                        : exc_word_many((float)Q, exc));
             select_put_record(sm, e, make_float4(cs.sc, cs.scmax, cs.ok ? 0.0f : 1.0f, 0.0f),
                               bias ? bias[e] : 0.0f);
         }
@@ -829,6 +836,265 @@ __global__ __launch_bounds__(KB > 32 ? 512 : 1024) void router_final_kernel(int 
             if (tid == 0) __hip_atomic_store(g.ctr, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
+}
+
+/* The reference's chain of one logit by one wave (chain_block for a wave): the lanes write blocks of
+ * exact products into the wave's ring, two by turns, the next block's operands on their way; every
+ * lane then runs the chain over them, sixteen products read ahead of the sixteen being added (one
+ * dependent fp64 add per column is what it takes). */
+__device__ double chain_wave(double (*ring)[RF_BLK], const float *w, const float *x, int hidden)
+{
+    constexpr int NP = RF_BLK / 64;
+    const int lane = threadIdx.x & 63, nb = (hidden + RF_BLK - 1) / RF_BLK;
+    float wq[NP], xq[NP];
+    auto load = [&](int b) {
+#pragma unroll
+        for (int q = 0; q < NP; q++) {
+            const int k = b * RF_BLK + lane + 64 * q;
+            wq[q] = k < hidden ? w[k] : 0.0f;
+            xq[q] = k < hidden ? x[k] : 0.0f;
+        }
+    };
+    double acc = 0.0;
+    load(0);
+    for (int b = 0; b < nb; b++) {
+        double *r = ring[b & 1];
+#pragma unroll
+        for (int q = 0; q < NP; q++) r[lane + 64 * q] = (double)wq[q] * (double)xq[q];
+        if (b + 1 < nb) load(b + 1);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        const int n = min(RF_BLK, hidden - b * RF_BLK);
+        const double2 *p2 = reinterpret_cast<const double2 *>(r);
+        int i = 0;
+        double2 c[8], d[8];
+#pragma unroll
+        for (int q = 0; q < 8; q++) c[q] = p2[q];
+        for (; i + 16 <= n; i += 16) {
+            const int nx = min(i + 16, RF_BLK - 16) / 2;
+#pragma unroll
+            for (int q = 0; q < 8; q++) d[q] = p2[nx + q];
+#pragma unroll
+            for (int q = 0; q < 8; q++) {
+                acc += c[q].x;
+                acc += c[q].y;
+            }
+#pragma unroll
+            for (int q = 0; q < 8; q++) c[q] = d[q];
+        }
+        for (; i < n; i++) acc += r[i];
+    }
+    return acc;
+}
+
+/* router_final_kernel for many tokens of up to 1024 experts: a wave per token, lane l holding experts
+ * l + 64 i (SL of them) in registers, so that no barrier joins waves and no wave waits while
+ * another selects (a workgroup per token kept 6 to 14 waves for the work of one). Scores, keys and
+ * certification as there; the selection is the threshold one of select_rounds with the lanes'
+ * largest choices for its row maxima and, past 64 candidates, topk wave maxima. 4096 tokens: 384
+ * experts, top 8, 24 us and, where a logit has to be recomputed, some 25 more for its chain of adds
+ * (a workgroup per token 60), whole routers 393 -> 352 and, 896 experts, top 16, 785 -> 686 us;
+ * 1000 tokens of 384 25 -> 12 us. Fewer than three tokens per CU stay on workgroups (300 tokens of
+ * 896: 23.6 us here, 19.6 there). What bounds it: the partials (12 bytes per chunk and logit) for
+ * many tokens, the chain of loads, certification and selection of one wave for few. */
+template <int SL>
+__global__ __launch_bounds__(256) void router_final_wave_kernel(int *idx, float *wt, int *nrecomp, const double *part,
+                                                                const float *rbound, int ksplit, int chunk,
+                                                                const float *x, const float *W, const float *bias, int T,
+                                                                int hidden, int n_experts, int topk, int renorm,
+                                                                float routed_scale, ExcTable exc)
+{
+    __shared__ __attribute__((aligned(16))) double ring[4][2][RF_BLK];
+    __shared__ uint64_t cand[4][64];
+    __shared__ float csc[4][64];
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int t = (int)blockIdx.x * 4 + wv;
+    if (t >= T) return;
+    int en[SL];                                        /* the lane's experts, the last one past the end */
+    double Q[SL], bs[SL];
+#pragma unroll
+    for (int i = 0; i < SL; i++) {
+        en[i] = min(lane + 64 * i, n_experts - 1);
+        Q[i] = bs[i] = 0.0;
+    }
+    for (int k = 0; k < ksplit; k++) {
+        const size_t o = ((size_t)k * T + t) * n_experts;
+        double pv[SL];
+        float rv[SL];
+#pragma unroll
+        for (int i = 0; i < SL; i++) {
+            pv[i] = part[o + en[i]];
+            rv[i] = rbound[o + en[i]];
+        }
+        const double ck = (double)min(chunk, hidden - k * chunk);
+#pragma unroll
+        for (int i = 0; i < SL; i++) {
+            bs[i] += ck * fabs(Q[i]) + 2.0 * (double)rv[i];
+            Q[i] += pv[i];
+            bs[i] += fabs(Q[i]);
+        }
+    }
+    /* scores; the exception words first (most of them known to be 0 from the small map) */
+    uint32_t word[SL];
+    {
+        uint32_t j[SL];
+#pragma unroll
+        for (int i = 0; i < SL; i++) j[i] = exc_slot((float)Q[i], exc);
+#pragma unroll
+        for (int i = 0; i < SL; i++) word[i] = exc_any(j[i], exc);
+#pragma unroll
+        for (int i = 0; i < SL; i++) word[i] = word[i] ? exc.bits[j[i]] : 0u;
+    }
+    float sc[SL], cm[SL];
+    uint32_t kc[SL];                                   /* choice_order of the choice, 0: cannot be selected */
+    uint32_t unc = 0u;                                 /* bit i: uncertified */
+    auto set = [&](int i, float s, float smax) {
+        const int e = lane + 64 * i;
+        const float b = bias ? bias[en[i]] : 0.0f, c = s + b;
+        sc[i] = s;
+        cm[i] = smax + b;
+        kc[i] = e < n_experts && c > -INFINITY ? choice_order(c) : 0u;
+    };
+    uint32_t slow = 0u;                                /* bit i: not inside one float's rounding interval */
+#pragma unroll
+    for (int i = 0; i < SL; i++) {
+        const float f = (float)Q[i], s = router_score_w(f, word[i], exc);
+        set(i, s, s);
+        if (fabs(Q[i]) <= 0x1.fffffffffffffp+1023 && lane + 64 * i < n_experts) {
+            const double B = certify_bound(Q[i], bs[i]);
+            double lo, hi;
+            round_interval(f, lo, hi);
+            if (!((Q[i] - B > lo) && (Q[i] + B < hi))) slow |= 1u << i;
+        }
+    }
+    while (__ballot(slow != 0u)) {
+        if (slow) {
+            const int s = __ffs((int)slow) - 1;
+            double q = 0.0, b = 0.0;
+#pragma unroll
+            for (int i = 0; i < SL; i++)
+                if (i == s) {
+                    q = Q[i];
+                    b = bs[i];
+                }
+            const Certified r = certify_score(q, b, exc, exc_word((float)q, exc));
+#pragma unroll
+            for (int i = 0; i < SL; i++)
+                if (i == s) set(i, r.sc, r.scmax);
+            if (!r.ok) unc |= 1u << s;
+            slow &= slow - 1u;
+        }
+    }
+    auto key_of = [&](int i) { return kc[i] ? ((uint64_t)kc[i] << 32) | (uint64_t)(0xffffffffu - (uint32_t)(lane + 64 * i)) : 0ull; };
+    uint64_t mysel = 0ull;
+    float mysc = 0.0f;
+    int nre = 0;
+    for (;;) {
+        uint32_t v = 0u;
+#pragma unroll
+        for (int i = 0; i < SL; i++) v = v > kc[i] ? v : kc[i];
+        int above = 0;
+        for (int i = 0; i < 64; i += 8)
+#pragma unroll
+            for (int q = 0; q < 8; q++) above += (uint32_t)__builtin_amdgcn_readlane((int)v, i + q) > v;
+        /* the topk-th largest of the lanes' maxima: at least topk keys lie at or above it (or all) */
+        const uint32_t t0 = wave_reduce_u32<false>(above < topk ? v : 0xffffffffu);
+        int n = 0;
+#pragma unroll
+        for (int i = 0; i < SL; i++) {
+            const bool in = kc[i] != 0u && kc[i] >= t0;
+            const uint64_t bm = __ballot(in);
+            const int slot = n + __popcll(bm & ((1ull << lane) - 1ull));
+            if (in && slot < 64) {
+                cand[wv][slot] = key_of(i);
+                csc[wv][slot] = sc[i];
+            }
+            n += __popcll(bm);
+        }
+        int nsel = n < topk ? n : topk;
+        if (n <= 64) {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            const uint64_t c = lane < n ? cand[wv][lane] : 0ull;
+            const float s = lane < n ? csc[wv][lane] : 0.0f;
+            const uint32_t ch = (uint32_t)(c >> 32), cl = (uint32_t)c;
+            int rank = 0;
+            for (int i = 0; i < n; i += 4)             /* (zeros past n) */
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const uint64_t o = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)ch, i + q) << 32) |
+                                       (uint32_t)__builtin_amdgcn_readlane((int)cl, i + q);
+                    rank += o > c;
+                }
+            /* lane j takes the key of rank j (unique; lanes without one all send 0 to lane n) */
+            const uint32_t sh = (uint32_t)__builtin_amdgcn_ds_permute(4 * rank, (int)ch);
+            const uint32_t sl = (uint32_t)__builtin_amdgcn_ds_permute(4 * rank, (int)cl);
+            const uint32_t ss = (uint32_t)__builtin_amdgcn_ds_permute(4 * rank, (int)__float_as_uint(s));
+            mysel = lane < nsel ? ((uint64_t)sh << 32) | sl : 0ull;
+            mysc = __uint_as_float(ss);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        } else {
+            uint32_t taken = 0u;
+            mysel = 0ull;
+            for (int j = 0; j < topk; j++) {           /* n > 64 >= topk: every one finds a key */
+                uint64_t head = 0ull;
+                int hi = 0;
+                float hs = 0.0f;
+#pragma unroll
+                for (int i = 0; i < SL; i++) {
+                    const uint64_t k = (taken >> i) & 1u ? 0ull : key_of(i);
+                    if (k > head) {
+                        head = k;
+                        hi = i;
+                        hs = sc[i];
+                    }
+                }
+                const uint64_t m = wave_max_key_fast(head);
+                const int from = __ffsll((unsigned long long)__ballot(head == m)) - 1;
+                const float s = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(hs), from));
+                if (lane == from) taken |= 1u << hi;
+                if (lane == j) {
+                    mysel = m;
+                    mysc = s;
+                }
+            }
+        }
+        /* uncertified logits that matter: selected, or able to reach the selection */
+        if (!__ballot(unc != 0u)) break;
+        const int lj = nsel > 0 ? nsel - 1 : 0;
+        const uint64_t last = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(mysel >> 32), lj) << 32) |
+                              (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)mysel, lj);
+        const float ckth = nsel > 0 ? key_choice(last) : -INFINITY;
+        uint32_t need = 0u;
+#pragma unroll
+        for (int i = 0; i < SL; i++)
+            if (((unc >> i) & 1u) && (nsel < topk || key_of(i) >= last || cm[i] >= ckth)) need |= 1u << i;
+        uint64_t left = __ballot(need != 0u);
+        if (!left) break;
+        while (left) {
+            const int L = __ffsll((unsigned long long)left) - 1;
+            const int s = __builtin_amdgcn_readlane(__ffs((int)need) - 1, L);
+            const double a = chain_wave(ring[wv], W + (size_t)(L + 64 * s) * hidden, x + (size_t)t * hidden, hidden);
+            const float r = router_score((float)a, exc);
+            if (lane == L) {
+#pragma unroll
+                for (int i = 0; i < SL; i++)
+                    if (i == s) set(i, r, r);
+                unc &= ~(1u << s);
+                need &= need - 1u;
+            }
+            nre++;
+            left = __ballot(need != 0u);
+        }
+    }
+    const int id = mysel != 0ull ? (int)(0xffffffffu - (uint32_t)mysel) : -1;
+    const float w = topk_weight(lane < topk && id >= 0 ? mysc : 0.0f, topk, renorm, routed_scale);
+    if (lane < topk) {
+        idx[(size_t)t * topk + lane] = id >= 0 ? id : 0;
+        wt[(size_t)t * topk + lane] = w;
+    }
+    if (nrecomp && lane == 0) nrecomp[t] = nre;
 }
 
 /* ---- expert-major gather -----------------------------------------------------------
@@ -1339,8 +1605,9 @@ extern "C" int k3k_split_bf16(uint16_t *hi, uint16_t *lo, const float *x, size_t
  * block per wave). */
 constexpr int RM_TB = 32, RM_EB = 64;
 
-extern "C" int k3k_router_chunk(int T, int hidden, int n_experts)
+extern "C" int k3k_router_chunk(int T, int hidden, int n_experts, long *load_out)
 {
+    if (load_out) *load_out = 0;
     if (T <= RS_T) return RS_CH;          /* one lane per (expert, 128-column chunk) */
     const long tiles = (long)((n_experts + RM_EB - 1) / RM_EB) * ((T + RM_TB - 1) / RM_TB);
     const long cus = k3k_cu_count() > 0 ? k3k_cu_count() : 1;
@@ -1353,7 +1620,11 @@ extern "C" int k3k_router_chunk(int T, int hidden, int n_experts)
         ks = (ks + K3_NXCD - 1) / K3_NXCD * K3_NXCD;
         while (ks > K3_NXCD && hidden / ks < 224) ks -= K3_NXCD;
         const long chunk = ((hidden + ks - 1) / ks + RP_KS - 1) / RP_KS * RP_KS;
-        if (chunk >= 224 && ((hidden + chunk - 1) / chunk) % K3_NXCD == 0) return (int)chunk;
+        const long n = (hidden + chunk - 1) / chunk;
+        if (chunk >= 224 && n % K3_NXCD == 0) {
+            if (load_out) *load_out = (tiles * n + cus - 1) / cus * chunk;
+            return (int)chunk;
+        }
     }
     /* chunks a multiple of 32 columns and at least 256; among those, the split whose
      * busiest CU has the least work (workgroups per CU x columns per workgroup), the most
@@ -1370,6 +1641,7 @@ extern "C" int k3k_router_chunk(int T, int hidden, int n_experts)
         const long load = per_cu * chunk;
         if (best_load < 0 || load <= best_load) { best_load = load; best_chunk = chunk; }
     }
+    if (load_out) *load_out = best_load;
     return (int)best_chunk;
 }
 
@@ -1528,8 +1800,8 @@ extern "C" int k3k_router_final(int *idx, float *wt, int *nrecomp, const double 
         return 0;
     }
     /* scored records (a few tokens) or the chunk partials: a lane per expert (two past
-     * 1024), all of a lane's partials in one load batch when they are at most 32 -- up to 512
-     * experts the batch is sized to the chunk count (2, 4, 8 or 16: no repeated loads, fewer
+     * 1024), all of a lane's partials in one load batch when they are at most 32 -- the
+     * batch is sized to the chunk count (2, 4, 8 or 16: no repeated loads, fewer
      * registers, more workgroups per CU) -- or 64 for up to 64 tokens and 512 experts (more
      * registers, fewer waves per CU: only while the tokens do not fill the chip). The
      * selection is two-level when the expert groups fit (select_rounds), else wave 0 selects
@@ -1539,18 +1811,37 @@ extern "C" int k3k_router_final(int *idx, float *wt, int *nrecomp, const double 
     hipLaunchKernelGGL((router_final_kernel<SL, SW, KB, PRE>), dim3(T), dim3(NT), 0, st, idx, wt, nrecomp, \
                        part, rbound, ks, chunk, x, W, bias, T, hidden, n_experts, topk, renorm,        \
                        routed_scale, e, gd)
-    if (pre && n_experts <= 512) K3_RF(1, 8, RF_KB, true, 64 * nw);
+#define K3_RFW(SL)                                                                                   \
+    hipLaunchKernelGGL((router_final_wave_kernel<SL>), dim3((unsigned)((T + 3) / 4)), dim3(256), 0, st, idx, wt, \
+                       nrecomp, part, rbound, ks, chunk, x, W, bias, T, hidden, n_experts, topk, renorm, \
+                       routed_scale, e)
+    /* many tokens: a wave each (router_final_wave_kernel) */
+    if (!pre && T >= 3 * k3k_cu_count() && n_experts <= 1024) {
+        if (nw <= 2) K3_RFW(2);
+        else if (nw <= 4) K3_RFW(4);
+        else if (nw <= 6) K3_RFW(6);
+        else if (nw <= 8) K3_RFW(8);
+        else if (nw <= 12) K3_RFW(12);
+        else if (nw <= 14) K3_RFW(14);
+        else K3_RFW(16);
+    } else if (pre && n_experts <= 512) K3_RF(1, 8, RF_KB, true, 64 * nw);
     else if (pre && n_experts <= 1024) K3_RF(1, 16, RF_KB, true, 64 * nw);
     else if (pre) K3_RF(2, 32, RF_KB, true, 64 * nw);
-    else if (n_experts <= 512 && ks <= 2) K3_RF(1, 8, 2, false, 64 * nw);
     else if (n_experts <= 512 && ks <= 4) K3_RF(1, 8, 4, false, 64 * nw);
     else if (n_experts <= 512 && ks <= 8) K3_RF(1, 8, 8, false, 64 * nw);
     else if (n_experts <= 512 && ks <= 16) K3_RF(1, 8, 16, false, 64 * nw);
     else if (n_experts <= 512 && ks > 32 && ks <= 64 && T <= 64) K3_RF(1, 8, 64, false, 64 * nw);
     else if (n_experts <= 512) K3_RF(1, 8, RF_KB, false, 64 * nw);
+    else if (n_experts <= 64 * RF_MAXW && ks <= 4) K3_RF(1, 16, 4, false, 64 * nw);
+    else if (n_experts <= 64 * RF_MAXW && ks <= 8) K3_RF(1, 16, 8, false, 64 * nw);
+    else if (n_experts <= 64 * RF_MAXW && ks <= 16) K3_RF(1, 16, 16, false, 64 * nw);
     else if (n_experts <= 64 * RF_MAXW) K3_RF(1, 16, RF_KB, false, 64 * nw);
+    else if (ks <= 4) K3_RF(2, 32, 4, false, 64 * nw);
+    else if (ks <= 8) K3_RF(2, 32, 8, false, 64 * nw);
+    else if (ks <= 16) K3_RF(2, 32, 16, false, 64 * nw);
     else K3_RF(2, 32, RF_KB, false, 64 * nw);
 #undef K3_RF
+#undef K3_RFW
     K3K_LAUNCH_CHECK("router_final launch");
     return 0;
 }

@@ -57,7 +57,12 @@
 namespace {
 
 constexpr int RI_ND = 6;                 /* digits per operand */
-constexpr int RI_LMAX = 10;              /* products of digits i, j with i + j <= RI_LMAX */
+/* Products of digits i, j with i + j <= RI_LMAX. At 9 what is left out (levels 10 and up, under
+ * 2^-23 of the bound R a chunk of 1792 columns has from its prefixes in units of 2^-53) still adds
+ * nothing to R; the level 10 sums would: 3 products of 33 for no certified logit more (partials of
+ * 4096 tokens x 384 experts 270 -> 257 us; at 8 the bound grows 16 times, and with it the
+ * recomputed logits). */
+constexpr int RI_LMAX = 9;
 constexpr int RI_NL = RI_LMAX - 1;       /* level accumulators, l = 2 .. RI_LMAX */
 constexpr int RI_STEP = 64;              /* columns per step: one int8 matrix instruction */
 constexpr int RI_TT = 64, RI_TE = 64;    /* workgroup tile: tokens, experts */
@@ -263,7 +268,7 @@ __device__ __forceinline__ float ri_bound_up(double rb)
 struct RiPair {
     int i, j;
 };
-constexpr int RI_NP = 33;                /* pairs with i, j <= RI_ND and i + j <= RI_LMAX */
+constexpr int RI_NP = 30;                /* pairs with i, j <= RI_ND and i + j <= RI_LMAX */
 struct RiPairs {
     RiPair p[RI_NP];
 };
@@ -446,27 +451,54 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 }  // namespace
 
 /* ---- host side ------------------------------------------------------------------------ */
-/* The int8 partials serve batches of at least RI_MIN_T tokens with rows of a multiple of
- * 256 columns; fewer tokens keep the fp64 kernels (at 512 tokens those took 84 us against
- * 100 us for the digits and the int8 partials). */
-constexpr int RI_MIN_T = 1024;
+constexpr int RI_MIN_T = 128;            /* fewer tokens: the fp64 kernels */
+constexpr int RI_MAXTT = 128;            /* more token tiles: no choice of chunks */
 
 static int ri_round(int v, int m) { return (v + m - 1) / m * m; }
 
 extern "C" int k3k_router_i8_chunk(int T, int hidden, int n_experts)
 {
     if (T < RI_MIN_T || hidden <= 0 || hidden % RI_STEP || n_experts <= 0) return 0;
-    const long tiles = (long)(ri_round(T, RI_TT) / RI_TT) * (ri_round(n_experts, RI_TE) / RI_TE);
-    const long cus = k3k_cu_count() > 0 ? k3k_cu_count() : 1;
-    /* the fewest chunks (equal, whole step groups of the split) that give every CU two
-     * workgroups, at most RI_CMAX columns each (a scale wave holds its row's chunk) */
+    /* (everything below depends on the token tiles only, so that k3k_router_i8_ws can go over them) */
+    const int Tp = ri_round(T, RI_TT);
+    const long ntt = Tp / RI_TT, nte = ri_round(n_experts, RI_TE) / RI_TE;
+    const long cus = k3k_cu_count() >= K3_NXCD ? k3k_cu_count() / K3_NXCD : 1;     /* per XCD */
+    /* The chunk count (equal chunks, whole step groups of the split, at most RI_CMAX columns each: a
+     * scale wave holds its row's chunk) with the least time on the busiest CU, a workgroup at a time:
+     * rounds on an XCD, which takes whole (chunk, token tile) pairs, x (steps + 10 for a workgroup's
+     * start and end and the partials it adds); the fewest among equals. (The fewest chunks that give
+     * every CU two workgroups, before: 2048 tokens of 128 experts 896 workgroups of 8 steps, 166 us
+     * with the final kernel, now 256 of 28, 103.) */
     if (hidden % (RI_STEP * RI_SPS)) return 0;
     const int ngrp = hidden / (RI_STEP * RI_SPS);
-    int ks = 1;
-    for (; ks < ngrp; ks++)
-        if (ngrp % ks == 0 && tiles * ks >= 2 * cus && hidden / ks <= RI_CMAX) break;
-    while (hidden / ks > RI_CMAX || ngrp % ks) ks++;
-    const size_t xbytes = (size_t)ri_round(T, RI_TT) * (size_t)hidden * RI_ND;
+    int ks = 0;
+    long best = 0;
+    for (int n = 1; n <= ngrp; n++) {
+        if (ngrp % n || hidden / n > RI_CMAX) continue;
+        const long per = (n * ntt + K3_NXCD - 1) / K3_NXCD * nte;
+        const long c = (per + cus - 1) / cus * (hidden / n / RI_STEP + 10);
+        if (!ks || c < best) {
+            ks = n;
+            best = c;
+        }
+        if (ntt > RI_MAXTT) break;             /* rounds enough: the longest chunks */
+    }
+    if (!ks) return 0;
+    /* Up to 1023 tokens: against the fp64 kernel, both in us, fitted to 91 shapes of 128 to 1000
+     * tokens and 128 to 1400 experts of 7168 columns (rms 18 us, most of it at the largest). fp64: the
+     * busiest CU's columns; int8: its steps, the digits of both operands, the partials. Whole router,
+     * fp64 / int8: 384 experts, 300 tokens 59 / 59, 400 67 / 71, 1000 141 / 109 us; 896 experts, 200
+     * tokens 86 / 76, 400 149 / 115, 1000 292 / 203; 128 experts, 512 tokens 36 / 54. From 1024 the
+     * int8 ones always. */
+    if (T < 1024) {
+        long load = 0;
+        const int c64 = k3k_router_chunk(Tp, hidden, n_experts, &load);
+        const double tn = 1e-6 * Tp * n_experts;
+        const double f64 = 0.0266 * (double)load - 2.3 * ((hidden + c64 - 1) / c64) * tn + 17.3;
+        const double i8 = 1.55 * (double)best + 1e-6 * hidden * ((double)Tp + n_experts) + 6.4 * ks * tn + 7.7;
+        if (i8 >= f64) return 0;
+    }
+    const size_t xbytes = (size_t)Tp * (size_t)hidden * RI_ND;
     const size_t wbytes = (size_t)ri_round(n_experts, RI_TE) * (size_t)hidden * RI_ND;
     if (xbytes >= ((size_t)1 << 31) || wbytes >= ((size_t)1 << 31)) return 0;
     return hidden / ks;
@@ -480,6 +512,23 @@ extern "C" size_t k3k_router_i8_bytes(int T, int hidden, int n_experts, int chun
     const size_t ks = (size_t)(hidden / chunk), Tp = ri_round(T, RI_TT), Ep = ri_round(n_experts, RI_TE);
     return ri_al(Tp * hidden * RI_ND) + ri_al(Ep * hidden * RI_ND) + ri_al(Tp * ks * sizeof(RiRow)) +
            ri_al(Ep * ks * sizeof(RiRow));
+}
+
+/* What the partials and the digits of any batch of up to T tokens take: a smaller batch may run on
+ * the int8 kernels, or with more chunks, where T tokens do not. */
+extern "C" size_t k3k_router_i8_ws(int T, int hidden, int n_experts)
+{
+    size_t most = 0;
+    const int top = ri_round(T, RI_TT) / RI_TT;
+    for (int tt = RI_MIN_T / RI_TT; tt <= top && tt <= RI_MAXTT; tt++) {
+        const int t = tt * RI_TT < T ? tt * RI_TT : T;
+        const int chunk = k3k_router_i8_chunk(t, hidden, n_experts);
+        if (!chunk) continue;
+        const size_t ks = (size_t)(hidden / chunk), p = ks < 2 ? 2 : ks;
+        const size_t n = ri_al(p * t * n_experts * 8) + ri_al(ks * t * n_experts * 4) + k3k_router_i8_bytes(t, hidden, n_experts, chunk);
+        if (n > most) most = n;
+    }
+    return most;
 }
 
 extern "C" int k3k_router_partial_i8(double *part, float *rbound, void *scratch, const float *x, int T,

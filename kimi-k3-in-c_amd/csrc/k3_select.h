@@ -16,7 +16,8 @@ namespace {
 struct ExcTable {
     const uint32_t *pairs;      /* sorted (key bits of v, libm expf(v) bits) */
     const uint32_t *index;      /* index[b] = first pair with (key >> 12) - base >= b */
-    const uint32_t *bits;       /* membership bitmap over |key| in [mmin, mmax], per sign */
+    const uint32_t *bits;       /* membership bitmap over |key| in [mmin, mmax], per sign, then a bit
+                                 * per word of it */
     uint32_t kmin, kmax, base, mmin, mwords;
     int n;
 };
@@ -31,6 +32,27 @@ __device__ __forceinline__ uint32_t exc_word(float logit, const ExcTable &x)
     const bool in = x.n > 0 && mag >= x.mmin && w < x.mwords;
     const k3_rsrc r = k3_make_rsrc(x.bits, x.n > 0 ? 8u * x.mwords : 0u);
     return k3_bload4(r, in ? ((key >> 31) * x.mwords + w) * 4u : 0xfffffff0u);
+}
+
+/* The same word where many logits are looked up: the word's slot (~0: outside the range), whether
+ * it has any bit -- from a map a 32nd of the size that stays in the L2s, where the bitmap is some tens
+ * of MB hit at random -- and, for about one logit in a hundred, the word. (4096 tokens x 896
+ * experts: final kernel 192 -> 164 us.) */
+__device__ __forceinline__ uint32_t exc_slot(float logit, const ExcTable &x)
+{
+    const uint32_t key = __float_as_uint(-logit), mag = key & 0x7fffffffu, w = (mag - x.mmin) >> 5;
+    return x.n > 0 && mag >= x.mmin && w < x.mwords ? (key >> 31) * x.mwords + w : 0xffffffffu;
+}
+__device__ __forceinline__ uint32_t exc_any(uint32_t slot, const ExcTable &x)
+{
+    const uint32_t nw = 2u * x.mwords;
+    const k3_rsrc r = k3_make_rsrc(x.bits + nw, x.n > 0 ? (nw + 31u) / 32u * 4u : 0u);
+    return (k3_bload4(r, slot != 0xffffffffu ? (slot >> 5) * 4u : 0xfffffff0u) >> (slot & 31)) & 1u;
+}
+__device__ __forceinline__ uint32_t exc_word_many(float logit, const ExcTable &x)
+{
+    const uint32_t j = exc_slot(logit, x);
+    return exc_any(j, x) ? x.bits[j] : 0u;
 }
 
 /* libm-exact score 1/(1+expf(v)), v = -logit: the deterministic correctly rounded
@@ -179,18 +201,31 @@ struct SelSmem {
     uint64_t last;                                 /* its k-th key and count */
     int nsel;
     int wcnt[16];                                  /* listed experts per wave */
+    uint32_t rmax[64], thr;                        /* threshold selection: row maxima, threshold, */
+    int ncand;                                     /* candidates (in cand) */
 };
 
 /* The reference's rule topk times (largest choice, lowest index among equals, strictly
  * above -inf, none left: idx 0, weight 0; k3_ops.c:459-467) over the scored experts in sm.
  * Keys are unique (the expert's index in the low word), so the selection is the topk
  * largest keys in order, however they are found:
- *  - two levels, when the ng = ceil(n_experts / 64) groups of 64 experts fit the
- *    workgroup's waves and ng * topk <= 256: wave g takes the topk largest keys of group g
- *    (one key per lane, each extraction one wave maximum, wave_max_key_fast), then wave 0
+ *  - by threshold, past 512 experts, when the ng = ceil(n_experts / 64) groups of 64 experts fit
+ *    the workgroup's waves and there are at least topk rows of 16 experts: wave g
+ *    reduces its rows to their largest choices; wave 0 takes the topk-th largest of the (at
+ *    most 64) row maxima, each lane counting the maxima above its own; at least topk keys lie
+ *    at or above it, so only keys there can be selected, and for choices in no particular
+ *    order they are few (about 1.3 topk). They are packed into LDS, and wave 0 ranks them by
+ *    counting, a lane per candidate;
+ *  - two levels, when that leaves more than 64 candidates (many equal choices, or choices in
+ *    order of their expert) or there are too few rows, and ng * topk <= 256: wave g takes the
+ *    topk largest keys of group g (one key per lane, each extraction one wave maximum,
+ *    wave_max_key_fast), then wave 0
  *    the topk largest of those ng * topk candidates (one to four per lane: a lane holds
  *    candidates l + 64 i and the largest of them, and after each pick the lane that held
- *    it takes its next);
+ *    it takes its next). Two chains of topk wave maxima: for 4096 tokens of 896 experts, top
+ *    16, the final kernel of a workgroup per token took 225 us with them and 192 with the threshold, one
+ *    token's 10.0 and 7.5 (up to 512 experts and 8 groups the two chains are as fast: 11.6 / 12.3 us
+ *    for 64 tokens of 384, top 8, so they keep them);
  *  - else wave 0 alone: lane l holds the keys of experts l + 64 i (SW of them) and the
  *    largest of its keys; after each extraction the lane that held it drops the key and
  *    takes its next largest.
@@ -214,10 +249,70 @@ __device__ uint64_t select_rounds(SelSmem<SW> &sm, const float *x, const float *
         return (e < n_experts && c > -INFINITY) ? ((uint64_t)choice_order(c) << 32) | (uint64_t)(0xffffffffu - (uint32_t)e)
                                                 : 0ull;
     };
+    const int nrow = ng * 4;                        /* rows of 16 experts, at most 64 */
+    const bool thr = SW == 16 && two && ng > 8 && nrow >= topk;
     nre = 0;
     uint64_t mysel = 0ull;
     for (int round = 0; round <= n_experts; round++) {
-        if (two) {
+        bool done = false;
+        if (SW == 16 && thr) {
+            const uint64_t k = wv < ng ? key_of(64 * wv + lane) : 0ull;
+            const uint32_t hi = (uint32_t)(k >> 32);
+            if (wv < ng) {
+                uint32_t m = hi;
+                auto mx = [](uint32_t a, uint32_t b) { return a > b ? a : b; };
+                m = mx(m, dpp_u32<0xB1, 0xf, 0u>(m));
+                m = mx(m, dpp_u32<0x4E, 0xf, 0u>(m));
+                m = mx(m, dpp_u32<0x141, 0xf, 0u>(m));
+                m = mx(m, dpp_u32<0x140, 0xf, 0u>(m));
+                if ((lane & 15) == 0) sm.rmax[4 * wv + (lane >> 4)] = m;
+            }
+            if (tid == 0) sm.ncand = 0;
+            __syncthreads();
+            if (wv == 0) {
+                const uint32_t v = lane < nrow ? sm.rmax[lane] : 0u;
+                int above = 0;
+                for (int i = 0; i < nrow; i += 8)               /* (nrow % 4 == 0; zeros past it) */
+#pragma unroll
+                    for (int q = 0; q < 8; q++) above += (uint32_t)__builtin_amdgcn_readlane((int)v, i + q) > v;
+                /* the topk-th largest of the maxima (rows without a key count as 0) */
+                const uint32_t t0 = wave_reduce_u32<false>(lane < nrow && above < topk ? v : 0xffffffffu);
+                if (lane == 0) sm.thr = t0;
+            }
+            __syncthreads();
+            const bool in = k != 0ull && hi >= sm.thr;
+            const uint64_t bm = __ballot(in);
+            if (bm) {
+                int base = 0;
+                if (lane == 0) base = atomicAdd(&sm.ncand, __popcll(bm));
+                base = __builtin_amdgcn_readfirstlane(base);
+                const int slot = base + __popcll(bm & ((1ull << lane) - 1ull));
+                if (in && slot < 64) sm.cand[slot] = k;
+            }
+            __syncthreads();
+            const int n = sm.ncand;
+            done = n <= 64;
+            if (done && wv == 0) {
+                const uint64_t c = lane < n ? sm.cand[lane] : 0ull;
+                const uint32_t ch = (uint32_t)(c >> 32), cl = (uint32_t)c;
+                int rank = 0;
+                for (int i = 0; i < n; i += 4)                  /* (zeros past n) */
+#pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        const uint64_t o = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)ch, i + q) << 32) |
+                                           (uint32_t)__builtin_amdgcn_readlane((int)cl, i + q);
+                        rank += o > c;
+                    }
+                /* lane j takes the key of rank j (unique; lanes without one all send 0 to lane n) */
+                const uint32_t sh = (uint32_t)__builtin_amdgcn_ds_permute(4 * rank, (int)ch);
+                const uint32_t sl = (uint32_t)__builtin_amdgcn_ds_permute(4 * rank, (int)cl);
+                const int nsel = n < topk ? n : topk;
+                mysel = lane < nsel ? ((uint64_t)sh << 32) | sl : 0ull;
+                if (lane == 0) sm.nsel = nsel;
+                if (nsel == 0 ? lane == 0 : lane == nsel - 1) sm.last = mysel;
+            }
+        }
+        if (two && !done) {
             /* level 1: group wv's topk largest keys (0 once none is left) */
             if (wv < ng) {
                 uint64_t k = key_of(64 * wv + lane);
@@ -279,6 +374,8 @@ __device__ uint64_t select_rounds(SelSmem<SW> &sm, const float *x, const float *
                     sm.last = last;
                 }
             }
+        }
+        if (two) {
             __syncthreads();
             /* every wave lists its group's uncertified logits that matter, in expert order */
             const int nsel = sm.nsel;
@@ -375,6 +472,19 @@ __device__ uint64_t select_rounds(SelSmem<SW> &sm, const float *x, const float *
     return mysel;
 }
 
+/* Lane j's weight from the unbiased score w of the j-th selected expert (0 for none), in a wave. */
+__device__ __forceinline__ float topk_weight(float w, int topk, int renorm, float routed_scale)
+{
+    if (renorm && topk > 1) {
+        double s = 0.0;
+        for (int j = 0; j < topk; j++)                      /* j ascending */
+            s += (double)__uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(w), j));
+        const float inv = (float)(1.0 / (s + 1e-20));
+        w = w * inv;
+    }
+    return w * routed_scale;
+}
+
 /* Wave 0, after select_rounds: lane j's expert (-1: none) and its weight -- the unbiased
  * score, renormalised by (float)(1/(sum_j double + 1e-20)) in j order when renorm and
  * topk > 1, times routed_scale (k3_ops.c:469-475); 0 for none. */
@@ -384,15 +494,7 @@ __device__ __forceinline__ void select_weight(const SelSmem<SW> &sm, uint64_t my
 {
     const int lane = threadIdx.x & 63;
     id = mysel != 0ull ? (int)(0xffffffffu - (uint32_t)mysel) : -1;
-    float w = (lane < topk && id >= 0) ? sm.sc[id] : 0.0f;
-    if (renorm && topk > 1) {
-        double s = 0.0;
-        for (int j = 0; j < topk; j++)                      /* j ascending */
-            s += (double)__uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(w), j));
-        const float inv = (float)(1.0 / (s + 1e-20));
-        w = w * inv;
-    }
-    wt = w * routed_scale;
+    wt = topk_weight((lane < topk && id >= 0) ? sm.sc[id] : 0.0f, topk, renorm, routed_scale);
 }
 
 /* The scored record of router_small_kernel for one expert: {score, score of the upper

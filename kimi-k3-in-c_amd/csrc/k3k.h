@@ -74,7 +74,8 @@ int k3k_split_bf16(uint16_t *hi, uint16_t *lo, const float *x, size_t n, void *s
  * and a membership bitmap so that a miss costs one load. */
 typedef struct {
     const uint32_t *pairs, *index;
-    const uint32_t *bits;      /* membership bits of |key| - mmin: [2 signs][mwords] words */
+    const uint32_t *bits;      /* membership bits of |key| - mmin: [2 signs][mwords] words, then
+                                * a bit per word, whether it has any */
     uint32_t kmin, kmax, base, mmin, mwords;
     int n;
 } K3kExc;
@@ -230,7 +231,8 @@ int k3k_gemv_q8(float *y, const float *x, const void *W, int in, int out, int nt
  * fp32 rounding and the logit matters), sigmoid with the host libm's expf, biased
  * first-strict-max top-k, renorm, scale -> idx/wt [T][topk]; nrecomp [T] (may be NULL)
  * receives the number of recomputed logits per token. */
-int k3k_router_chunk(int T, int hidden, int n_experts);
+/* load (may be NULL): the columns of the busiest CU's workgroups */
+int k3k_router_chunk(int T, int hidden, int n_experts, long *load);
 /* 1 when k3k_router_partial scores and certifies the logits itself (a few tokens): its
  * part then holds one 16-byte record per logit, which a selecting decode gate/up reads. */
 int k3k_router_small(int T, int hidden);
@@ -258,6 +260,7 @@ int k3k_router_partial(double *part, float *rbound, const float *x, int T, const
  * k3k_router_chunk's chunk); the scratch they need; the partials (x and W 16-byte aligned,
  * chunk from k3k_router_i8_chunk). */
 int k3k_router_i8_chunk(int T, int hidden, int n_experts);
+size_t k3k_router_i8_ws(int T, int hidden, int n_experts);
 size_t k3k_router_i8_bytes(int T, int hidden, int n_experts, int chunk);
 int k3k_router_partial_i8(double *part, float *rbound, void *scratch, const float *x, int T,
                           const float *W, int hidden, int n_experts, int chunk, int *ctr, int *idx,
