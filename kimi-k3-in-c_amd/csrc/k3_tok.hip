@@ -95,6 +95,7 @@ __device__ __noinline__ float tok_plain_dot(const void *W, const float *x, size_
     for (int k = 0; k < in; k += 4)
 #pragma unroll
         for (int e = 0; e < 4; e++) {
+            if (k + e >= in) break;
             const size_t i = row * (size_t)in + k + e;
             const float w = BF ? k3_bf16_to_f32(((const uint16_t *)W)[i]) : ((const float *)W)[i];
             s[e] = fmaf(w, x[k + e], s[e]);
@@ -120,7 +121,10 @@ __device__ __forceinline__ void tok_cut(k3_u32x4 a, k3_u32x4 b, uint4 &h, uint4 
     l = make_uint4(up(q[0], q[1]), up(q[2], q[3]), up(q[4], q[5]), up(q[6], q[7]));
 }
 
-/* Stages of 32 columns. WT: the weights' type; XT 0: fp32 activations, 1: two bf16 terms.
+/* Stages of 32 columns. WT: the weights' type; XT 0: fp32 activations, 1: two bf16 terms, 2: fp32, and
+ * any K and alignment: a piece may start at any element, so it is loaded into registers (a stage
+ * ahead) and stored into LDS, and the stage that K ends in is loaded by elements; 64 tokens of
+ * 7169 -> 3584 47 us in bf16, 4044 on a wave per row and token, 25 aligned.
  * GLU: tiles 0 and 1 are rpt rows of W and the same rows of W2, y = act(tile 0, tile 1).
  * WT MX: the codes come 128 columns at a time (a piece is a block of 32) into buffers of their
  * own, one chunk ahead, and their scale bytes into registers (lane: row r16, block g; a permute
@@ -161,7 +165,7 @@ __global__ __launch_bounds__(64 * KW) void tok_gemm_kernel(TokArgs a)
     const k3_rsrc rw = k3_make_rsrc((const char *)a.W + row0 * wrow, (uint32_t)(nrow * wrow));
     const k3_rsrc rw2 = k3_make_rsrc(GLU ? (const char *)a.W2 + row0 * wrow : (const char *)a.W, GLU ? (uint32_t)(nrow * wrow) : 0u);
     const k3_rsrc rs = k3_make_rsrc(MX ? a.scales + (size_t)row0 * (a.in / 32) : nullptr, MX ? (uint32_t)nrow * (uint32_t)(a.in / 32) : 0u);
-    const k3_rsrc rx = XT ? k3_make_rsrc(a.xhi + (size_t)tok0 * a.in, a.lo_off + (uint32_t)ntok * (uint32_t)a.in * 2u)
+    const k3_rsrc rx = XT == 1 ? k3_make_rsrc(a.xhi + (size_t)tok0 * a.in, a.lo_off + (uint32_t)ntok * (uint32_t)a.in * 2u)
                           : k3_make_rsrc(a.x + (size_t)tok0 * a.in, (uint32_t)ntok * (uint32_t)a.in * 4u);
     /* the wave's share, whole chunks of MX codes */
     constexpr int U = MX ? 4 : 1;
@@ -179,14 +183,15 @@ __global__ __launch_bounds__(64 * KW) void tok_gemm_kernel(TokArgs a)
         const int pr = isw ? PRW : PRX, row = sl / pr;
         const int p = (sl % pr) ^ ((row / (isw ? RLW : RLX)) & (pr - 1));
         const int wr = GLU ? row & 15 : row;
+        const uint32_t NONE = XT == 2 ? 16u * p : OOB;     /* XT 2: the first row again, for nothing */
         if (isw) {
-            voff[i] = wr < nrow ? (uint32_t)wr * (uint32_t)a.in * ES + 16u * p : OOB;
+            voff[i] = wr < nrow ? (uint32_t)wr * (uint32_t)a.in * ES + 16u * p : NONE;
             col[i] = p * (16 / ES);
-        } else if (XT) {                           /* pieces 0-3: hi, 4-7: lo */
+        } else if (XT == 1) {                      /* pieces 0-3: hi, 4-7: lo */
             voff[i] = row < ntok ? (uint32_t)row * (uint32_t)a.in * 2u + 16u * (p & 3) + (p >> 2) * a.lo_off : OOB;
             col[i] = (p & 3) * 8;
         } else {
-            voff[i] = row < ntok ? (uint32_t)row * (uint32_t)a.in * 4u + 16u * p : OOB;
+            voff[i] = row < ntok ? (uint32_t)row * (uint32_t)a.in * 4u + 16u * p : NONE;
             col[i] = p * 4;
         }
     }
@@ -224,6 +229,37 @@ __global__ __launch_bounds__(64 * KW) void tok_gemm_kernel(TokArgs a)
                      ss * (32u * (isw ? ES : XT ? 2 : 4)));
         }
     };
+    k3_u32x4 reg[XT == 2 ? ND : 1];
+    auto fetch = [&](int s) {
+        typedef k3_u32x4 any_u32x4 __attribute__((aligned(2)));
+        const int left = s < s1 ? a.in - 32 * s : 0;
+#pragma unroll
+        for (int i = 0; i < ND; i++) {
+            const bool isw = i < MT * SLW / 64;
+            const char *q = (isw ? (const char *)a.W + row0 * wrow : (const char *)(a.x + (size_t)tok0 * a.in)) + voff[i];
+            if (left >= 32) {
+                reg[i] = *reinterpret_cast<const any_u32x4 *>(q + (size_t)s * (32 * (isw ? ES : 4)));
+            } else {
+                q += (size_t)s * (32 * (isw ? ES : 4));
+                uint32_t v[4] = {0u, 0u, 0u, 0u};
+                if (isw && ES == 2) {
+#pragma unroll
+                    for (int e = 0; e < 8; e++)
+                        if ((int)col[i] + e < left) v[e >> 1] |= (uint32_t)reinterpret_cast<const uint16_t *>(q)[e] << (16 * (e & 1));
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        if ((int)col[i] + e < left) v[e] = reinterpret_cast<const uint32_t *>(q)[e];
+                }
+                reg[i] = k3_u32x4{v[0], v[1], v[2], v[3]};
+            }
+        }
+    };
+    auto stash = [&](auto slot) {
+        k3_u32x4 *d = buf(slot);
+#pragma unroll
+        for (int i = 0; i < ND; i++) d[wv * WSL + 64 * i + lane] = reg[i];
+    };
     /* Sums in two levels, so that rounding grows with the square root of K's parts: bf16, the
      * matrix instructions of SEG stages start from zero (seg) and their sum goes onto acc; fp32,
      * four chains of two instructions a stage, summed as a tree. (One chain over a wave's whole
@@ -248,7 +284,7 @@ __global__ __launch_bounds__(64 * KW) void tok_gemm_kernel(TokArgs a)
     }
 #pragma unroll
     for (int h = 0; h < 2; h++) {
-        ix[h] = wv * WSL + MT * SLW + r16 * PRX + ((XT ? 4 * h + g : 2 * g + h) ^ ((r16 / RLX) & (PRX - 1)));
+        ix[h] = wv * WSL + MT * SLW + r16 * PRX + ((XT == 1 ? 4 * h + g : 2 * g + h) ^ ((r16 / RLX) & (PRX - 1)));
         /* the last block of an odd N8 holds 8 tokens: columns 8..15 read some of its slots
          * again (a result column depends on its own operand column only, and these go unused) */
         il[h] = N8 & 1 ? ix[h] - (r16 & 8) * PRX : ix[h];
@@ -275,7 +311,7 @@ __global__ __launch_bounds__(64 * KW) void tok_gemm_kernel(TokArgs a)
         for (int b = 0; b < NB; b++)
 #pragma unroll
             for (int h = 0; h < 2; h++) xv[b][h] = d[(b + 1 < NB ? ix[h] : il[h]) + b * 128];
-        if constexpr (BF && XT) {
+        if constexpr (BF && XT == 1) {
 #pragma unroll
             for (int b = 0; b < NB; b++) {
 #pragma unroll
@@ -331,6 +367,16 @@ __global__ __launch_bounds__(64 * KW) void tok_gemm_kernel(TokArgs a)
     /* MX: the chunk copies lie between stage copies, so a stage's wait lets fewer stages be in
      * flight, never more; a chunk's were issued before its first stage's. */
     constexpr int UN = MX ? 8 : ST;                /* stages per loop */
+    if constexpr (XT == 2) {
+        fetch(s0);
+        for (int s = s0; s < s1; s += UN)
+            k3_tok_for<UN>([&](auto st) {
+                constexpr int S = decltype(st)::value;
+                stash(std::integral_constant<int, S % ST>{});
+                fetch(s + S + 1);
+                comp(std::integral_constant<int, S % ST>{}, st);
+            });
+    } else {
     if constexpr (MX) copy_w(s0 / 4, std::integral_constant<int, 0>{});
     k3_tok_for<ST - 1>([&](auto sl) { copy(s0 + decltype(sl)::value, sl); });
     for (int s = s0; s < s1; s += UN)              /* a stage past the share multiplies zeros */
@@ -344,6 +390,7 @@ __global__ __launch_bounds__(64 * KW) void tok_gemm_kernel(TokArgs a)
             __builtin_amdgcn_sched_barrier(0);
             comp(std::integral_constant<int, S % ST>{}, st);
         });
+    }
     /* the waves' sums, in wave order */
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
@@ -369,7 +416,7 @@ __global__ __launch_bounds__(64 * KW) void tok_gemm_kernel(TokArgs a)
                 for (int k = 0; k < KW - 1; k++) v[h] += red[(k * MT * NB + (m + h) * NB + b) * 64 + lane];
             }
             if (t >= a.ntok || 16 * b + r16 >= 8 * N8 || lr >= nrow) continue;
-            if constexpr (!MX && !XT) {
+            if constexpr (!MX && XT != 1) {
 #pragma unroll
                 for (int h = 0; h < (GLU ? 2 : 1); h++)
 #pragma unroll
@@ -401,7 +448,7 @@ int launch_tok(TokArgs a, hipStream_t st)
     constexpr int SKB = MX ? N8 : MT * (WT == TOK_F32 ? 2 : 1) + N8, CKB = MX ? 2 * MT : 0;
     constexpr int KW = 8 * (2 * SKB + CKB) <= 160 ? 8 : 4;
     constexpr int RKB = (KW - 1) * MT * ((N8 + 1) / 2) - KW * SKB;       /* the sums beyond buffer 0 */
-    constexpr int S4 = (160 - (RKB > 0 ? RKB : 0) - KW * CKB) / (KW * SKB), ST = S4 >= 4 ? 4 : MX ? 2 : S4;
+    constexpr int S4 = (160 - (RKB > 0 ? RKB : 0) - KW * CKB) / (KW * SKB), ST = XT == 2 ? 2 : S4 >= 4 ? 4 : MX ? 2 : S4;
     const int rows = GLU ? a.rpt : 16 * MT;
     a.ntt = (a.ntok + 8 * N8 - 1) / (8 * N8);
     a.items = (a.out + rows - 1) / rows * a.ntt;
@@ -466,6 +513,17 @@ int dispatch_tok(const TokArgs &a, hipStream_t st)
     }
 }
 
+/* any K and alignment: fewer shapes */
+template <int WT>
+int dispatch_any(const TokArgs &a, hipStream_t st)
+{
+    const bool two = (a.out + 31) / 32 * ((a.ntok + 63) / 64) >= k3k_cu_count();
+    if (a.ntok <= 8) return two ? launch_tok<WT, 2, 0, 2, 1>(a, st) : launch_tok<WT, 2, 0, 1, 1>(a, st);
+    if (a.ntok <= 16) return two ? launch_tok<WT, 2, 0, 2, 2>(a, st) : launch_tok<WT, 2, 0, 1, 2>(a, st);
+    if (a.ntok <= 32) return two ? launch_tok<WT, 2, 0, 2, 4>(a, st) : launch_tok<WT, 2, 0, 1, 4>(a, st);
+    return two ? launch_tok<WT, 2, 0, 2, 8>(a, st) : launch_tok<WT, 2, 0, 1, 8>(a, st);
+}
+
 }  // namespace
 
 /* in % 8 == 0, x and W 16-byte aligned, and a row block's operand under 2 GiB. Up to four tokens
@@ -476,15 +534,17 @@ static int shape_ok(const void *x, const void *W, int in)
     return in >= 8 && in % 8 == 0 && in < (1 << 22) && (((uintptr_t)x | (uintptr_t)W) & 15) == 0;
 }
 
+/* One token of aligned rows stays on the vector units, and so do up to four of short rows: their
+ * sums are the more accurate there. */
 extern "C" int k3k_tok_ok(const float *x, const void *W, int in, int ntok)
 {
-    return ntok > 1 && (ntok > 4 || in >= 512) && shape_ok(x, W, in);
+    return (ntok > 4 || in >= 512) && in >= 8 && in < (1 << 22) && (ntok > 1 || !shape_ok(x, W, in));
 }
 
 extern "C" int k3k_tok_gemm(float *y, const float *x, const void *W, int bf16, int in, int out, int ntok, int ldy,
                             int accumulate, void *stream)
 {
-    if (!shape_ok(x, W, in)) return k3k_fail("tok gemm shape", hipErrorInvalidValue);
+    if (in < 8 || in >= (1 << 22)) return k3k_fail("tok gemm shape", hipErrorInvalidValue);
     if (out <= 0) return 0;
     TokArgs a = {};
     a.y = y;
@@ -495,6 +555,8 @@ extern "C" int k3k_tok_gemm(float *y, const float *x, const void *W, int bf16, i
     a.ntok = ntok;
     a.ldy = ldy;
     a.accumulate = accumulate;
+    if (!shape_ok(x, W, in))
+        return bf16 ? dispatch_any<TOK_BF16>(a, (hipStream_t)stream) : dispatch_any<TOK_F32>(a, (hipStream_t)stream);
     return bf16 ? dispatch_tok<TOK_BF16, 0>(a, (hipStream_t)stream) : dispatch_tok<TOK_F32, 0>(a, (hipStream_t)stream);
 }
 
