@@ -36,3 +36,27 @@ def test_router_select_edges(gpu, orc, k3, T, N, K):
             i2, w2 = orc.router(X[t], W, bias, K, 1, 2.5)
             assert np.array_equal(idx[t], i2), (t, idx[t], i2)
             assert np.array_equal(bits(wt[t]), bits(w2)), t
+
+
+@pytest.mark.parametrize("T,N,K", [(256, 896, 8), (128, 896, 16), (200, 1000, 10), (600, 640, 3)])
+def test_router_int8_partials_with_gather(gpu, orc, k3, T, N, K):
+    """The routed layer at sizes whose partials come from the int8 kernels (or nearly) and whose
+    gather runs in the final kernel's last workgroup; no expert is in the bank, so the layer
+    is routing and gather alone."""
+    from test_gpu_moe_device import stable_gather
+    hid, inter = 7168, 512
+    say(f"case: routing and gather {N} experts top-{K}, {T} tokens")
+    W = k3.gen_normal(N * hid, 21 + N).reshape(N, hid) * np.float32(0.02)
+    X = k3.gen_normal(T * hid, 22 + T).reshape(T, hid)
+    bias = k3.gen_normal(N, 23, 0.0, 0.02)
+    b = gpu.DevBank([None] * N, hid, inter)
+    try:
+        out, idx, wt, perm, off, drops = gpu.moe_routed_device(b, X, W, bias, K, inter=inter)
+    finally:
+        b.free()
+    assert drops == T * K and not out.any()
+    p2, off2 = stable_gather(idx, N)
+    assert np.array_equal(perm, p2) and np.array_equal(off, off2)
+    for t in range(T):
+        i2, w2 = orc.router(X[t], W, bias, K, 1, 1.0)
+        assert np.array_equal(idx[t], i2) and np.array_equal(bits(wt[t]), bits(w2)), t
