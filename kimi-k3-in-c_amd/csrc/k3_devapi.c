@@ -193,11 +193,12 @@ int k3d_matmul_mxfp4(float *y, const float *x, int ntok, const uint8_t *packed,
     if (k3k_mx_small_ok(ntok, in, prec == 0 ? 2 : 1, rows, x)) {
         a.xf32 = x;                 /* one or two tokens: the kernel splits x itself */
     } else if (k3k_tok_mx_ok(w.xhi, w.xlo, packed, in, ntok)) {
-        /* three tokens and more (7168 -> 2048: 13.4 -> 11.2 us at 3, 273 -> 54 at 512); one term
-         * asked for: two cost no more here (172 -> 54) and are the more accurate */
-        if (k3k_split_bf16(w.xhi, w.xlo, x, (size_t)ntok * in, stream)) return fail("split");
+        /* three tokens and more (7168 -> 2048: 13.4 -> 11.2 us at 3, 273 -> 54 at 512, one term
+         * 172 -> 54) */
+        uint16_t *lo = prec == 0 ? w.xlo : NULL;
+        if (k3k_split_bf16(w.xhi, lo, x, (size_t)ntok * in, stream)) return fail("split");
         k3k_prof_mark(stream, K3D_STAGE_BEGIN);
-        if (k3k_tok_mx(y, w.xhi, w.xlo, packed, scales, in, rows, ntok, rows, stream)) return fail("tok_mx");
+        if (k3k_tok_mx(y, w.xhi, lo, packed, scales, in, rows, ntok, rows, stream)) return fail("tok_mx");
         k3k_prof_mark(stream, K3D_STAGE_GEMV);
         return 0;
     } else {

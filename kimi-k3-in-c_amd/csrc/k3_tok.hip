@@ -18,8 +18,9 @@
  *     so bits of x below that are dropped: only an |x| under 2^-109 has any.
  *   fp32 weights: v_mfma_f32_16x16x4_f32 on the values as they are.
  *   MXFP4 weights (k3_matmul_mxfp4 of the reference for three tokens and more): the codes are
- *     exact in bf16 under their block's scale; x comes as two rounded bf16 terms, the entry
- *     point's precision. The expert streaming kernel, which reads the weights once per 16 or 32
+ *     exact in bf16 under their block's scale; x comes as two rounded bf16 terms, or one where
+ *     the entry point's caller asked for that (the other's products are of zeros: a kernel
+ *     without them would save little, the weights and x bound it). The expert streaming kernel, which reads the weights once per 16 or 32
  *     tokens through a register ring, took 16 / 39 / 273 us for 7168 -> 2048 at 8 / 64 / 512
  *     tokens and 3575 at 512 of 12288 -> 16384; here 11.5 / 22 / 54 and 635. K of any multiple
  *     of 32: the scales come a byte at a time, since a row's start is at no multiple of 4 (dwords
@@ -78,7 +79,7 @@ struct TokArgs {
     float *y;
     const float *x;                       /* fp32 activations, or */
     const uint16_t *xhi;                  /* their two bf16 terms, lo_off bytes apart */
-    uint32_t lo_off;
+    uint32_t lo_off;                      /* (0: one term, the other reads as zeros) */
     const void *W, *W2;                   /* W2: GLU's up matrix */
     const uint8_t *scales;                /* MX */
     int in, out, ntok, ldy, accumulate;
@@ -188,7 +189,7 @@ __global__ __launch_bounds__(64 * KW) void tok_gemm_kernel(TokArgs a)
             voff[i] = wr < nrow ? (uint32_t)wr * (uint32_t)a.in * ES + 16u * p : NONE;
             col[i] = p * (16 / ES);
         } else if (XT == 1) {                      /* pieces 0-3: hi, 4-7: lo */
-            voff[i] = row < ntok ? (uint32_t)row * (uint32_t)a.in * 2u + 16u * (p & 3) + (p >> 2) * a.lo_off : OOB;
+            voff[i] = row < ntok && (p < 4 || a.lo_off) ? (uint32_t)row * (uint32_t)a.in * 2u + 16u * (p & 3) + (p >> 2) * a.lo_off : OOB;
             col[i] = (p & 3) * 8;
         } else {
             voff[i] = row < ntok ? (uint32_t)row * (uint32_t)a.in * 4u + 16u * p : NONE;
@@ -593,6 +594,7 @@ extern "C" int k3k_tok_glu(float *y, const float *x, const uint16_t *Wg, const u
 /* both terms reachable from xhi with 32-bit offsets */
 static int terms_ok(const uint16_t *xhi, const uint16_t *xlo, int in, int ntok, uint32_t *lo_off)
 {
+    if (!xlo) xlo = xhi;                   /* one term */
     const uint64_t d = (uint64_t)((const char *)xlo - (const char *)xhi);
     if (xlo < xhi || d + (uint64_t)ntok * in * 2 >= 0x80000000u || (((uintptr_t)xhi | (uintptr_t)xlo) & 15)) return 0;
     *lo_off = (uint32_t)d;

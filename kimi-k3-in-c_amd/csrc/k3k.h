@@ -215,7 +215,7 @@ int k3k_tok_glu(float *y, const float *x, const uint16_t *Wg, const uint16_t *Wu
 int k3k_tok_terms_ok(const uint16_t *xhi, const uint16_t *xlo, const uint16_t *W, int in, int ntok);
 int k3k_tok_terms(float *y, int ldy, int accumulate, const uint16_t *W, const uint16_t *xhi, const uint16_t *xlo, int in,
                   int out, int ntok, void *stream);
-/* MXFP4 weights (row-major, group 32) times three tokens and more given as two bf16 terms, where
+/* MXFP4 weights (row-major, group 32) times three tokens and more given as two bf16 terms, or one (xlo NULL), where
  * k3k_tok_mx_ok holds (in % 32 == 0, packed 16-byte aligned, the terms within 2 GiB of each other). */
 int k3k_tok_mx_ok(const uint16_t *xhi, const uint16_t *xlo, const void *packed, int in, int ntok);
 int k3k_tok_mx(float *y, const uint16_t *xhi, const uint16_t *xlo, const void *packed, const uint8_t *scales, int in,

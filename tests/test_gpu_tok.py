@@ -11,6 +11,13 @@ from test_gpu_dense import dev_matmul, say
 pytestmark = pytest.mark.gpu
 
 
+def bf16_rne(x):
+    """Finite fp32 values rounded to bf16, nearest even, as fp64."""
+    u = np.ascontiguousarray(x, np.float32).view(np.uint32).astype(np.uint64)
+    u = ((u + 0x7FFF + ((u >> 16) & 1)) >> 16 << 16).astype(np.uint32)
+    return u.view(np.float32).astype(np.float64)
+
+
 @pytest.mark.parametrize("bf16", [True, False])
 @pytest.mark.parametrize("T,inn,out", [(2, 8, 1), (3, 7168, 12288), (16, 24, 17), (17, 64, 16), (33, 1000, 129), (37, 7168, 3584),
                                        (64, 104, 4100), (65, 264, 300), (130, 2056, 1031), (256, 512, 4099),
@@ -69,7 +76,8 @@ def test_tok_matmul_nonfinite(gpu, k3, bf16, inn):
                                         (3, 32, 5), (19, 224, 100), (40, 1504, 515), (100, 4128, 70)])
 def test_tok_mxfp4_edges(gpu, k3, T, inn, rows):
     """k3d_matmul_mxfp4 from three tokens: the activations are two bf16 terms, off by at most
-    2^-17 of each (8 bits a term, rounded, and a sign), and a block whose scale is NaN is 0."""
+    2^-17 of each (8 bits a term, rounded, and a sign), or one, rounded to nearest even; a block
+    whose scale is NaN is 0."""
     say(f"case: mxfp4 {T} tokens {inn} -> {rows}")
     rng = np.random.default_rng(T)
     codes = rng.integers(0, 256, (rows, inn // 2), dtype=np.uint8)
@@ -88,7 +96,11 @@ def test_tok_mxfp4_edges(gpu, k3, T, inn, rows):
         for prec in (0, 1):
             gpu.check(L.k3d_matmul_mxfp4(dy.ptr, dx.ptr, T, dp.ptr, ds.ptr, inn, rows, prec, ws.ptr, ws.nbytes, None), "mxfp4")
             Y = dy.download(np.empty((T, rows), np.float32))
-            assert (np.abs(Y - want) <= (2.0**-17 + 1e-6) * bound).all(), prec
+            if prec == 0:
+                assert (np.abs(Y - want) <= (2.0**-17 + 1e-6) * bound).all()
+            else:                       # the products of the rounded activations, summed in fp32
+                one = bf16_rne(X)
+                assert (np.abs(Y - one @ W.T) <= 1e-6 * (np.abs(one) @ np.abs(W.T))).all()
     finally:
         for b in bufs:
             b.free()
