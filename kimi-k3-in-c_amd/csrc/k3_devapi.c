@@ -833,7 +833,7 @@ int k3d_shared_expert(float *y, int accumulate, const float *x, int T, const uin
     if (T <= 32 && (long)Tp * hidden <= 131072 && inter <= 16 * k3k_cu_count() && ws_bytes >= (size_t)T * inter * 4 &&
         k3k_tok_glu_ok(x, w1, w3, hidden) && k3k_tok_glu_ok(ws, w2, w2, inter)) {
         float *a32 = (float *)ws;
-        if (k3k_tok_glu(a32, x, w1, w3, hidden, inter, T, act, b1, b2, stream)) return fail("shared gate/up");
+        if (k3k_tok_glu(a32, x, w1, w3, hidden, inter, T, act, b1, b2, prec == 0 ? 3 : 1, stream)) return fail("shared gate/up");
         if (k3k_tok_gemm(y, a32, w2, 1, inter, hidden, T, hidden, accumulate, stream)) return fail("shared down");
         k3k_prof_mark(stream, K3D_STAGE_SHARED);
         return 0;

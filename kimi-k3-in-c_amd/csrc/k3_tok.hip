@@ -122,11 +122,27 @@ __device__ __forceinline__ void tok_cut(k3_u32x4 a, k3_u32x4 b, uint4 &h, uint4 
     l = make_uint4(up(q[0], q[1]), up(q[2], q[3]), up(q[4], q[5]), up(q[6], q[7]));
 }
 
+/* eight floats -> one bf16 term each, to nearest even (v_cvt_pk_bf16_f32; 8 tokens of 7168 -> 2048
+ * through the shared expert 20.2 us, 24.0 with k3_bf16_rne, three terms 21.7) */
+__device__ __forceinline__ uint4 tok_round(k3_u32x4 a, k3_u32x4 b)
+{
+    typedef float f2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 h2 __attribute__((ext_vector_type(2)));
+    const uint32_t u[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    uint32_t p[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+        p[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f2{__uint_as_float(u[2 * e]), __uint_as_float(u[2 * e + 1])}), h2));
+    return make_uint4(p[0], p[1], p[2], p[3]);
+}
+
 /* Stages of 32 columns. WT: the weights' type; XT 0: fp32 activations, 1: two bf16 terms, 2: fp32, and
  * any K and alignment: a piece may start at any element, so it is loaded into registers (a stage
  * ahead) and stored into LDS, and the stage that K ends in is loaded by elements; 64 tokens of
  * 7169 -> 3584 47 us in bf16, 4044 on a wave per row and token, 25 aligned.
- * GLU: tiles 0 and 1 are rpt rows of W and the same rows of W2, y = act(tile 0, tile 1).
+ * GLU: tiles 0 and 1 are rpt rows of W and the same rows of W2, y = act(tile 0, tile 1). GLU 2: x
+ * is rounded to one bf16 term, and so is y (stored as fp32, whose cut is that term and zeros): the
+ * one-term precision of the shared expert.
  * WT MX: the codes come 128 columns at a time (a piece is a block of 32) into buffers of their
  * own, one chunk ahead, and their scale bytes into registers (lane: row r16, block g; a permute
  * hands a stage's to its rows' lanes); lane group g takes dword g of the block a stage
@@ -327,18 +343,23 @@ __global__ __launch_bounds__(64 * KW) void tok_gemm_kernel(TokArgs a)
                     for (int m = 0; m < MT; m++) acc[m][b] += seg[m][b];
             }
         } else if constexpr (BF) {
-            uint4 t[2][3];
-            tok_cut(xv[0][0], xv[0][1], t[0][0], t[0][1], t[0][2]);
+            constexpr int NT = GLU == 2 ? 1 : 3;
+            uint4 t[2][NT];
+            auto terms = [&](int b, uint4 *o) {
+                if constexpr (NT == 1) o[0] = tok_round(xv[b][0], xv[b][1]);
+                else tok_cut(xv[b][0], xv[b][1], o[0], o[1], o[2]);
+            };
+            terms(0, t[0]);
 #pragma unroll
             for (int b = 0; b < NB; b++) {
-                if (b + 1 < NB) tok_cut(xv[b + 1][0], xv[b + 1][1], t[(b + 1) & 1][0], t[(b + 1) & 1][1], t[(b + 1) & 1][2]);
+                if (b + 1 < NB) terms(b + 1, t[(b + 1) & 1]);
 #pragma unroll
-                for (int k = 2; k >= 0; k--)
+                for (int k = NT - 1; k >= 0; k--)
 #pragma unroll
                     for (int m = 0; m < MT; m++)
                         seg[m][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(k3_bf16x8, w[m][0]),
                                                                             k3_as_bf16x8(t[b & 1][k]),
-                                                                            S % SEG == 0 && k == 2 ? zero : seg[m][b], 0, 0, 0);
+                                                                            S % SEG == 0 && k == NT - 1 ? zero : seg[m][b], 0, 0, 0);
                 if (S % SEG == SEG - 1)
 #pragma unroll
                     for (int m = 0; m < MT; m++) acc[m][b] += seg[m][b];
@@ -417,7 +438,7 @@ __global__ __launch_bounds__(64 * KW) void tok_gemm_kernel(TokArgs a)
                 for (int k = 0; k < KW - 1; k++) v[h] += red[(k * MT * NB + (m + h) * NB + b) * 64 + lane];
             }
             if (t >= a.ntok || 16 * b + r16 >= 8 * N8 || lr >= nrow) continue;
-            if constexpr (!MX && XT != 1) {
+            if constexpr (!MX && XT != 1 && GLU != 2) {        /* (one term has no such case) */
 #pragma unroll
                 for (int h = 0; h < (GLU ? 2 : 1); h++)
 #pragma unroll
@@ -427,7 +448,10 @@ __global__ __launch_bounds__(64 * KW) void tok_gemm_kernel(TokArgs a)
             }
             if constexpr (GLU)
 #pragma unroll
-                for (int e = 0; e < 4; e++) v[0][e] = k3_act_pair(v[0][e], v[1][e], a.act, a.b1, a.b2);
+                for (int e = 0; e < 4; e++) {
+                    v[0][e] = k3_act_pair(v[0][e], v[1][e], a.act, a.b1, a.b2);
+                    if (GLU == 2) v[0][e] = k3_bf16_to_f32(k3_bf16_rne(v[0][e]));
+                }
             float *o = a.y + (size_t)t * a.ldy + r;
             if (vec) {
                 if (a.accumulate) v[0] = *reinterpret_cast<const k3_f32x4 *>(o) + v[0];
@@ -567,7 +591,7 @@ extern "C" int k3k_tok_glu_ok(const void *x, const void *Wg, const void *Wu, int
 }
 
 extern "C" int k3k_tok_glu(float *y, const float *x, const uint16_t *Wg, const uint16_t *Wu, int in, int out, int ntok,
-                           int act, float b1, float b2, void *stream)
+                           int act, float b1, float b2, int terms, void *stream)
 {
     if (!k3k_tok_glu_ok(x, Wg, Wu, in)) return k3k_fail("tok glu shape", hipErrorInvalidValue);
     if (out <= 0) return 0;
@@ -586,9 +610,14 @@ extern "C" int k3k_tok_glu(float *y, const float *x, const uint16_t *Wg, const u
      * rounds of them: 37.6 us with the down product, 38.7 on the GEMMs): the weight stream, not the
      * products, is what takes the time */
     a.rpt = (out + 7) / 8 <= k3k_cu_count() ? 8 : 16;
-    return ntok <= 8    ? launch_tok<TOK_BF16, 0, 1, 2, 1>(a, (hipStream_t)stream)
-           : ntok <= 16 ? launch_tok<TOK_BF16, 0, 1, 2, 2>(a, (hipStream_t)stream)
-                        : launch_tok<TOK_BF16, 0, 1, 2, 4>(a, (hipStream_t)stream);
+    hipStream_t st = (hipStream_t)stream;
+    if (terms == 1)
+        return ntok <= 8    ? launch_tok<TOK_BF16, 0, 2, 2, 1>(a, st)
+               : ntok <= 16 ? launch_tok<TOK_BF16, 0, 2, 2, 2>(a, st)
+                            : launch_tok<TOK_BF16, 0, 2, 2, 4>(a, st);
+    return ntok <= 8    ? launch_tok<TOK_BF16, 0, 1, 2, 1>(a, st)
+           : ntok <= 16 ? launch_tok<TOK_BF16, 0, 1, 2, 2>(a, st)
+                        : launch_tok<TOK_BF16, 0, 1, 2, 4>(a, st);
 }
 
 /* both terms reachable from xhi with 32-bit offsets */

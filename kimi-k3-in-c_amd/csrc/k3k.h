@@ -207,11 +207,11 @@ int k3k_tok_ok(const float *x, const void *W, int in, int ntok);
 int k3k_tok_gemm(float *y, const float *x, const void *W, int bf16, int in, int out, int ntok, int ldy, int accumulate,
                  void *stream);
 /* y[t][r] = act(gate, up) of bf16 weights, fp32 x, where k3k_tok_glu_ok holds (as k3k_tok_gemm:
- * in % 8 == 0, 16-byte aligned); k3k_tok_terms: y[t][r] (=, or +=) the products with x as two bf16 terms,
+ * in % 8 == 0, 16-byte aligned); terms 1: x and y rounded to bf16, else 3. k3k_tok_terms: y[t][r] (=, or +=) the products with x as two bf16 terms,
  * where k3k_tok_terms_ok holds (in % 8 == 0, 16-byte aligned). */
 int k3k_tok_glu_ok(const void *x, const void *Wg, const void *Wu, int in);
 int k3k_tok_glu(float *y, const float *x, const uint16_t *Wg, const uint16_t *Wu, int in, int out, int ntok, int act,
-                float b1, float b2, void *stream);
+                float b1, float b2, int terms, void *stream);
 int k3k_tok_terms_ok(const uint16_t *xhi, const uint16_t *xlo, const uint16_t *W, int in, int ntok);
 int k3k_tok_terms(float *y, int ldy, int accumulate, const uint16_t *W, const uint16_t *xhi, const uint16_t *xlo, int in,
                   int out, int ntok, void *stream);

@@ -131,3 +131,22 @@ def test_shared_expert_few_tokens(gpu, k3, act, T, hidden, inter):
                 assert np.abs(got - ref).max() <= 1e-4 * np.abs(ref).max()
             else:
                 assert np.linalg.norm(got - ref) <= 2e-2 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("T,hidden,inter", [(1, 256, 512), (3, 4096, 256), (8, 7168, 192), (16, 512, 1024), (17, 1024, 64),
+                                            (32, 4096, 128), (33, 4096, 128), (130, 512, 1024)])
+def test_shared_expert_one_term(gpu, k3, T, hidden, inter):
+    """prec 1 rounds the activations to one bf16 term, x and act(gate, up) alike, whatever kernel
+    serves the token count. Against that computed in fp64: what is left is fp32 sums, and act
+    values that these carry over a rounding boundary, a few of `inter` at 2^-8 each; products
+    of unrounded activations would be off by 2e-3."""
+    say(f"case: shared expert, one term, {T} tokens {hidden} -> {inter}")
+    W = [k3.gen_bf16_normal(hidden * inter, 51 + i + T, 0.0, 0.03) for i in range(3)]
+    F = [(w.astype(np.uint32) << 16).view(np.float32).astype(np.float64) for w in W]
+    X = k3.gen_normal(T * hidden, 60 + T).reshape(T, hidden)
+    xr = bf16_rne(X)
+    g, u = xr @ F[0].reshape(inter, hidden).T, xr @ F[1].reshape(inter, hidden).T
+    want = bf16_rne((g / (1.0 + np.exp(-g)) * u).astype(np.float32)) @ F[2].reshape(hidden, inter).T
+    got = gpu.shared_expert_device(X, *[w.reshape(s) for w, s in zip(W, ((inter, hidden), (inter, hidden), (hidden, inter)))],
+                                   hidden, inter, act=1, prec=1, y0=None)
+    assert np.linalg.norm(got - want) <= 5e-4 * np.linalg.norm(want)
