@@ -144,8 +144,8 @@ int k3d_moe_routed(float *out, int *idx, float *wt, const float *x, int T,
  * hipMalloc). No counterpart in the reference. The scratch lives in a static device array
  * of K3D_STATIC_WS_BYTES (40 MiB) that each GPU holds until the process ends: enough for
  * decode batches of up to 64 tokens at hidden 7168 / inter 2048 / 384 experts / top-8 or
- * at 3584 / 3072 / 896 / top-16 (k3d_moe_ws of the call must not exceed it; larger calls
- * return an error). k3d_init must have run on the device first (it looks the array up and
+ * at 3584 / 3072 / 896 / top-16 (what the call itself takes must not exceed it, which can be less
+ * than k3d_moe_ws, sized for any smaller batch too; larger calls return an error). k3d_init must have run on the device first (it looks the array up and
  * makes the one-time uploads). All calls on one GPU share the array: calls that overlap
  * on one GPU race. Otherwise identical to k3d_moe_routed, results bit for bit. */
 #define K3D_STATIC_WS_BYTES ((size_t)40 << 20)

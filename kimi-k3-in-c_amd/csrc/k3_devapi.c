@@ -241,26 +241,41 @@ typedef struct {
     double *part;
     float *rbound;
     int *nrecomp;
-    int *ctr;                   /* the final kernel's arrival counter, when it gathers */
+    int *ctr;                   /* the final kernel's arrival counter, when it gathers, and the chunk it summed */
     int chunk;
     void *i8;                   /* scratch of the int8 partials (NULL: the fp64 ones) */
 } RtWs;
 
-static size_t router_layout(Carve *c, RtWs *w, int T, int hidden, int n_experts)
+static void router_layout(Carve *c, RtWs *w, int T, int hidden, int n_experts, int chunk, int i8)
 {
-    const int c8 = k3k_router_i8_chunk(T, hidden, n_experts);
-    w->chunk = c8 ? c8 : k3k_router_chunk(T, hidden, n_experts, NULL);
-    const size_t ks = (size_t)((hidden + w->chunk - 1) / w->chunk);
+    const size_t ks = (size_t)((hidden + chunk - 1) / chunk);
+    w->chunk = chunk;
+    w->nrecomp = (int *)take(c, (size_t)T * 4);
+    w->ctr = (int *)take(c, 8);
     /* chunk partials, or (a few tokens) one 16-byte scored record per logit */
     w->part = (double *)take(c, (ks < 2 ? 2 : ks) * T * n_experts * 8);
     w->rbound = (float *)take(c, ks * T * n_experts * 4);
-    w->nrecomp = (int *)take(c, (size_t)T * 4);
-    w->ctr = (int *)take(c, 4);
-    w->i8 = c8 ? take(c, k3k_router_i8_bytes(T, hidden, n_experts, c8)) : NULL;
-    return c->off;
+    w->i8 = i8 ? take(c, k3k_router_i8_bytes(T, hidden, n_experts, chunk)) : NULL;
 }
 
-/* What router_layout takes for any batch of up to T tokens: scratch sized for T tokens serves
+/* The router's part of a workspace that ends at ws_bytes: the int8 partials where they serve the
+ * batch and fit, else the fp64 ones (idx and weights are the same bits). 0 if neither fits; *need
+ * (may be NULL): the smaller of the two. */
+static int router_plan(Carve *c, RtWs *w, size_t ws_bytes, int T, int hidden, int n_experts, size_t *need)
+{
+    const int chunk[2] = {k3k_router_i8_chunk(T, hidden, n_experts), k3k_router_chunk(T, hidden, n_experts, NULL)};
+    const Carve start = *c;
+    for (int i = 0; i < 2; i++) {
+        if (!chunk[i]) continue;
+        *c = start;
+        router_layout(c, w, T, hidden, n_experts, chunk[i], i == 0);
+        if (need && (i == 0 || !chunk[0] || c->off < *need)) *need = c->off;
+        if (c->off <= ws_bytes) return 1;
+    }
+    return 0;
+}
+
+/* What the router takes for any batch of up to T tokens: scratch sized for T tokens serves
  * fewer, which may take the other partials, or more chunks. (The fp64 kernel's chunks: at most 12
  * workgroups of 2048 logits per CU, and 28 of 256 columns of 7168; what it takes past that it takes
  * for T tokens too.) The calls themselves ask for what they take. */
@@ -268,7 +283,7 @@ static size_t router_size(Carve *c, int T, int hidden, int n_experts)
 {
     const size_t start = c->off;
     RtWs w;
-    router_layout(c, &w, T, hidden, n_experts);
+    (void)router_plan(c, &w, (size_t)-1, T, hidden, n_experts, NULL);
     if (T >= 128) {
         const size_t tn = (size_t)T * n_experts, f64 = (size_t)12 * 2048 * (k3k_cu_count() > 0 ? k3k_cu_count() : 1);
         const size_t all = (size_t)((hidden + 255) / 256) * tn, i8 = k3k_router_i8_ws(T, hidden, n_experts);
@@ -311,7 +326,7 @@ static int router_run(int *idx, float *wt, const float *x, int T, const float *W
                                   exc, stream)) {
         return fail("router_partial");
     }
-    if (k3k_router_final(idx, wt, w->nrecomp, w->part, w->rbound, w->chunk, x, W, bias, T, hidden,
+    if (k3k_router_final(idx, wt, w->nrecomp, w->ctr + 1, w->part, w->rbound, w->chunk, x, W, bias, T, hidden,
                          n_experts, topk, renorm, routed_scale, exc, gather ? &g : NULL, stream))
         return fail("router_final");
     return 0;
@@ -322,7 +337,7 @@ int k3d_router_recomputed(int *h_counts, const void *ws, int T, int hidden, int 
     if (T <= 0) return 0;
     Carve c = {(char *)ws, 0};
     RtWs w;
-    router_layout(&c, &w, T, hidden, n_experts);
+    router_layout(&c, &w, T, hidden, n_experts, hidden, 0);    /* (where the counts are depends on T alone) */
     if (k3k_d2h(h_counts, w.nrecomp, (size_t)T * 4, NULL) || k3k_sync(NULL)) return fail("router_recomputed");
     return 0;
 }
@@ -333,7 +348,12 @@ int k3d_router_partials(double *h_part, float *h_rbound, int *h_chunk, size_t ca
     if (T <= 4 || k3k_router_small(T, hidden)) return bad("k3d_router_partials: a few tokens are scored whole");
     Carve c = {(char *)ws, 0};
     RtWs w;
-    router_layout(&c, &w, T, hidden, n_experts);
+    int chunk = 0;
+    router_layout(&c, &w, T, hidden, n_experts, hidden, 0);
+    if (k3k_d2h(&chunk, w.ctr + 1, 4, NULL) || k3k_sync(NULL)) return fail("router_partials");
+    if (chunk <= 0) return bad("k3d_router_partials: no router call has used the workspace");
+    c.off = 0;
+    router_layout(&c, &w, T, hidden, n_experts, chunk, 0);
     const int ks = (hidden + w.chunk - 1) / w.chunk;
     const size_t n = (size_t)ks * T * n_experts;
     if (n > cap) return bad("k3d_router_partials: cap");
@@ -352,7 +372,7 @@ int k3d_router(int *idx, float *wt, const float *x, int T, const float *W, const
     if (n_experts < 1 || n_experts > 2048) return bad("k3d_router: n_experts outside 1..2048");
     Carve c = {(char *)ws, 0};
     RtWs w;
-    if (ws_bytes < router_layout(&c, &w, T, hidden, n_experts)) return bad("k3d_router: workspace too small");
+    if (!router_plan(&c, &w, ws_bytes, T, hidden, n_experts, NULL)) return bad("k3d_router: workspace too small");
     return router_run(idx, wt, x, T, W, bias, hidden, n_experts, topk, renorm, routed_scale, &w, NULL,
                       stream);
 }
@@ -435,12 +455,13 @@ static size_t moe_layout(Carve *c, MoeWs *w, int T, int hidden, int inter, int n
 {
     const size_t N = (size_t)T * topk;
     const int maxjobs = (int)(N < (size_t)n_experts ? N : (size_t)n_experts);
-    /* first list: one pass per expert beside a second list, else up to N / pass_tok full ones more */
-    const int pt[2] = {moe_pass_tok(T, hidden, inter, n_experts, topk, prec, K3D_LAYOUT_ROWS),
-                       moe_pass_tok(T, hidden, inter, n_experts, topk, prec, K3D_LAYOUT_TILED)};
+    /* first list: one pass per expert beside a second list, else up to N / pass_tok full ones more;
+     * for whichever layout has more */
     w->max_passes = maxjobs;
-    if (!moe_two_lists(T, hidden, inter, n_experts, topk, prec, K3D_LAYOUT_ROWS))
-        w->max_passes += (int)(N / (size_t)(pt[0] < pt[1] ? pt[0] : pt[1])) + 1;
+    for (int lay = K3D_LAYOUT_ROWS; lay <= K3D_LAYOUT_TILED; lay++) {
+        const int pt = moe_pass_tok(T, hidden, inter, n_experts, topk, prec, lay), mp = maxjobs + (int)(N / (size_t)pt) + 1;
+        if (!moe_two_lists(T, hidden, inter, n_experts, topk, prec, lay) && mp > w->max_passes) w->max_passes = mp;
+    }
     w->xhi = (uint16_t *)take(c, (size_t)T * hidden * 2);
     w->xlo = prec == 0 ? (uint16_t *)take(c, (size_t)T * hidden * 2) : NULL;
     w->ahi = (uint16_t *)take(c, N * inter * 2);
@@ -450,14 +471,16 @@ static size_t moe_layout(Carve *c, MoeWs *w, int T, int hidden, int inter, int n
     w->job_expert = (int *)take(c, (size_t)maxjobs * 4);
     w->job_off = (int *)take(c, (size_t)maxjobs * 4);
     w->job_cnt = (int *)take(c, (size_t)maxjobs * 4);
-    w->pass_job = (int *)take(c, (size_t)w->max_passes * 4);
-    w->pass_tp = (int *)take(c, (size_t)w->max_passes * 4);
     /* second list: experts of more than 8 assignments, each pass of up to 96 (48, 32) tokens -- at
-     * most N / that full passes plus one per such expert */
+     * most N / 9 of them (9 assignments a pass at the least), behind the first list, which then has at
+     * most one pass per expert, in its arrays */
     const int pt2 = moe_pass_tok2(T, hidden, inter, n_experts, topk, prec, K3D_LAYOUT_TILED);
-    w->max_passes2 = pt2 ? (int)(N / (size_t)pt2 + N / 9 + 2) : 0;
-    w->pass_job2 = pt2 ? (int *)take(c, (size_t)w->max_passes2 * 4) : NULL;
-    w->pass_tp2 = pt2 ? (int *)take(c, (size_t)w->max_passes2 * 4) : NULL;
+    w->max_passes2 = pt2 ? (int)(N / 9 + 1) : 0;
+    const size_t np = (size_t)(maxjobs + w->max_passes2 > w->max_passes ? maxjobs + w->max_passes2 : w->max_passes);
+    w->pass_job = (int *)take(c, np * 4);
+    w->pass_tp = (int *)take(c, np * 4);
+    w->pass_job2 = pt2 ? w->pass_job + maxjobs : NULL;
+    w->pass_tp2 = pt2 ? w->pass_tp + maxjobs : NULL;
     w->counts = (int *)take(c, (size_t)(4 + K3K_QUEUE_INTS) * 4);
     {
         const size_t gs = k3k_gather_scratch(T, topk, n_experts);
@@ -475,6 +498,15 @@ size_t k3d_moe_ws(int T, int hidden, int inter, int n_experts, int topk, int pre
     MoeWs w;
     moe_layout(&c, &w, T, hidden, inter, n_experts, topk, prec);
     return router_size(&c, T, hidden, n_experts);
+}
+
+int k3dx_moe_fits(size_t bytes, int T, int hidden, int inter, int n_experts, int topk, int prec, size_t *need)
+{
+    Carve c = {NULL, 0};
+    MoeWs w;
+    RtWs r;
+    moe_layout(&c, &w, T, hidden, inter, n_experts, topk, prec);
+    return router_plan(&c, &r, bytes, T, hidden, n_experts, need);
 }
 
 static int moe_check(const char *fn, int hidden, int inter, int n_experts, int topk, int layout)
@@ -683,7 +715,7 @@ int k3d_moe_experts(float *out, const int *idx, const float *wt, const float *x,
     MoeWs w;
     RtWs r;
     moe_layout(&c, &w, T, hidden, inter, n_experts, topk, prec);
-    if (ws_bytes < router_layout(&c, &r, T, hidden, n_experts)) return bad("k3d_moe_experts: workspace too small");
+    if (!router_plan(&c, &r, ws_bytes, T, hidden, n_experts, NULL)) return bad("k3d_moe_experts: workspace too small");
     k3k_prof_mark(stream, K3D_STAGE_BEGIN);
     return moe_experts_ws(out, idx, wt, x, T, bank, layout, hidden, inter, n_experts, topk, act,
                           b1, b2, prec, &w, perm_out, offsets_out, drops_out, NULL, 0, 0, stream);
@@ -702,7 +734,7 @@ int k3d_moe_routed(float *out, int *idx, float *wt, const float *x, int T, const
     MoeWs w;
     RtWs r;
     moe_layout(&c, &w, T, hidden, inter, n_experts, topk, prec);
-    if (ws_bytes < router_layout(&c, &r, T, hidden, n_experts)) return bad("k3d_moe_routed: workspace too small");
+    if (!router_plan(&c, &r, ws_bytes, T, hidden, n_experts, NULL)) return bad("k3d_moe_routed: workspace too small");
     k3k_prof_mark(stream, K3D_STAGE_BEGIN);
     if (moe_decode_ok(T, hidden, inter, topk, x) && k3k_router_small(T, hidden) && n_experts <= 512 &&
         !perm_out && !offsets_out) {

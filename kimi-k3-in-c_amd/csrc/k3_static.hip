@@ -59,8 +59,8 @@ extern "C" int k3d_moe_routed_static(float *out, int *idx, float *wt, const floa
                                      void *stream)
 {
     if (T <= 0) return 0;
-    const size_t need = k3d_moe_ws(T, hidden, inter, n_experts, topk, prec);
-    if (need > K3D_STATIC_WS_BYTES) {
+    size_t need = 0;          /* (k3d_moe_ws would be for any smaller batch too) */
+    if (!k3dx_moe_fits(K3D_STATIC_WS_BYTES, T, hidden, inter, n_experts, topk, prec, &need)) {
         char msg[200];
         snprintf(msg, sizeof msg,
                  "k3d_moe_routed_static: this layer needs %zu bytes of scratch, the static "

@@ -230,7 +230,7 @@ int k3k_gemv_q8(float *y, const float *x, const void *W, int in, int out, int nt
  * (the reference's sequential fp64 chain recomputed where the bound cannot decide the
  * fp32 rounding and the logit matters), sigmoid with the host libm's expf, biased
  * first-strict-max top-k, renorm, scale -> idx/wt [T][topk]; nrecomp [T] (may be NULL)
- * receives the number of recomputed logits per token. */
+ * receives the number of recomputed logits per token, *used (may be NULL) the chunk width. */
 /* load (may be NULL): the columns of the busiest CU's workgroups */
 int k3k_router_chunk(int T, int hidden, int n_experts, long *load);
 /* 1 when k3k_router_partial scores and certifies the logits itself (a few tokens): its
@@ -266,7 +266,7 @@ int k3k_router_partial_i8(double *part, float *rbound, void *scratch, const floa
                           const float *W, int hidden, int n_experts, int chunk, int *ctr, int *idx,
                           int n_idx, void *stream);
 /* gather (may be NULL): also run the gather of idx, as k3k_gather would. */
-int k3k_router_final(int *idx, float *wt, int *nrecomp, const double *part, const float *rbound,
+int k3k_router_final(int *idx, float *wt, int *nrecomp, int *used, const double *part, const float *rbound,
                      int chunk, const float *x, const float *W, const float *bias, int T,
                      int hidden, int n_experts, int topk, int renorm, float routed_scale,
                      const K3kExc *exc, const K3kGatherArgs *gather, void *stream);
@@ -335,6 +335,8 @@ int k3k_scale(float *out, const float *in, float s, size_t n, void *stream);
 int k3s_static_setup(void);
 /* Error text for a k3d_* entry point implemented outside k3_devapi.c; returns -2. */
 int k3dx_bad(const char *msg);
+/* whether `bytes` hold the scratch of one routed layer call; *need: the least that does */
+int k3dx_moe_fits(size_t bytes, int T, int hidden, int inter, int n_experts, int topk, int prec, size_t *need);
 
 #ifdef __cplusplus
 }
