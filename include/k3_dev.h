@@ -7,7 +7,8 @@
  * already resident in HBM (a serving loop, the benchmark): every pointer is a DEVICE
  * pointer, work is enqueued on the caller's HIP stream (NULL = the null stream) and the
  * call returns without synchronising. None of them allocates: scratch comes from a
- * caller-provided workspace of the size the matching *_ws() function reports. They
+ * caller-provided workspace of the size the matching *_ws() function reports, which also
+ * serves any smaller batch of the same widths. They
  * return 0, or a negative value with a message available from k3d_error() (kept per host
  * thread).
  *

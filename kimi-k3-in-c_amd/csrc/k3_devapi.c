@@ -275,24 +275,30 @@ static int router_plan(Carve *c, RtWs *w, size_t ws_bytes, int T, int hidden, in
     return 0;
 }
 
-/* What the router takes for any batch of up to T tokens: scratch sized for T tokens serves
- * fewer, which may take the other partials, or more chunks. (The fp64 kernel's chunks: at most 12
- * workgroups of 2048 logits per CU, and 28 of 256 columns of 7168; what it takes past that it takes
- * for T tokens too.) The calls themselves ask for what they take. */
+/* What the router takes for any batch of up to T tokens, with either partials: scratch sized for T
+ * tokens serves fewer, which may take the other ones, or more chunks. Between the token counts gone
+ * over here what a call takes only grows with them: the fp64 kernels' chunks depend on the tokens'
+ * 32s (and on there being up to 4) and are one past six tiles per CU, the int8 kernels' on their 64s
+ * and are one past k3k_router_i8_most's first limit, up to its second, past which they serve none. */
 static size_t router_size(Carve *c, int T, int hidden, int n_experts)
 {
-    const size_t start = c->off;
-    RtWs w;
-    (void)router_plan(c, &w, (size_t)-1, T, hidden, n_experts, NULL);
-    if (T >= 128) {
-        const size_t tn = (size_t)T * n_experts, f64 = (size_t)12 * 2048 * (k3k_cu_count() > 0 ? k3k_cu_count() : 1);
-        const size_t all = (size_t)((hidden + 255) / 256) * tn, i8 = k3k_router_i8_ws(T, hidden, n_experts);
-        size_t any = (all < f64 ? all : f64) * 12;
-        if (any < i8) any = i8;
-        any += (size_t)T * 4 + 5 * 256;        /* nrecomp, ctr, the parts' rounding */
-        if (c->off - start < any) c->off = start + any;
+    const Carve start = *c;
+    const long cus = k3k_cu_count() > 0 ? k3k_cu_count() : 1, nee = (n_experts + 63) / 64;
+    int i8, top = k3k_router_i8_most(hidden, &i8);
+    if (top < 32 * (6 * cus / nee + 2)) top = (int)(32 * (6 * cus / nee + 2));
+    size_t most = start.off;
+    for (int t = T; t > 0; t = t > i8 && i8 > top ? i8 : t > top ? top : t > 32 ? (t - 1) / 32 * 32 : t > 4 ? 4 : 0) {
+        const int chunk[2] = {k3k_router_i8_chunk(t, hidden, n_experts), k3k_router_chunk(t, hidden, n_experts, NULL)};
+        for (int i = 0; i < 2; i++) {
+            RtWs w;
+            if (!chunk[i]) continue;
+            *c = start;
+            router_layout(c, &w, t, hidden, n_experts, chunk[i], i == 0);
+            if (c->off > most) most = c->off;
+        }
     }
-    return c->off;
+    c->off = most;
+    return most;
 }
 
 size_t k3d_router_ws(int T, int hidden, int n_experts)
@@ -496,7 +502,11 @@ size_t k3d_moe_ws(int T, int hidden, int inter, int n_experts, int topk, int pre
 {
     Carve c = {NULL, 0};
     MoeWs w;
+    const size_t N = (size_t)T * topk;
     moe_layout(&c, &w, T, hidden, inter, n_experts, topk, prec);
+    /* room for fewer tokens as well: of what moe_layout takes, only the pass lists (at most N / 8 + 1
+     * passes beyond one per expert) and the decode path's sums can be more with fewer */
+    c.off += 2 * 4 * (N / 8 + 1) + (N > 16 ? (size_t)16 * 2 * inter * 4 : 0) + 4 * 256;
     return router_size(&c, T, hidden, n_experts);
 }
 

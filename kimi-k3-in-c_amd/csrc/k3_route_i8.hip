@@ -459,7 +459,8 @@ static int ri_round(int v, int m) { return (v + m - 1) / m * m; }
 extern "C" int k3k_router_i8_chunk(int T, int hidden, int n_experts)
 {
     if (T < RI_MIN_T || hidden <= 0 || hidden % RI_STEP || n_experts <= 0) return 0;
-    /* (everything below depends on the token tiles only, so that k3k_router_i8_ws can go over them) */
+    /* (below 1024 tokens and from there on, what follows depends on the token tiles only: workspace
+     * sizes go over those) */
     const int Tp = ri_round(T, RI_TT);
     const long ntt = Tp / RI_TT, nte = ri_round(n_experts, RI_TE) / RI_TE;
     const long cus = k3k_cu_count() >= K3_NXCD ? k3k_cu_count() / K3_NXCD : 1;     /* per XCD */
@@ -514,21 +515,12 @@ extern "C" size_t k3k_router_i8_bytes(int T, int hidden, int n_experts, int chun
            ri_al(Ep * ks * sizeof(RiRow));
 }
 
-/* What the partials and the digits of any batch of up to T tokens take: a smaller batch may run on
- * the int8 kernels, or with more chunks, where T tokens do not. */
-extern "C" size_t k3k_router_i8_ws(int T, int hidden, int n_experts)
+/* Past the returned token count the chunks are the same for all, up to *last tokens; none are
+ * served past those. */
+extern "C" int k3k_router_i8_most(int hidden, int *last)
 {
-    size_t most = 0;
-    const int top = ri_round(T, RI_TT) / RI_TT;
-    for (int tt = RI_MIN_T / RI_TT; tt <= top && tt <= RI_MAXTT; tt++) {
-        const int t = tt * RI_TT < T ? tt * RI_TT : T;
-        const int chunk = k3k_router_i8_chunk(t, hidden, n_experts);
-        if (!chunk) continue;
-        const size_t ks = (size_t)(hidden / chunk), p = ks < 2 ? 2 : ks;
-        const size_t n = ri_al(p * t * n_experts * 8) + ri_al(ks * t * n_experts * 4) + k3k_router_i8_bytes(t, hidden, n_experts, chunk);
-        if (n > most) most = n;
-    }
-    return most;
+    *last = hidden > 0 ? (int)((((size_t)1 << 31) - 1) / ((size_t)hidden * RI_ND) / RI_TT * RI_TT) : 0;
+    return RI_MAXTT * RI_TT;
 }
 
 extern "C" int k3k_router_partial_i8(double *part, float *rbound, void *scratch, const float *x, int T,

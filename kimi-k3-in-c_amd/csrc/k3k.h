@@ -260,7 +260,7 @@ int k3k_router_partial(double *part, float *rbound, const float *x, int T, const
  * k3k_router_chunk's chunk); the scratch they need; the partials (x and W 16-byte aligned,
  * chunk from k3k_router_i8_chunk). */
 int k3k_router_i8_chunk(int T, int hidden, int n_experts);
-size_t k3k_router_i8_ws(int T, int hidden, int n_experts);
+int k3k_router_i8_most(int hidden, int *last);
 size_t k3k_router_i8_bytes(int T, int hidden, int n_experts, int chunk);
 int k3k_router_partial_i8(double *part, float *rbound, void *scratch, const float *x, int T,
                           const float *W, int hidden, int n_experts, int chunk, int *ctr, int *idx,

@@ -28,9 +28,9 @@ def sizes(tmp_path_factory):
                     "-L/opt/rocm/lib", "-Wl,-rpath,/opt/rocm/lib", "-lamdhip64", "-lstdc++", "-lgomp", "-lpthread", "-lm"],
                    check=True)
 
-    def ask(shapes):
+    def ask(shapes, step=1):
         text = "".join("%d %d %d %d %d %d\n" % s for s in shapes)
-        out = subprocess.run([exe, "256"], input=text, capture_output=True, text=True, check=True).stdout
+        out = subprocess.run([exe, "256", str(step)], input=text, capture_output=True, text=True, check=True).stdout
         rows = [tuple(map(int, ln.split())) for ln in out.splitlines()]
         assert len(rows) == len(shapes)
         return rows
@@ -57,7 +57,7 @@ def plain_need(T, hidden, inter, n, k, prec, router):
                                    (285, 4096, 3584, 512, 2, 1)])
 def test_static_workspace_holds(sizes, shape):
     (least, takes, ws, *_), = sizes([shape])
-    assert least <= 40 * MIB < ws and least <= takes
+    assert least <= 40 * MIB and least <= takes <= ws
 
 
 def test_least_scratch(sizes):
@@ -73,3 +73,20 @@ def test_least_scratch(sizes):
         hist = al((N + 511) // 512 * n * 4) if N > 2048 and n <= 1024 else 0
         assert least <= takes <= ws and rleast <= rtakes <= rws, s
         assert least <= plain_need(*s, rleast) + al((4 + 4 * 8) * 4) + hist, s
+
+
+def test_size_covers_smaller_batches(sizes):
+    """k3d_moe_ws and k3d_router_ws of T tokens are enough for any batch of up to T, whichever
+    partials and pass lists it takes."""
+    rng = random.Random(11)
+    shapes = [(127, 7168, 512, 384, 8, 0), (7, 7168, 512, 384, 8, 0), (255, 7168, 512, 128, 8, 0), (548, 7168, 512, 64, 8, 0)]
+    shapes += [(rng.randint(1, 1500), 512 * rng.randint(1, 16), 512 * rng.randint(1, 8), rng.choice((3, 60, 64, 128, 384, 896, 1400)),
+                rng.choice((1, 2, 4, 8, 16)), rng.randint(0, 1)) for _ in range(120)]
+    shapes += [(rng.randint(1, 1500), 32 * rng.randint(1, 256), 32 * rng.randint(1, 128), rng.randint(1, 2048),
+                rng.randint(1, 24), rng.randint(0, 1)) for _ in range(120)]
+    for s, (_, _, ws, _, _, rws, most, rmost) in zip(shapes, sizes(shapes)):
+        assert rmost <= rws and most <= ws, s
+    # long prompts, past the last change of a chunk count (49,932 tokens: the int8 kernels' last)
+    shapes = [(t, h, 512, n, 2, 1) for t in (20000, 60000) for h in (512, 7168) for n in (40, 64, 896)]
+    for s, (_, _, ws, _, _, rws, most, rmost) in zip(shapes, sizes(shapes, 32)):
+        assert rmost <= rws and most <= ws, s
