@@ -259,17 +259,24 @@ static void router_layout(Carve *c, RtWs *w, int T, int hidden, int n_experts, i
 }
 
 /* The router's part of a workspace that ends at ws_bytes: the int8 partials where they serve the
- * batch and fit, else the fp64 ones (idx and weights are the same bits). 0 if neither fits; *need
- * (may be NULL): the smaller of the two. */
-static int router_plan(Carve *c, RtWs *w, size_t ws_bytes, int T, int hidden, int n_experts, size_t *need)
+ * batch (`rows16`: 16-byte aligned x and W) and fit, else the fp64 ones with their own chunks (idx
+ * and weights are the same bits); rows that are not aligned take the int8 partials' chunks where
+ * only those fit (608 tokens of 512 experts: 1792 columns a chunk, up to 7168 on the busiest CU,
+ * where its own chunks leave 4320). 0 if nothing fits; *need (may be NULL): the least that does. */
+static int router_plan(Carve *c, RtWs *w, size_t ws_bytes, int rows16, int T, int hidden, int n_experts, size_t *need)
 {
-    const int chunk[2] = {k3k_router_i8_chunk(T, hidden, n_experts), k3k_router_chunk(T, hidden, n_experts, NULL)};
+    const int c8 = k3k_router_i8_chunk(T, hidden, n_experts), c64 = k3k_router_chunk(T, hidden, n_experts, NULL);
+    const struct {
+        int chunk, i8;
+    } way[3] = {{rows16 ? c8 : 0, 1}, {c64, 0}, {rows16 ? 0 : c8, 0}};
     const Carve start = *c;
-    for (int i = 0; i < 2; i++) {
-        if (!chunk[i]) continue;
+    int first = 1;
+    for (int i = 0; i < 3; i++) {
+        if (!way[i].chunk) continue;
         *c = start;
-        router_layout(c, w, T, hidden, n_experts, chunk[i], i == 0);
-        if (need && (i == 0 || !chunk[0] || c->off < *need)) *need = c->off;
+        router_layout(c, w, T, hidden, n_experts, way[i].chunk, way[i].i8);
+        if (need && (first || c->off < *need)) *need = c->off;
+        first = 0;
         if (c->off <= ws_bytes) return 1;
     }
     return 0;
@@ -307,6 +314,8 @@ size_t k3d_router_ws(int T, int hidden, int n_experts)
     return router_size(&c, T, hidden, n_experts);
 }
 
+static int rows_aligned(const void *x, const void *W) { return (((uintptr_t)x | (uintptr_t)W) & 15) == 0; }
+
 /* gather (may be NULL): the router's final kernel also runs the expert-major gather */
 static int router_run(int *idx, float *wt, const float *x, int T, const float *W,
                       const float *bias, int hidden, int n_experts, int topk, int renorm,
@@ -320,9 +329,7 @@ static int router_run(int *idx, float *wt, const float *x, int T, const float *W
         g = *gather;
         g.ctr = w->ctr;
     }
-    /* the int8 partials where they apply (16-byte aligned rows), else the fp64 ones with the
-     * same chunks */
-    if (w->i8 && !((((uintptr_t)x) | ((uintptr_t)W)) % 16)) {
+    if (w->i8) {
         if (k3k_router_partial_i8(w->part, w->rbound, w->i8, x, T, W, hidden, n_experts, w->chunk,
                                   gather ? w->ctr : NULL, gather ? idx : NULL, gather ? T * topk : 0,
                                   stream))
@@ -378,7 +385,7 @@ int k3d_router(int *idx, float *wt, const float *x, int T, const float *W, const
     if (n_experts < 1 || n_experts > 2048) return bad("k3d_router: n_experts outside 1..2048");
     Carve c = {(char *)ws, 0};
     RtWs w;
-    if (!router_plan(&c, &w, ws_bytes, T, hidden, n_experts, NULL)) return bad("k3d_router: workspace too small");
+    if (!router_plan(&c, &w, ws_bytes, rows_aligned(x, W), T, hidden, n_experts, NULL)) return bad("k3d_router: workspace too small");
     return router_run(idx, wt, x, T, W, bias, hidden, n_experts, topk, renorm, routed_scale, &w, NULL,
                       stream);
 }
@@ -516,7 +523,7 @@ int k3dx_moe_fits(size_t bytes, int T, int hidden, int inter, int n_experts, int
     MoeWs w;
     RtWs r;
     moe_layout(&c, &w, T, hidden, inter, n_experts, topk, prec);
-    return router_plan(&c, &r, bytes, T, hidden, n_experts, need);
+    return router_plan(&c, &r, bytes, 1, T, hidden, n_experts, need);
 }
 
 static int moe_check(const char *fn, int hidden, int inter, int n_experts, int topk, int layout)
@@ -725,7 +732,7 @@ int k3d_moe_experts(float *out, const int *idx, const float *wt, const float *x,
     MoeWs w;
     RtWs r;
     moe_layout(&c, &w, T, hidden, inter, n_experts, topk, prec);
-    if (!router_plan(&c, &r, ws_bytes, T, hidden, n_experts, NULL)) return bad("k3d_moe_experts: workspace too small");
+    if (!router_plan(&c, &r, ws_bytes, 1, T, hidden, n_experts, NULL)) return bad("k3d_moe_experts: workspace too small");
     k3k_prof_mark(stream, K3D_STAGE_BEGIN);
     return moe_experts_ws(out, idx, wt, x, T, bank, layout, hidden, inter, n_experts, topk, act,
                           b1, b2, prec, &w, perm_out, offsets_out, drops_out, NULL, 0, 0, stream);
@@ -744,7 +751,7 @@ int k3d_moe_routed(float *out, int *idx, float *wt, const float *x, int T, const
     MoeWs w;
     RtWs r;
     moe_layout(&c, &w, T, hidden, inter, n_experts, topk, prec);
-    if (!router_plan(&c, &r, ws_bytes, T, hidden, n_experts, NULL)) return bad("k3d_moe_routed: workspace too small");
+    if (!router_plan(&c, &r, ws_bytes, rows_aligned(x, router_w), T, hidden, n_experts, NULL)) return bad("k3d_moe_routed: workspace too small");
     k3k_prof_mark(stream, K3D_STAGE_BEGIN);
     if (moe_decode_ok(T, hidden, inter, topk, x) && k3k_router_small(T, hidden) && n_experts <= 512 &&
         !perm_out && !offsets_out) {

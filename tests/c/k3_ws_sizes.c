@@ -18,15 +18,14 @@ int __wrap_k3k_cu_count(void);
 int __wrap_k3k_cu_count(void) { return g_cus; }
 
 /* the bytes of a call with room for all it would take: its layer part before the router's (moe), and
- * the fp64 partials where `f64` */
+ * the fp64 partials where `f64` (rows that are not aligned) */
 static size_t takes(int T, int hidden, int inter, int n, int k, int prec, int moe, int f64)
 {
     Carve c = {NULL, 0};
     MoeWs w;
     RtWs r;
     if (moe) moe_layout(&c, &w, T, hidden, inter, n, k, prec);
-    if (f64) router_layout(&c, &r, T, hidden, n, k3k_router_chunk(T, hidden, n, NULL), 0);
-    else (void)router_plan(&c, &r, (size_t)-1, T, hidden, n, NULL);
+    (void)router_plan(&c, &r, (size_t)-1, !f64, T, hidden, n, NULL);
     return c.off;
 }
 
@@ -41,7 +40,7 @@ int main(int argc, char **argv)
         Carve c = {NULL, 0};
         RtWs r;
         (void)k3dx_moe_fits(0, T, h, i, n, k, prec, &least[1]);
-        (void)router_plan(&c, &r, 0, T, h, n, &least[0]);
+        (void)router_plan(&c, &r, 0, 1, T, h, n, &least[0]);
         for (int t = 1; t <= T; t = t + step < T || t == T ? t + step : T)
             for (int v = 0; v < 4; v++) {
                 const size_t m = takes(t, h, i, n, k, prec, v & 1, v >> 1);

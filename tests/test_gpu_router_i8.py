@@ -135,3 +135,46 @@ def test_router_i8_biased_top16(gpu, orc):
         i2, w2 = orc.router(X[t], W, bias, 16, 1, 2.827)
         assert np.array_equal(idx[t], i2), t
         assert np.array_equal(bits(wt[t]), bits(w2)), t
+
+
+@pytest.mark.parametrize("off_x,off_w", [(4, 0), (0, 4), (8, 12)])
+@pytest.mark.parametrize("T,N,K", [(608, 512, 8), (300, 896, 16), (1030, 384, 8)])
+def test_router_unaligned_rows(gpu, k3, T, N, K, off_x, off_w):
+    """x or W off 16 bytes at token counts that take the int8 partials when aligned: the fp64
+    partials, with their own chunks and not the int8 ones' (at 608 tokens of 512 experts, 1792
+    columns, those left the busiest CU four of them, 7168 columns), to the same bits."""
+    say(f"case: router of unaligned rows T={T} N={N} x+{off_x} W+{off_w}")
+    X = k3.gen_normal(T * HID, 31 + T).reshape(T, HID)
+    W = k3.gen_normal(N * HID, 32 + N).reshape(N, HID) * np.float32(0.02)
+    want = gpu.router_device(X, W, None, K, partials=True)
+    c8 = gpu.router_device.partials[2]
+    L = gpu.lib()
+    wsb = L.k3d_router_ws(T, HID, N)
+    cap = ((HID + 63) // 64) * T * N
+    part, rb, ch = np.empty(cap, np.float64), np.empty(cap, np.float32), np.zeros(1, np.int32)
+    idx, wt = np.empty((T, K), np.int32), np.empty((T, K), np.float32)
+    bufs = [gpu.DevBuf(n) for n in (X.nbytes + 16, W.nbytes + 16, idx.nbytes, wt.nbytes, wsb)]
+    try:
+        dx, dw, di, dwt, ws = bufs
+        dx.upload(X, off_x)
+        dw.upload(W, off_w)
+        gpu.check(L.k3d_router(di.ptr, dwt.ptr, dx.ptr + off_x, T, dw.ptr + off_w, None, HID, N, K, 1, 1.0, ws.ptr, wsb, None), "router")
+        gpu.check(L.k3d_sync(None))
+        di.download(idx)
+        dwt.download(wt)
+        ks = L.k3d_router_partials(part.ctypes.data, rb.ctypes.data, ch.ctypes.data, cap, ws.ptr, T, HID, N)
+    finally:
+        for b in bufs:
+            b.free()
+    assert np.array_equal(idx, want[0]) and np.array_equal(bits(wt), bits(want[1]))
+    chunk = int(ch[0])
+    assert ks == -(-HID // chunk)
+    n = ks * T * N
+    check_contract(part[:n].reshape(ks, T, N), rb[:n].reshape(ks, T, N), chunk, W, X, [0, T - 1])
+
+    def columns(c):                 # of the busiest of 256 CUs: tiles of 32 tokens x 64 experts, a chunk each
+        return -(-(-(-T // 32) * -(-N // 64) * -(-HID // c)) // 256) * c
+    say(f"  chunk {chunk} (int8 {c8}), busiest CU {columns(chunk)} columns ({columns(c8)})")
+    assert columns(chunk) <= columns(c8)
+    if (T, N) == (608, 512):
+        assert c8 % 256 == 0 and columns(chunk) < columns(c8)
