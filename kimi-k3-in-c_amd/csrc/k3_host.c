@@ -672,13 +672,13 @@ static size_t wbytes(int wdt, int in, int out)
 }
 
 /* Whether a bf16 product of ntok tokens has 128 x 64 tiles for three fifths of the CUs, so that
- * the matrix-core GEMM (k3_gemm.hip, two activation terms) is the faster one. Below, and for one
- * token, it streams through k3k_gemv_bf16, whose several-token kernel takes the fp32 activations
- * as they are (7168 -> 3584: 37 tokens 21 us against 78 for the split and the GEMM, 256 tokens
+ * the matrix-core GEMM (k3_gemm.hip, two activation terms) is the faster one. Below, and for up to
+ * four tokens, whose products keep the accuracy of fp32 activations at any width, it streams
+ * through k3k_gemv_bf16, whose several-token kernel takes the activations as they are (7168 -> 3584: 37 tokens 21 us against 78 for the split and the GEMM, 256 tokens
  * (112 tiles) 55 against 78, 333 tokens (168) 96 against 78). */
 static int mmw_gemm(int wdt, int ntok, int in, int out)
 {
-    return wdt == K3_WBF16 && in % 64 == 0 &&
+    return wdt == K3_WBF16 && ntok > 4 && in % 64 == 0 &&
            (long)((out + 127) / 128) * ((ntok + 63) / 64) * 5 >= (long)k3k_cu_count() * 3 &&
            (unsigned long long)out * in * 2 < 0x80000000ull && (unsigned long long)ntok * in * 2 < 0x80000000ull;
 }
@@ -689,7 +689,7 @@ static void mmw_on(float *y_d, const float *x_d, int ntok, const void *W, int wd
 {
     const void *dw = weights(slot, W, wbytes(wdt, in, out));
     int rc;
-    if (ntok > 1 && mmw_gemm(wdt, ntok, in, out)) {
+    if (mmw_gemm(wdt, ntok, in, out)) {
         uint16_t *xs = (uint16_t *)buf(xs_slot, (size_t)ntok * in * 4);
         uint16_t *xl = xs + (size_t)ntok * in;
         check(k3k_split_bf16(xs, xl, x_d, (size_t)ntok * in, stream), "activation split");
@@ -883,7 +883,7 @@ static float *shared_on(const float *dx, const K3MoeW *w, const K3Cfg *c, int T,
     const int E = c->hidden, SI = c->moe_inter * c->n_shared;
     float *sdn = (float *)buf(B_SSDN, (size_t)T * E * 4);
     const uint16_t *w1 = (const uint16_t *)k3_dev_lookup(w->sh1), *w3 = (const uint16_t *)k3_dev_lookup(w->sh3);
-    if (T > 1 && w1 && w3 && E % 64 == 0 && SI % 64 == 0 && mmw_gemm(w->wdt, T, E, SI) &&
+    if (w1 && w3 && E % 64 == 0 && SI % 64 == 0 && mmw_gemm(w->wdt, T, E, SI) &&
         mmw_gemm(w->wdt, T, SI, E)) {
         /* many tokens: gate, up and the activation in one GEMM, its result as bf16 terms */
         uint16_t *xs = (uint16_t *)buf(B_SXS, (size_t)T * E * 4), *as = (uint16_t *)buf(B_SACT, (size_t)T * SI * 4);

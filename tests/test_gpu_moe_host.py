@@ -58,3 +58,33 @@ def test_resident_bank_same_as_fetched(gpu, wl, T):
             gpu.dev_unregister(W[a])
         full.destroy()
         part.destroy()
+
+
+def shared_fp64(x, W):
+    """sh2 . situ(sh1 x, sh3 x) of bf16 weights in fp64 (b1 = 4, b2 = 25)."""
+    f = {k: (W[k].astype(np.uint32) << 16).view(np.float32).astype(np.float64) for k in ("sh1", "sh3", "sh2")}
+    g, u = x.astype(np.float64) @ f["sh1"].T, x.astype(np.float64) @ f["sh3"].T
+    return (4.0 * np.tanh(g / 4.0) / (1.0 + np.exp(-g)) * 25.0 * np.tanh(u / 25.0)) @ f["sh2"].T
+
+
+@pytest.mark.parametrize("resident", [False, True])
+@pytest.mark.parametrize("T", [1, 2, 4])
+def test_wide_trunk_few_tokens(gpu, wl, T, resident):
+    """Up to four tokens keep fp32 activations in the trunk products however wide the matrix is
+    (two bf16 terms would show 2.5e-6). Every fetch fails, so the block's output is its shared
+    expert alone, whose gate and up have 20480 rows."""
+    from oracle import PySource
+    say(f"case: wide trunk T={T} resident={resident}")
+    cfg, W, _ = wl.latent_layer(512, 64, 10240, 4, 1, tag="host.wide", n_generated=0)
+    x = wl.tokens(T, 512, tag=f"host.wide.{T}")
+    names = ("gate", "down", "up", "sh1", "sh3", "sh2") if resident else ()
+    src = PySource({})                                   # (held while the library calls it)
+    try:
+        for a in names:
+            gpu.dev_register(W[a])
+        got = gpu.moe(x, cfg, W, 1, src.ptr, 1)
+    finally:
+        for a in names:
+            gpu.dev_unregister(W[a])
+    want = shared_fp64(x, W)
+    assert got[3] >= 1 and np.linalg.norm(got[0] - want) <= 1e-6 * np.linalg.norm(want)
