@@ -57,11 +57,13 @@
 namespace {
 
 constexpr int RI_ND = 6;                 /* digits per operand */
-/* Products of digits i, j with i + j <= RI_LMAX. At 9 what is left out (levels 10 and up, under
- * 2^-23 of the bound R a chunk of 1792 columns has from its prefixes in units of 2^-53) still adds
- * nothing to R; the level 10 sums would: 3 products of 33 for no certified logit more (partials of
- * 4096 tokens x 384 experts 270 -> 257 us; at 8 the bound grows 16 times, and with it the
- * recomputed logits). */
+/* Products of digits i, j with i + j <= RI_LMAX. The level 10 sums, 3 products of 33, change next to
+ * nothing: 1030 tokens x 384 experts, chunks of 3584 columns, the partials' mean error is 2.95 2^-53
+ * without and 2.92 with them, and the bound R the same for N(0, 1) rows (6847 in 2^-53); rows with
+ * three values 30 / 100 / 1000 times the rest have an R of 1.21e4 / 5.19e4 / 2.68e6 without and
+ * 9.2e3 / 3.31e4 / 2.46e6 with them, and neither leaves a logit to recompute (nor at 4096 x 384 and
+ * 2048 x 896). Without, partials of 4096 tokens x 384 experts 270 -> 257 us; at 8 the bound of N(0, 1)
+ * rows grows 16 times, and with it the recomputed logits. */
 constexpr int RI_LMAX = 9;
 constexpr int RI_NL = RI_LMAX - 1;       /* level accumulators, l = 2 .. RI_LMAX */
 constexpr int RI_STEP = 64;              /* columns per step: one int8 matrix instruction */
