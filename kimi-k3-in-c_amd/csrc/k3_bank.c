@@ -48,9 +48,10 @@ struct K3DevBank {
     uint64_t *used_at, clock;
     uint64_t *pin, epoch;       /* pin[s] == epoch while a MoE call holds the slot */
     int in_call;
-    /* device copy of the slots' pointers, [n_layers][n_experts] (NULL pointers: not resident),
-     * made on first use; a layer's part is rewritten when its slots have changed */
-    K3ExpertQ *table;
+    /* the slots' pointers on the device, [n_layers][n_experts] (NULL pointers: not resident), and
+     * the host array they are copied from; a layer's part is rewritten when it is asked for and its
+     * slots have changed */
+    K3ExpertQ *table, *mirror;
     unsigned char *stale;       /* [n_layers] */
     int *nres;                  /* [n_layers] experts resident */
     K3DevBankStats st;
@@ -310,6 +311,9 @@ K3DevBank *k3_devbank_create(int n_layers, int n_experts, int width, int inter, 
         goto fail;
     }
     memset(b->stale, 1, (size_t)n_layers);
+    /* (a bank without a table still serves: its callers send the pointers with each call) */
+    b->mirror = (K3ExpertQ *)calloc(nkey, sizeof(K3ExpertQ));
+    if (b->mirror) b->table = (K3ExpertQ *)k3k_malloc(nkey * sizeof(K3ExpertQ));
     for (size_t k = 0; k < nkey; k++) b->slot_of[k] = -1;
     for (int s = 0; s < slots; s++) b->key_of[s] = -1;
     b->arena = (char *)k3k_malloc((size_t)slots * b->slot_bytes);
@@ -344,6 +348,8 @@ fail:
         free(b->pin);
         free(b->stale);
         free(b->nres);
+        k3k_free(b->table);
+        free(b->mirror);
         free(b);
     }
     b = NULL;
@@ -410,6 +416,7 @@ void k3_devbank_destroy(K3DevBank *b)
     free(b->stale);
     free(b->nres);
     k3k_free(b->table);
+    free(b->mirror);
     free(b);
     k3h_unlock();
 }
@@ -440,29 +447,21 @@ void k3_bank_call(K3ExpertSrc *src, int begin)
     b->in_call = begin;
 }
 
-const void *k3_bank_table(const K3ExpertSrc *src, int layer, int n_experts, int *all)
+const void *k3_bank_table(const K3ExpertSrc *src, int layer, int n_experts, int whole)
 {
-    *all = 0;
     if (!src || src->get != src_get) return NULL;
     K3DevBank *b = (K3DevBank *)src->ctx;
-    if (layer < 0 || layer >= b->n_layers || n_experts != b->n_experts) return NULL;
-    const size_t row = (size_t)n_experts * sizeof(K3ExpertQ);
-    if (!b->table) {
-        b->table = (K3ExpertQ *)k3k_malloc((size_t)b->n_layers * row);
-        if (!b->table) return NULL;
-    }
-    char *dev = (char *)b->table + (size_t)layer * row;
+    if (!b->table || layer < 0 || layer >= b->n_layers || n_experts != b->n_experts) return NULL;
+    if (whole && b->nres[layer] != n_experts) return NULL;
+    const size_t o = (size_t)layer * n_experts;
     if (b->stale[layer]) {
-        K3ExpertQ *h = (K3ExpertQ *)calloc((size_t)n_experts, sizeof(K3ExpertQ));
-        if (!h) return NULL;
-        const int *slot = b->slot_of + (size_t)layer * n_experts;
+        /* (no wait: the part is next rewritten after another admission, which waits for the
+         * stream, and what a call sends is done when it returns) */
+        memset(b->mirror + o, 0, (size_t)n_experts * sizeof(K3ExpertQ));
         for (int e = 0; e < n_experts; e++)
-            if (slot[e] >= 0) fill_q(b, slot[e], &h[e]);
-        const int rc = k3k_h2d(dev, h, row, k3h_stream()) || k3k_sync(k3h_stream());
-        free(h);
-        if (rc) return NULL;
+            if (b->slot_of[o + e] >= 0) fill_q(b, b->slot_of[o + e], &b->mirror[o + e]);
+        if (k3k_h2d(b->table + o, b->mirror + o, (size_t)n_experts * sizeof(K3ExpertQ), k3h_stream())) return NULL;
         b->stale[layer] = 0;
     }
-    *all = b->nres[layer] == n_experts;
-    return dev;
+    return b->table + o;
 }

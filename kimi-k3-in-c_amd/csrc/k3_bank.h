@@ -33,10 +33,11 @@ void k3_bank_call(K3ExpertSrc *src, int begin);
 int k3_bank_full(const K3ExpertSrc *src, int layer, int expert);
 
 /* The device array of a bank's slot pointers of `layer`, [n_experts] K3ExpertQ (NULL pointers:
- * not resident), current as of the call, and in *all whether every expert is resident; it holds
- * until the bank next admits or evicts. NULL for any other source, and for a bank of another
- * expert count. Called under the library's lock. */
-const void *k3_bank_table(const K3ExpertSrc *src, int layer, int n_experts, int *all);
+ * not resident), as of the call, for work on the library's stream; it holds until the bank next
+ * admits or evicts. NULL for any other source, for a bank of another expert count and, with
+ * `whole`, while an expert of the layer is not resident (nothing is sent then). Called under the
+ * library's lock. */
+const void *k3_bank_table(const K3ExpertSrc *src, int layer, int n_experts, int whole);
 
 #ifdef __cplusplus
 }

@@ -770,8 +770,7 @@ static void run_fetched(Fetch *f)
         check(k3k_h2d(f->di, f->pidx, TK * 4, g_stream), "host to device copy");
         check(k3k_h2d(f->dwt, f->hwt, TK * 4, g_stream), "host to device copy");
     }
-    int all;
-    const void *table = f->bank_layout >= 0 ? k3_bank_table(f->w->src, f->w->layer, f->N, &all) : NULL;
+    const void *table = f->bank_layout >= 0 ? k3_bank_table(f->w->src, f->w->layer, f->N, 0) : NULL;
     const int layout = f->bank_layout >= 0 ? f->bank_layout : K3D_LAYOUT_ROWS;
     for (int b0 = 0; b0 < T; b0 += MOE_DEV_BLOCK) {
         const int nb = T - b0 < MOE_DEV_BLOCK ? T - b0 : MOE_DEV_BLOCK;
@@ -997,10 +996,10 @@ static void moe_latent(float *out, const float *x, const K3MoeW *w, const K3Cfg 
      * experts run from the bank's own device table on the routing as the router wrote it, and
      * the host follows with the bank's bookkeeping (the same get / getmany calls, all hits)
      * while the block runs, instead of between the two. */
-    int all = 0;
     const void *table = w->src && !w->cache_only && L % 32 == 0 && I % 32 == 0 &&
                                 k3_bank_layout(w->src, L, I) >= 0
-                            ? k3_bank_table(w->src, w->layer, N, &all) : NULL;
+                            ? k3_bank_table(w->src, w->layer, N, 1) : NULL;
+    const int all = table != NULL;
     if (all) {
         for (int b0 = 0; b0 < T; b0 += MOE_DEV_BLOCK) {
             const int nb = T - b0 < MOE_DEV_BLOCK ? T - b0 : MOE_DEV_BLOCK;

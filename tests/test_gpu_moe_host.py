@@ -88,3 +88,36 @@ def test_wide_trunk_few_tokens(gpu, wl, T, resident):
             gpu.dev_unregister(W[a])
     want = shared_fp64(x, W)
     assert got[3] >= 1 and np.linalg.norm(got[0] - want) <= 1e-6 * np.linalg.norm(want)
+
+
+def test_overcommitted_bank_layers(gpu, orc, wl):
+    """Two layers of 24 experts in 36 slots: each layer's calls evict experts of the other, so a
+    layer is whole in one call and not in the next, and the device table is rewritten and left
+    alone by turns. Every call against the oracle."""
+    import ctypes as C
+    from conftest import max_err_rel_inf
+    from oracle import PySource, oracle_moe_q
+    say("case: two layers in an overcommitted bank")
+    cfg, W, ex = wl.latent_layer(1024, 512, 512, 24, 4, n_shared=1, tag="host.over")
+    _, _, other = wl.latent_layer(1024, 512, 512, 24, 4, n_shared=1, tag="host.over2")
+    layers = [ex, other]
+
+    @gpu.GETFN
+    def get(self, layer, e, out):
+        q = out.contents
+        q.p1, q.s1, q.p3, q.s3, q.p2, q.s2 = [a.ctypes.data for a in layers[layer][e].t]
+        return 0
+
+    up = gpu.K3ExpertSrc(get, gpu.GETMANYFN(), gpu.GETFN(), None)
+    bank = gpu.HbmBank(2, 24, 512, 512, 36, upstream_ptr=C.addressof(up))
+    try:
+        for step, (layer, T) in enumerate([(0, 70), (0, 1), (1, 1), (0, 3), (1, 70), (1, 1), (0, 1), (0, 70), (0, 2), (1, 2)]):
+            x = wl.tokens(T, 1024, tag=f"host.over.{step}")
+            got = gpu.moe(x, cfg, W, 1, bank.src, int(T > 1), layer=layer)
+            src = PySource(layers[layer])
+            want = oracle_moe_q(orc, x, cfg, W, 1, src, int(T > 1), layer=layer)
+            assert max_err_rel_inf(got[0], want[0]) <= 1e-4, step
+            assert got[3] == 0 and np.array_equal(got[1], want[1]) and np.array_equal(got[2], want[2], equal_nan=True)
+        assert bank.stats()["evictions"] > 0 and bank.stats()["failures"] == 0
+    finally:
+        bank.destroy()
