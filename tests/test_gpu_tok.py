@@ -71,6 +71,43 @@ def test_tok_matmul_nonfinite(gpu, k3, bf16, inn):
     assert (np.abs(Y - want)[fin] <= (1e-6 * bound + tiny)[fin]).all()
 
 
+@pytest.mark.parametrize("bf16", [True, False])
+@pytest.mark.parametrize("T,inn,out", [(40, 7168, 2048), (64, 4099, 1000)])
+def test_tok_matmul_nan_tokens_cost(gpu, k3, bf16, T, inn, out):
+    """Tokens of NaN (padding) leave the others' results as they are and cost little: their outputs
+    need no recomputing. (One dot product after another by single lanes took over 100 times
+    the clean call.)"""
+    import time
+    say(f"case: NaN tokens {T} tokens {inn} -> {out} bf16={bf16}")
+    Wb = k3.gen_bf16_normal(inn * out, 95, 0.0, 0.02).reshape(out, inn)
+    W = Wb if bf16 else (Wb.astype(np.uint32) << 16).view(np.float32)
+    X = k3.gen_normal(T * inn, 96).reshape(T, inn)
+    Xn = X.copy()
+    Xn[[3, T - 1]] = np.nan
+    L = gpu.lib()
+    fn = L.k3d_matmul_bf16 if bf16 else L.k3d_matmul_f32
+    bufs = [gpu.DevBuf(X.nbytes).upload(X), gpu.DevBuf(X.nbytes).upload(Xn), gpu.DevBuf(W.nbytes).upload(W), gpu.DevBuf(T * out * 4)]
+    res, took = [], []
+    try:
+        for dx in bufs[:2]:
+            best = 1e9
+            for _ in range(5):
+                gpu.check(L.k3d_sync(None))
+                t0 = time.perf_counter()
+                for _ in range(5):
+                    gpu.check(fn(bufs[3].ptr, dx.ptr, T, bufs[2].ptr, inn, out, None), "matmul")
+                gpu.check(L.k3d_sync(None))
+                best = min(best, time.perf_counter() - t0)
+            took.append(best / 5)
+            res.append(bufs[3].download(np.empty((T, out), np.float32)))
+    finally:
+        for b in bufs:
+            b.free()
+    say(f"  {took[0] * 1e6:.1f} us, with two NaN tokens {took[1] * 1e6:.1f}")
+    keep = [t for t in range(T) if t not in (3, T - 1)]
+    assert np.isnan(res[1][[3, T - 1]]).all() and np.array_equal(res[0][keep], res[1][keep])
+    assert took[1] <= 10 * took[0] + 2e-5
+
 @pytest.mark.parametrize("T,inn,rows", [(3, 128, 1), (3, 7168, 2048), (8, 256, 17), (9, 384, 48), (17, 1152, 130), (33, 3584, 4097),
                                         (64, 896, 300), (65, 512, 4100), (130, 2176, 71), (257, 128, 1031),
                                         (3, 32, 5), (19, 224, 100), (40, 1504, 515), (100, 4128, 70)])
