@@ -5,17 +5,20 @@
  * Replaces k3_matmul (src/core/k3_ops.c:265-291), k3_matmul_bf16 (:1108-1213) and
  * k3_matmul_q8 (:1221-1289) of the reference for the decode shapes.
  *
- * gemv_rows_kernel (one token, row length a multiple of 8, 16-byte aligned operands): a wave
- * owns RW rows; lane l takes the 8-element chunks l, l+64, l+128, ... of every row, and issues
- * the loads of U chunks of all RW rows (and the matching x chunks) before any arithmetic, so a
- * lane keeps U*RW 16-byte weight loads in flight and each x chunk it loads serves RW rows. Per lane the products are accumulated in fp32 in ascending column
+ * gemv_rows_kernel (one token; ANY: any row length and alignment): a wave owns RW rows; lane
+ * l takes the 8-element chunks l, l+64, l+128, ... of every row, and issues the loads of U
+ * chunks of all RW rows (and the matching x chunks) before any arithmetic, so a lane keeps
+ * U*RW 16-byte weight loads in flight and each x chunk it loads serves RW rows. Per lane the
+ * products are accumulated in fp32 in ascending column
  * order, then the wave reduces with a butterfly. The fp32 and bf16 kernels are one
  * template, so on weights that are the same values they perform the same operations in
  * the same order and agree bit for bit (the reference holds the same property between its
- * two kernels, tests/unit/test_ops.c:798-848). Accumulation is fp32 where the reference
- * uses fp64; the difference is far inside max|err| <= 1e-4 ||ref||inf. More
- * tokens go to the matrix cores (k3_tok.hip; two tokens of 7168 -> 3584 in bf16: 13.0 us here,
- * 10.3 there). gemv_kernel, one wave per row and token, takes the shapes neither does.
+ * two kernels, tests/unit/test_ops.c:798-848), for one token of any row length. Accumulation
+ * is fp32 where the reference uses fp64; the difference is far inside max|err| <= 1e-4
+ * ||ref||inf. More tokens go to the matrix cores (k3_tok.hip; two tokens of 7168 -> 3584 in
+ * bf16: 13.0 us here, 10.3 there): there the two types are cut and summed differently and agree
+ * within rounding only, and a token's sums depend on how many come with it. gemv_kernel, one wave
+ * per row and token, takes the shapes neither does.
  */
 #include "k3_common.h"
 #include "k3k.h"
@@ -101,21 +104,51 @@ __global__ __launch_bounds__(256) void gemv_q8_kernel(float *y, const float *x, 
 }
 
 
-/* Raw 8-element weight chunk: one 16-byte load (bf16) or two (fp32), non-temporal (weights
- * streamed once per launch). */
+/* Raw 8-element weight chunk: one 16-byte load (bf16) or two (fp32), non-temporal where aligned
+ * (weights streamed once per launch). */
 typedef unsigned int k3u32x4 __attribute__((ext_vector_type(4)));
 typedef float k3f32x4 __attribute__((ext_vector_type(4)));
 
+typedef k3u32x4 k3u32x4_any __attribute__((aligned(2)));
+typedef k3f32x4 k3f32x4_any __attribute__((aligned(4)));
+
+template <bool ANY>
 __device__ __forceinline__ uint4 ld16(const void *p)
 {
-    const k3u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const k3u32x4 *>(p));
+    k3u32x4 v;
+    if constexpr (ANY) v = *reinterpret_cast<const k3u32x4_any *>(p);
+    else v = __builtin_nontemporal_load(reinterpret_cast<const k3u32x4 *>(p));
     return make_uint4(v.x, v.y, v.z, v.w);
+}
+template <bool ANY>
+__device__ __forceinline__ float4 ldx4(const float *p)
+{
+    if constexpr (ANY) {
+        const k3f32x4 v = *reinterpret_cast<const k3f32x4_any *>(p);
+        return make_float4(v.x, v.y, v.z, v.w);
+    } else {
+        return *reinterpret_cast<const float4 *>(p);
+    }
+}
+/* the first n (< 8) elements at p, zeros behind them */
+template <typename T>
+__device__ __forceinline__ void ld_tail(T (&v)[8], const T *p, int n)
+{
+#pragma unroll
+    for (int k = 0; k < 8; k++) v[k] = k < n ? p[k] : T(0);
 }
 
 template <typename WT> struct Chunk8;
 template <> struct Chunk8<uint16_t> {
     uint4 v;
-    __device__ __forceinline__ void load(const uint16_t *p) { v = ld16(p); }
+    template <bool ANY>
+    __device__ __forceinline__ void load(const uint16_t *p) { v = ld16<ANY>(p); }
+    __device__ __forceinline__ void tail(const uint16_t *p, int n)
+    {
+        uint16_t t[8];
+        ld_tail(t, p, n);
+        v = make_uint4(t[0] | (uint32_t)t[1] << 16, t[2] | (uint32_t)t[3] << 16, t[4] | (uint32_t)t[5] << 16, t[6] | (uint32_t)t[7] << 16);
+    }
     __device__ __forceinline__ float at(int k) const
     {
         const uint32_t u = k < 2 ? v.x : k < 4 ? v.y : k < 6 ? v.z : v.w;
@@ -124,9 +157,17 @@ template <> struct Chunk8<uint16_t> {
 };
 template <> struct Chunk8<float> {
     float4 a, b;
+    __device__ __forceinline__ void tail(const float *p, int n)
+    {
+        float t[8];
+        ld_tail(t, p, n);
+        a = make_float4(t[0], t[1], t[2], t[3]);
+        b = make_float4(t[4], t[5], t[6], t[7]);
+    }
+    template <bool ANY>
     __device__ __forceinline__ void load(const float *p)
     {
-        const uint4 u = ld16(p), v = ld16(p + 4);
+        const uint4 u = ld16<ANY>(p), v = ld16<ANY>(p + 4);
         a = make_float4(__uint_as_float(u.x), __uint_as_float(u.y), __uint_as_float(u.z), __uint_as_float(u.w));
         b = make_float4(__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w));
     }
@@ -137,14 +178,14 @@ template <> struct Chunk8<float> {
     }
 };
 
-template <typename WT, int RW, int U>
+template <typename WT, int RW, int U, bool ANY>
 __global__ __launch_bounds__(256) void gemv_rows_kernel(float *__restrict__ y, const float *__restrict__ x,
                                                         const WT *__restrict__ W, int in, int out)
 {
     const int lane = threadIdx.x & 63;
     const int r0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * RW;
     if (r0 >= out) return;
-    const int nch = in >> 3;
+    const int nch = ANY ? (in + 7) >> 3 : in >> 3;
     const WT *row[RW];
 #pragma unroll
     for (int r = 0; r < RW; r++) row[r] = W + (size_t)min(r0 + r, out - 1) * in;
@@ -157,11 +198,18 @@ __global__ __launch_bounds__(256) void gemv_rows_kernel(float *__restrict__ y, c
 #pragma unroll
         for (int u = 0; u < U; u++) {
             const int c = cb + 64 * u;
-            if (c < nch) {
+            if (ANY ? 8 * (c + 1) <= in : c < nch) {
 #pragma unroll
-                for (int r = 0; r < RW; r++) w[u][r].load(row[r] + 8 * (size_t)c);
-                xa[u] = reinterpret_cast<const float4 *>(x + 8 * (size_t)c)[0];
-                xb[u] = reinterpret_cast<const float4 *>(x + 8 * (size_t)c)[1];
+                for (int r = 0; r < RW; r++) w[u][r].template load<ANY>(row[r] + 8 * (size_t)c);
+                xa[u] = ldx4<ANY>(x + 8 * (size_t)c);
+                xb[u] = ldx4<ANY>(x + 8 * (size_t)c + 4);
+            } else if (ANY && c < nch) {           /* the row's last in % 8 */
+                float t[8];
+#pragma unroll
+                for (int r = 0; r < RW; r++) w[u][r].tail(row[r] + 8 * (size_t)c, in - 8 * c);
+                ld_tail(t, x + 8 * (size_t)c, in - 8 * c);
+                xa[u] = make_float4(t[0], t[1], t[2], t[3]);
+                xb[u] = make_float4(t[4], t[5], t[6], t[7]);
             }
         }
 #pragma unroll
@@ -219,7 +267,7 @@ __global__ __launch_bounds__(256) void gemv_glu_kernel(float *__restrict__ y, co
             const int c = cb + 64 * u;
             if (c < nch) {
 #pragma unroll
-                for (int r = 0; r < 2; r++) w[u][r].load(row[r] + 8 * (size_t)c);
+                for (int r = 0; r < 2; r++) w[u][r].template load<false>(row[r] + 8 * (size_t)c);
                 xa[u] = reinterpret_cast<const float4 *>(x + 8 * (size_t)c)[0];
                 xb[u] = reinterpret_cast<const float4 *>(x + 8 * (size_t)c)[1];
             }
@@ -253,11 +301,16 @@ __global__ __launch_bounds__(256) void gemv_glu_kernel(float *__restrict__ y, co
  * cached loads: 5.6 TB/s). */
 constexpr int GV_RW = 2;
 
+/* One token of a row length that is no multiple of 8, or operands that are not 16-byte aligned: the
+ * same loads at the elements they start at, through the caches, since neighbouring lanes share lines
+ * (7169 -> 3584 in bf16 11.0 us, fp32 16.7; non-temporal 13.0 and 24.0; the several-token kernel 15.1
+ * and 20.4; a wave per row, one load after the other, 74.9 and 99.2). */
 template <typename WT>
-void launch_gemv(float *y, const float *x, const WT *W, int in, int out, hipStream_t st)
+void launch_gemv(float *y, const float *x, const WT *W, int in, int out, bool vec, hipStream_t st)
 {
-    hipLaunchKernelGGL((gemv_rows_kernel<WT, GV_RW, 8>), dim3((unsigned)((out + 4 * GV_RW - 1) / (4 * GV_RW))),
-                       dim3(256), 0, st, y, x, W, in, out);
+    const dim3 grid((unsigned)((out + 4 * GV_RW - 1) / (4 * GV_RW)));
+    if (vec) hipLaunchKernelGGL((gemv_rows_kernel<WT, GV_RW, 8, false>), grid, dim3(256), 0, st, y, x, W, in, out);
+    else hipLaunchKernelGGL((gemv_rows_kernel<WT, GV_RW, 8, true>), grid, dim3(256), 0, st, y, x, W, in, out);
 }
 
 bool aligned16(const void *p) { return ((uintptr_t)p & 15u) == 0; }
@@ -268,9 +321,9 @@ extern "C" int k3k_gemv_f32(float *y, const float *x, const float *W, int in, in
                             int ldy, void *stream)
 {
     if (out <= 0 || ntok <= 0) return 0;
-    if (k3k_tok_ok(x, W, in, ntok)) return k3k_tok_gemm(y, x, W, 0, in, out, ntok, ldy, 0, stream);
+    if (k3k_tok_ok(in, ntok)) return k3k_tok_gemm(y, x, W, 0, in, out, ntok, ldy, 0, stream);
     const int vec = (in % 8 == 0) && aligned16(x) && aligned16(W);
-    if (vec && in > 0 && ntok == 1) launch_gemv<float>(y, x, W, in, out, (hipStream_t)stream);
+    if (in > 0 && ntok == 1) launch_gemv<float>(y, x, W, in, out, vec, (hipStream_t)stream);
     else hipLaunchKernelGGL(gemv_kernel<float>, dim3((out + 3) / 4, ntok), dim3(256), 0,
                             (hipStream_t)stream, y, x, W, in, out, vec, ldy);
     K3K_LAUNCH_CHECK("gemv_f32 launch");
@@ -281,9 +334,9 @@ extern "C" int k3k_gemv_bf16(float *y, const float *x, const uint16_t *W, int in
                              int ntok, int ldy, void *stream)
 {
     if (out <= 0 || ntok <= 0) return 0;
-    if (k3k_tok_ok(x, W, in, ntok)) return k3k_tok_gemm(y, x, W, 1, in, out, ntok, ldy, 0, stream);
+    if (k3k_tok_ok(in, ntok)) return k3k_tok_gemm(y, x, W, 1, in, out, ntok, ldy, 0, stream);
     const int vec = (in % 8 == 0) && aligned16(x) && aligned16(W);
-    if (vec && in > 0 && ntok == 1) launch_gemv<uint16_t>(y, x, W, in, out, (hipStream_t)stream);
+    if (in > 0 && ntok == 1) launch_gemv<uint16_t>(y, x, W, in, out, vec, (hipStream_t)stream);
     else hipLaunchKernelGGL(gemv_kernel<uint16_t>, dim3((out + 3) / 4, ntok), dim3(256), 0,
                             (hipStream_t)stream, y, x, W, in, out, vec, ldy);
     K3K_LAUNCH_CHECK("gemv_bf16 launch");

@@ -648,11 +648,11 @@ static int shape_ok(const void *x, const void *W, int in)
     return in >= 8 && in % 8 == 0 && in < (1 << 22) && (((uintptr_t)x | (uintptr_t)W) & 15) == 0;
 }
 
-/* One token of aligned rows stays on the vector units, and so do up to four of short rows: their
- * sums are the more accurate there. */
-extern "C" int k3k_tok_ok(const float *x, const void *W, int in, int ntok)
+/* One token stays on the vector units, where fp32 and bf16 weights of the same values give the same
+ * bits, and so do up to four of short rows, whose sums are the more accurate there. */
+extern "C" int k3k_tok_ok(int in, int ntok)
 {
-    return (ntok > 4 || in >= 512) && in >= 8 && in < (1 << 22) && (ntok > 1 || !shape_ok(x, W, in));
+    return ntok > 1 && (ntok > 4 || in >= 512) && in >= 8 && in < (1 << 22);
 }
 
 extern "C" int k3k_tok_gemm(float *y, const float *x, const void *W, int bf16, int in, int out, int ntok, int ldy,

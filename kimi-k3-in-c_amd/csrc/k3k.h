@@ -201,9 +201,8 @@ int k3k_gemv_bf16(float *y, const float *x, const uint16_t *W, int in, int out, 
 int k3k_gemv_glu(float *y, const float *x, const void *Wg, const void *Wu, int bf16, int in, int out, int act,
                  float b1, float b2, void *stream);
 /* k3k_gemv_f32 / _bf16 for two tokens and more on the matrix cores (k3_tok.hip): W bf16 (bf16 1) or fp32,
- * where k3k_tok_ok holds; one token too where in % 8 != 0 or x or W is not 16-byte aligned.
- * k3k_gemv_* send their calls there. */
-int k3k_tok_ok(const float *x, const void *W, int in, int ntok);
+ * where k3k_tok_ok holds, at any alignment; one token too. k3k_gemv_* send their calls there. */
+int k3k_tok_ok(int in, int ntok);
 int k3k_tok_gemm(float *y, const float *x, const void *W, int bf16, int in, int out, int ntok, int ldy, int accumulate,
                  void *stream);
 /* y[t][r] = act(gate, up) of bf16 weights, fp32 x, where k3k_tok_glu_ok holds (as k3k_tok_gemm:

@@ -108,6 +108,39 @@ def test_tok_matmul_nan_tokens_cost(gpu, k3, bf16, T, inn, out):
     assert np.isnan(res[1][[3, T - 1]]).all() and np.array_equal(res[0][keep], res[1][keep])
     assert took[1] <= 10 * took[0] + 2e-5
 
+
+@pytest.mark.parametrize("T,inn,out", [(1, 1, 3), (1, 7, 5), (1, 520, 40), (1, 513, 33), (1, 1001, 999), (1, 4099, 70), (1, 7169, 300),
+                                       (2, 520, 65), (5, 512, 40), (33, 1024, 129), (64, 264, 300)])
+def test_matmul_any_alignment(gpu, k3, T, inn, out):
+    """Any row length, and x, W at any element: against fp64, and for one token bf16 weights give
+    the bits of fp32 weights of the same values (the reference's invariant), at every alignment."""
+    say(f"case: alignments, {T} tokens {inn} -> {out}")
+    Wb = k3.gen_bf16_normal(inn * out, 15 + inn, 0.0, 0.02).reshape(out, inn)
+    Wf = (Wb.astype(np.uint32) << 16).view(np.float32)
+    X = k3.gen_normal(T * inn, 16 + inn).reshape(T, inn)
+    want, bound = X.astype(np.float64) @ Wf.T.astype(np.float64), np.abs(X.astype(np.float64)) @ np.abs(Wf.T.astype(np.float64))
+    L = gpu.lib()
+    bufs = [gpu.DevBuf(a.nbytes + 64) for a in (X, Wb, Wf)] + [gpu.DevBuf(T * out * 4)]
+    dx, db, df, dy = bufs
+    first = None
+    try:
+        for ox, ow in ((0, 0), (1, 0), (0, 1), (3, 5), (2, 8)):
+            dx.upload(X, 4 * ox)
+            db.upload(Wb, 2 * ow)
+            df.upload(Wf, 4 * ow)
+            got = []
+            for fn, w in ((L.k3d_matmul_bf16, db.ptr + 2 * ow), (L.k3d_matmul_f32, df.ptr + 4 * ow)):
+                gpu.check(fn(dy.ptr, dx.ptr + 4 * ox, T, w, inn, out, None), "matmul")
+                got.append(dy.download(np.empty((T, out), np.float32)))
+                assert (np.abs(got[-1] - want) <= 1e-6 * bound).all(), (ox, ow)
+            if T == 1:
+                first = got[0] if first is None else first
+                assert np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32)), (ox, ow)
+                assert np.array_equal(got[0].view(np.uint32), first.view(np.uint32)), (ox, ow)
+    finally:
+        for b in bufs:
+            b.free()
+
 @pytest.mark.parametrize("T,inn,rows", [(3, 128, 1), (3, 7168, 2048), (8, 256, 17), (9, 384, 48), (17, 1152, 130), (33, 3584, 4097),
                                         (64, 896, 300), (65, 512, 4100), (130, 2176, 71), (257, 128, 1031),
                                         (3, 32, 5), (19, 224, 100), (40, 1504, 515), (100, 4128, 70)])
