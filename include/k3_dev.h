@@ -18,8 +18,9 @@
  * from several host threads on different streams, at once, never share a stream or an
  * event, and each gives the result it gives alone. A stream's side stream is made by
  * k3d_stream_create (the null stream's by k3d_init), or by the first call on a stream made
- * elsewhere; at most 256 caller streams at once. Calls that overlap on one stream, or
- * share a workspace, race.
+ * elsewhere; at most 256 caller streams at once have one (k3d_stream_create then fails, and on
+ * a stream made elsewhere everything runs on the stream itself). Calls that overlap on one
+ * stream, or share a workspace, race.
  *
  * Each names the reference function whose arithmetic it performs.
  */

@@ -208,14 +208,15 @@ extern "C" int k3k_sync(void *stream)
 /* ---- side streams --------------------------------------------------------------------
  * Work that may run beside the caller's (the activation split beside the router, the hot
  * experts' pass list; in the host entry points also the shared expert, on the second one)
- * goes to a side stream of the caller's stream: two per caller stream,
+ * goes to a side stream of the caller's stream: up to two per caller stream,
  * created with the default priority, non-blocking, with its own fork and join events.
  * Work is forked after what is already queued on the caller's stream and joined back into
  * it; both are event waits, so a stream being captured into a graph captures the side work
  * too, and calls that overlap on different caller streams never share a stream or an
- * event. Entries are made by k3k_side_init (the null stream, at initialisation), by
- * k3k_stream_create, or on a caller stream's first fork; k3k_stream_destroy removes its
- * stream's entry. */
+ * event. The first one is made by k3k_side_init (the null stream's, at initialisation), by
+ * k3k_stream_create, or on a caller stream's first fork, the second on its first use;
+ * k3k_stream_destroy removes its stream's entry. Past K3_SIDE_MAX caller streams, one that
+ * was made elsewhere has none: what would run beside it runs on it. */
 #define K3_SIDE_MAX 256
 struct K3Side {
     hipStream_t caller, side[2];
@@ -225,68 +226,80 @@ static K3Side g_side[K3_SIDE_MAX];
 static int g_nside = 0;
 static pthread_mutex_t g_side_mu = PTHREAD_MUTEX_INITIALIZER;
 
-/* The entry of caller stream s (made if absent), or NULL with the error set. */
-static K3Side *side_of(hipStream_t s)
+static void side_drop(K3Side *n, int k)
+{
+    if (n->join[k]) (void)hipEventDestroy(n->join[k]);
+    if (n->fork[k]) (void)hipEventDestroy(n->fork[k]);
+    if (n->side[k]) (void)hipStreamDestroy(n->side[k]);
+    n->join[k] = n->fork[k] = nullptr;
+    n->side[k] = nullptr;
+}
+
+/* Into *out the entry of caller stream s, with side stream k. `make`: made if absent. 1 if there is
+ * none (nothing to make it of, or not to be made), -1 with the error set. */
+static int side_of(hipStream_t s, int k, bool make, K3Side *out)
 {
     pthread_mutex_lock(&g_side_mu);
     K3Side *r = nullptr;
+    int rc = 1;
     for (int i = 0; i < g_nside; i++)
         if (g_side[i].caller == s) {
             r = &g_side[i];
             break;
         }
-    if (!r) {
-        if (g_nside == K3_SIDE_MAX) {
-            k3k_fail("side stream: more than 256 caller streams", hipErrorInvalidValue);
-        } else {
-            K3Side n = {};
-            n.caller = s;
-            hipError_t e = hipSuccess;
-            for (int k = 0; k < 2; k++) {
-                if (e == hipSuccess) e = hipStreamCreateWithFlags(&n.side[k], hipStreamNonBlocking);
-                if (e == hipSuccess) e = hipEventCreateWithFlags(&n.fork[k], hipEventDisableTiming);
-                if (e == hipSuccess) e = hipEventCreateWithFlags(&n.join[k], hipEventDisableTiming);
-            }
-            if (e == hipSuccess) {
-                g_side[g_nside] = n;
-                r = &g_side[g_nside++];
-            } else {
-                k3k_fail("side stream: create", e);
-                for (int k = 0; k < 2; k++) {
-                    if (n.join[k]) (void)hipEventDestroy(n.join[k]);
-                    if (n.fork[k]) (void)hipEventDestroy(n.fork[k]);
-                    if (n.side[k]) (void)hipStreamDestroy(n.side[k]);
-                }
-            }
+    if (!r && make && g_nside < K3_SIDE_MAX) {
+        r = &g_side[g_nside];
+        *r = K3Side{};
+        r->caller = s;
+    }
+    if (r && !r->side[k] && make) {
+        hipError_t e = hipStreamCreateWithFlags(&r->side[k], hipStreamNonBlocking);
+        if (e == hipSuccess) e = hipEventCreateWithFlags(&r->fork[k], hipEventDisableTiming);
+        if (e == hipSuccess) e = hipEventCreateWithFlags(&r->join[k], hipEventDisableTiming);
+        if (e != hipSuccess) {
+            side_drop(r, k);
+            rc = k3k_fail("side stream: create", e);
+        } else if (r == &g_side[g_nside]) {
+            g_nside++;
         }
     }
+    if (r && r->side[k]) {
+        *out = *r;
+        rc = 0;
+    }
     pthread_mutex_unlock(&g_side_mu);
-    return r;
+    return rc;
 }
 
 extern "C" int k3k_side_init(void)
 {
     if (k3k_init()) return -1;
-    return side_of(nullptr) ? 0 : -1;
+    K3Side sd;
+    const int rc = side_of(nullptr, 0, true, &sd);
+    return rc > 0 ? k3k_fail("side stream: more than 256 caller streams", hipErrorInvalidValue) : rc;
 }
 
 extern "C" int k3k_fork(void *stream, int which, void **side)
 {
-    K3Side *sd = side_of((hipStream_t)stream);
-    if (!sd) return -1;
-    hipError_t e = hipEventRecord(sd->fork[which], (hipStream_t)stream);
-    if (e == hipSuccess) e = hipStreamWaitEvent(sd->side[which], sd->fork[which], 0);
+    K3Side sd;
+    const int rc = side_of((hipStream_t)stream, which, true, &sd);
+    if (rc < 0) return rc;
+    *side = stream;
+    if (rc) return 0;
+    hipError_t e = hipEventRecord(sd.fork[which], (hipStream_t)stream);
+    if (e == hipSuccess) e = hipStreamWaitEvent(sd.side[which], sd.fork[which], 0);
     if (e != hipSuccess) return k3k_fail("fork", e);
-    *side = sd->side[which];
+    *side = sd.side[which];
     return 0;
 }
 
 extern "C" int k3k_join(void *stream, int which)
 {
-    K3Side *sd = side_of((hipStream_t)stream);
-    if (!sd) return -1;
-    hipError_t e = hipEventRecord(sd->join[which], sd->side[which]);
-    if (e == hipSuccess) e = hipStreamWaitEvent((hipStream_t)stream, sd->join[which], 0);
+    K3Side sd;
+    const int rc = side_of((hipStream_t)stream, which, false, &sd);
+    if (rc) return rc < 0 ? rc : 0;
+    hipError_t e = hipEventRecord(sd.join[which], sd.side[which]);
+    if (e == hipSuccess) e = hipStreamWaitEvent((hipStream_t)stream, sd.join[which], 0);
     return e == hipSuccess ? 0 : k3k_fail("join", e);
 }
 
@@ -298,7 +311,10 @@ extern "C" void *k3k_stream_create(void)
         k3k_fail("hipStreamCreate", e);
         return nullptr;
     }
-    if (!side_of(s)) {
+    K3Side sd;
+    const int rc = side_of(s, 0, true, &sd);
+    if (rc) {
+        if (rc > 0) k3k_fail("side stream: more than 256 caller streams", hipErrorInvalidValue);
         (void)hipStreamDestroy(s);
         return nullptr;
     }
@@ -312,10 +328,8 @@ extern "C" int k3k_stream_destroy(void *stream)
     for (int i = 0; i < g_nside; i++)
         if (g_side[i].caller == (hipStream_t)stream) {
             for (int k = 0; k < 2; k++) {
-                (void)hipStreamSynchronize(g_side[i].side[k]);
-                (void)hipEventDestroy(g_side[i].fork[k]);
-                (void)hipEventDestroy(g_side[i].join[k]);
-                (void)hipStreamDestroy(g_side[i].side[k]);
+                if (g_side[i].side[k]) (void)hipStreamSynchronize(g_side[i].side[k]);
+                side_drop(&g_side[i], k);
             }
             g_side[i] = g_side[--g_nside];
             break;
