@@ -121,3 +121,71 @@ def test_overcommitted_bank_layers(gpu, orc, wl):
         assert bank.stats()["evictions"] > 0 and bank.stats()["failures"] == 0
     finally:
         bank.destroy()
+
+
+@pytest.mark.parametrize("T", [1, 40, 333])
+def test_resident_shared_expert(gpu, wl, T):
+    """The shared expert on resident weights where its products run on the row kernel (one token),
+    on the several-token kernel and on the two-term GEMMs (333 tokens fill their tiles both ways):
+    every fetch fails, so the block's output is its shared expert alone, against fp64."""
+    from oracle import PySource
+    say(f"case: resident shared expert T={T}")
+    cfg, W, _ = wl.latent_layer(3584, 64, 1792, 4, 1, tag="host.shared", n_generated=0)
+    x = wl.tokens(T, 3584, tag=f"host.shared.{T}")
+    src = PySource({})
+    names = ("gate", "down", "up", "sh1", "sh3", "sh2")
+    try:
+        for a in names:
+            gpu.dev_register(W[a])
+        got = gpu.moe(x, cfg, W, 1, src.ptr, 1)[0]
+    finally:
+        for a in names:
+            gpu.dev_unregister(W[a])
+    want = shared_fp64(x, W)
+    assert np.linalg.norm(got - want) <= (1e-5 if T == 333 else 1e-6) * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("T", [1, 333])
+def test_resident_block_against_oracle(gpu, orc, wl, T):
+    """The whole block with its trunk resident and every expert in the HBM bank, one token and
+    enough for the GEMMs and the second pass list, against the oracle token by token."""
+    from conftest import max_err_rel_inf
+    from oracle import PySource, oracle_moe_q
+    say(f"case: resident block T={T}")
+    cfg, W, ex = wl.latent_layer(3584, 512, 1536, 24, 4, n_shared=3, tag="host.block")
+    x = wl.tokens(T, 3584, tag=f"host.block.{T}")
+    bank = gpu.HbmBank(1, 24, 512, 1536, 24)
+    names = ("gate", "down", "up", "sh1", "sh3", "sh2")
+    try:
+        for e in ex:
+            bank.put_run(0, e, wl.expert_run(ex[e]))
+        for a in names:
+            gpu.dev_register(W[a])
+        got = gpu.moe(x, cfg, W, 1, bank.src, int(T > 1))
+    finally:
+        for a in names:
+            gpu.dev_unregister(W[a])
+        bank.destroy()
+    assert got[3] == 0
+    for t in sorted({0, 1, 63, 64, 200, T - 1} & set(range(T))):
+        src = PySource(ex)
+        want = oracle_moe_q(orc, x[t:t + 1], cfg, W, 1, src, 0)
+        assert max_err_rel_inf(got[0][t:t + 1], want[0]) <= 1e-4, t
+
+
+def test_staging_rounds(gpu, orc, wl):
+    """x and the output in more than one round of the 32 MiB staging, the last one ragged."""
+    from conftest import max_err_rel_inf
+    from oracle import PySource, oracle_moe_q
+    T, E = 17003, 512
+    say(f"case: staging rounds, {T * E * 4 / 2**20:.1f} MiB")
+    cfg, W, ex = wl.latent_layer(E, 64, 32, 4, 2, n_shared=1, tag="host.stage")
+    x = wl.tokens(T, E, tag="host.stage")
+    src = PySource(ex)
+    got = gpu.moe(x, cfg, W, 1, src.ptr, 1)
+    assert got[3] == 0
+    for t in [0, 1, 4095, 4096, 8191, 16383, 16384, 16385, 16999, T - 2, T - 1]:
+        one = PySource(ex)
+        want = oracle_moe_q(orc, x[t:t + 1], cfg, W, 1, one, 0)
+        assert max_err_rel_inf(got[0][t:t + 1], want[0]) <= 1e-4, t
+    assert not np.array_equal(got[0][16384], got[0][0])

@@ -220,7 +220,8 @@ def test_k3_moe_threads(gpu, orc, wl, k3layer):
     import threading
     cfg, W, experts = k3layer
     xs = [tokens(wl, 3), tokens(wl, 1)]
-    alone = [gpu.moe(x, cfg, W, 1, PySource(experts).ptr, 1)[0] for x in xs]
+    first = [PySource(experts), PySource(experts)]      # (held while the library calls them)
+    alone = [gpu.moe(x, cfg, W, 1, s.ptr, 1)[0] for x, s in zip(xs, first)]
     res = [None, None]
     srcs = [PySource(experts), PySource(experts)]
 

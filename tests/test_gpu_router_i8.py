@@ -12,8 +12,9 @@ every branch of the split: rows whose largest value is 128 or more (scaled down,
 values may lose bits to the subnormal range), zero rows, values spread over many binades
 (left-out remainders), tiny and subnormal values, and a non-finite value (its chunk falls
 back to a plain fp64 chain). idx and weight bits equal the oracle's per-token router
-(k3_ops.c:419-478) for every token. The int8 partials serve 1024 tokens and more; the fp64
-matrix-core partials of fewer tokens are held to the same contract."""
+(k3_ops.c:419-478) for every token. The int8 partials serve 1024 tokens and more, and from 128
+where a cost rule finds them the faster ones (400 tokens of 896 experts, 608 of 512); the fp64
+matrix-core partials of the others are held to the same contract."""
 import sys
 
 import numpy as np
@@ -79,7 +80,7 @@ def check_contract(part, rb, chunk, W, X, tokens):
     return worst_err, worst_pre
 
 
-@pytest.mark.parametrize("T,N,K", [(1030, 384, 8), (1100, 200, 6)])
+@pytest.mark.parametrize("T,N,K", [(1030, 384, 8), (1100, 200, 6), (400, 896, 16), (608, 512, 8)])
 def test_router_i8_partials_and_selection(gpu, orc, T, N, K):
     say(f"case: int8 router partials T={T} N={N} K={K}")
     W, X = special_inputs(T, N, T + N)
@@ -101,7 +102,7 @@ def test_router_i8_partials_and_selection(gpu, orc, T, N, K):
 
 @pytest.mark.parametrize("T,N", [(300, 384), (64, 200)])
 def test_router_fp64_partials_contract(gpu, orc, T, N):
-    """The same contract for the fp64 matrix-core partials that serve 5 to 1023 tokens
+    """The same contract for the fp64 matrix-core partials, which serve these batches
     (router_partial_mfma_kernel, k3_route.hip), on the same special rows: the chunk sums
     within 2^-53 R_k of the exact ones, R_k above the exact prefix magnitudes, and idx /
     weight bits equal to the oracle's."""

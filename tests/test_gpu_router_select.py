@@ -40,8 +40,8 @@ def test_router_select_edges(gpu, orc, k3, T, N, K):
 
 @pytest.mark.parametrize("T,N,K", [(256, 896, 8), (128, 896, 16), (200, 1000, 10), (600, 640, 3)])
 def test_router_int8_partials_with_gather(gpu, orc, k3, T, N, K):
-    """The routed layer at sizes whose partials come from the int8 kernels (or nearly) and whose
-    gather runs in the final kernel's last workgroup; no expert is in the bank, so the layer
+    """The routed layer at sizes whose partials come from the int8 kernels (at 128 tokens still
+    from the fp64 ones) and whose gather runs in the final kernel's last workgroup; no expert is in the bank, so the layer
     is routing and gather alone."""
     from test_gpu_moe_device import stable_gather
     hid, inter = 7168, 512

@@ -176,6 +176,33 @@ def test_tok_mxfp4_edges(gpu, k3, T, inn, rows):
             b.free()
 
 
+
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("T,inn,rows", [(3, 256, 40), (40, 1504, 130), (70, 512, 515)])
+def test_mxfp4_codes_off_16_bytes(gpu, k3, T, inn, rows, prec):
+    """k3d_matmul_mxfp4 of three tokens and more with codes that do not start at a multiple of 16
+    bytes, which the several-token kernel does not take: the expert kernel, at the same
+    precision."""
+    say(f"case: mxfp4 codes at +8, {T} tokens {inn} -> {rows} prec={prec}")
+    rng = np.random.default_rng(T + rows)
+    codes = rng.integers(0, 256, (rows, inn // 2), dtype=np.uint8)
+    scales = rng.integers(118, 127, (rows, inn // 32), dtype=np.uint8)
+    X = k3.gen_normal(T * inn, 8 + T).reshape(T, inn)
+    val = np.array([0, .5, 1, 1.5, 2, 3, 4, 6, -0., -.5, -1, -1.5, -2, -3, -4, -6])
+    W = np.stack([val[codes & 15], val[codes >> 4]], axis=2).reshape(rows, inn) * np.repeat(2.0 ** (scales.astype(np.float64) - 127), 32, axis=1)
+    x = X.astype(np.float64) if prec == 0 else bf16_rne(X)
+    L = gpu.lib()
+    bufs = [gpu.DevBuf(X.nbytes).upload(X), gpu.DevBuf(codes.nbytes + 16).upload(codes, 8), gpu.DevBuf(scales.nbytes).upload(scales),
+            gpu.DevBuf(L.k3d_matmul_mxfp4_ws(T, inn)), gpu.DevBuf(T * rows * 4)]
+    dx, dp, ds, ws, dy = bufs
+    try:
+        gpu.check(L.k3d_matmul_mxfp4(dy.ptr, dx.ptr, T, dp.ptr + 8, ds.ptr, inn, rows, prec, ws.ptr, ws.nbytes, None), "mxfp4")
+        Y = dy.download(np.empty((T, rows), np.float32))
+    finally:
+        for b in bufs:
+            b.free()
+    assert (np.abs(Y - x @ W.T) <= ((2.0**-17 if prec == 0 else 0.0) + 1e-6) * (np.abs(x) @ np.abs(W.T))).all()
+
 @pytest.mark.parametrize("act", [0, 1])
 @pytest.mark.parametrize("T,hidden,inter", [(1, 64, 64), (2, 7168, 192), (8, 128, 4096), (9, 448, 4160), (16, 7168, 2048), (17, 7168, 64),
                                             (32, 4096, 128), (33, 64, 2048), (64, 192, 2048), (65, 320, 1984), (128, 64, 1024)])
