@@ -295,12 +295,12 @@ static size_t router_size(Carve *c, int T, int hidden, int n_experts)
     if (top < 32 * (6 * cus / nee + 2)) top = (int)(32 * (6 * cus / nee + 2));
     size_t most = start.off;
     for (int t = T; t > 0; t = t > i8 && i8 > top ? i8 : t > top ? top : t > 32 ? (t - 1) / 32 * 32 : t > 4 ? 4 : 0) {
-        const int chunk[2] = {k3k_router_i8_chunk(t, hidden, n_experts), k3k_router_chunk(t, hidden, n_experts, NULL)};
-        for (int i = 0; i < 2; i++) {
+        for (int i = t == T || t % 64 == 0 ? 0 : 1; i < 2; i++) {
             RtWs w;
-            if (!chunk[i]) continue;
+            const int chunk = i ? k3k_router_chunk(t, hidden, n_experts, NULL) : k3k_router_i8_chunk(t, hidden, n_experts);
+            if (!chunk) continue;
             *c = start;
-            router_layout(c, &w, t, hidden, n_experts, chunk[i], i == 0);
+            router_layout(c, &w, t, hidden, n_experts, chunk, i == 0);
             if (c->off > most) most = c->off;
         }
     }
