@@ -57,14 +57,11 @@
 namespace {
 
 constexpr int RI_ND = 6;                 /* digits per operand */
-/* Products of digits i, j with i + j <= RI_LMAX. The level 10 sums, 3 products of 33, change next to
- * nothing: 1030 tokens x 384 experts, chunks of 3584 columns, the partials' mean error is 2.95 2^-53
- * without and 2.92 with them, and the bound R the same for N(0, 1) rows (6847 in 2^-53); rows with
- * three values 30 / 100 / 1000 times the rest have an R of 1.21e4 / 5.19e4 / 2.68e6 without and
- * 9.2e3 / 3.31e4 / 2.46e6 with them, and neither leaves a logit to recompute (nor at 4096 x 384 and
- * 2048 x 896). Without, partials of 4096 tokens x 384 experts 270 -> 257 us; at 8 the bound of N(0, 1)
- * rows grows 16 times, and with it the recomputed logits. */
-constexpr int RI_LMAX = 9;
+/* Products of digits i, j with i + j <= RI_LMAX. At 9, 3 products of 33 less, the partials of 4096
+ * tokens x 384 experts take 257 us instead of 270, but they are held in fewer bits: on N(0, 1) rows the
+ * mean error against 64 bits grows by 0.5-1 % and the bound R by 15 %, on rows with three values 30 /
+ * 100 / 1000 times the rest R by up to 60 / 60 / 30 % (400 to 1030 tokens x 384 to 896 experts). */
+constexpr int RI_LMAX = 10;
 constexpr int RI_NL = RI_LMAX - 1;       /* level accumulators, l = 2 .. RI_LMAX */
 constexpr int RI_STEP = 64;              /* columns per step: one int8 matrix instruction */
 constexpr int RI_TT = 64, RI_TE = 64;    /* workgroup tile: tokens, experts */
@@ -270,7 +267,7 @@ __device__ __forceinline__ float ri_bound_up(double rb)
 struct RiPair {
     int i, j;
 };
-constexpr int RI_NP = 30;                /* pairs with i, j <= RI_ND and i + j <= RI_LMAX */
+constexpr int RI_NP = 33;                /* pairs with i, j <= RI_ND and i + j <= RI_LMAX */
 struct RiPairs {
     RiPair p[RI_NP];
 };

@@ -179,3 +179,20 @@ def test_router_unaligned_rows(gpu, k3, T, N, K, off_x, off_w):
     assert columns(chunk) <= columns(c8)
     if (T, N) == (608, 512):
         assert c8 % 256 == 0 and columns(chunk) < columns(c8)
+
+
+def test_router_i8_lowest_level(gpu):
+    """Products of both rows' fifth digits (level 10, the lowest kept) are in the sums: every row's
+    largest value meets a zero, and the one product left, a 2^-30 times b 2^-30 under a scale of
+    2^6, is digit 16 a times digit 16 b. The partials are that product exactly."""
+    T, N, K = 1030, 384, 8
+    say(f"case: int8 router partials, lowest level, T={T} N={N}")
+    a, b = 1 + np.arange(T) % 7, 1 + np.arange(N) % 7
+    X, W = np.zeros((T, HID), np.float32), np.zeros((N, HID), np.float32)
+    X[:, 0] = W[:, 1] = 1.0
+    X[:, 2], W[:, 2] = a * 2.0**-30, b * 2.0**-30
+    gpu.router_device(X, W, None, K, partials=True)
+    part, rb, chunk = gpu.router_device.partials
+    assert chunk >= 256 and chunk % 256 == 0
+    assert np.array_equal(part[0], np.outer(a, b) * 2.0**-60) and not part[1:].any()
+    check_contract(part, rb, chunk, W, X, [0, 6, T - 1])
