@@ -261,11 +261,11 @@ static void router_layout(Carve *c, RtWs *w, int T, int hidden, int n_experts, i
 /* The router's part of a workspace that ends at ws_bytes: the int8 partials where they serve the
  * batch (`rows16`: 16-byte aligned x and W) and fit, else the fp64 ones with their own chunks (idx
  * and weights are the same bits); rows that are not aligned take the int8 partials' chunks where
- * only those fit (608 tokens of 512 experts: 1792 columns a chunk, up to 7168 on the busiest CU,
- * where its own chunks leave 4320). 0 if nothing fits; *need (may be NULL): the least that does. */
+ * only those fit (1030 tokens of 384 experts: 3584 columns a chunk, 7168 on the busiest CU, where
+ * its own chunks leave 5600). 0 if nothing fits; *need (may be NULL): the least that does. */
 static int router_plan(Carve *c, RtWs *w, size_t ws_bytes, int rows16, int T, int hidden, int n_experts, size_t *need)
 {
-    const int c8 = k3k_router_i8_chunk(T, hidden, n_experts), c64 = k3k_router_chunk(T, hidden, n_experts, NULL);
+    const int c8 = k3k_router_i8_chunk(T, hidden, n_experts), c64 = k3k_router_chunk(T, hidden, n_experts);
     const struct {
         int chunk, i8;
     } way[3] = {{rows16 ? c8 : 0, 1}, {c64, 0}, {rows16 ? 0 : c8, 0}};
@@ -297,7 +297,7 @@ static size_t router_size(Carve *c, int T, int hidden, int n_experts)
     for (int t = T; t > 0; t = t > i8 && i8 > top ? i8 : t > top ? top : t > 32 ? (t - 1) / 32 * 32 : t > 4 ? 4 : 0) {
         for (int i = t == T || t % 64 == 0 ? 0 : 1; i < 2; i++) {
             RtWs w;
-            const int chunk = i ? k3k_router_chunk(t, hidden, n_experts, NULL) : k3k_router_i8_chunk(t, hidden, n_experts);
+            const int chunk = i ? k3k_router_chunk(t, hidden, n_experts) : k3k_router_i8_chunk(t, hidden, n_experts);
             if (!chunk) continue;
             *c = start;
             router_layout(c, &w, t, hidden, n_experts, chunk, i == 0);

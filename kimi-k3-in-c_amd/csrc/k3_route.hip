@@ -1607,9 +1607,8 @@ extern "C" int k3k_split_bf16(uint16_t *hi, uint16_t *lo, const float *x, size_t
  * block per wave). */
 constexpr int RM_TB = 32, RM_EB = 64;
 
-extern "C" int k3k_router_chunk(int T, int hidden, int n_experts, long *load_out)
+extern "C" int k3k_router_chunk(int T, int hidden, int n_experts)
 {
-    if (load_out) *load_out = 0;
     if (T <= RS_T) return RS_CH;          /* one lane per (expert, 128-column chunk) */
     const long tiles = (long)((n_experts + RM_EB - 1) / RM_EB) * ((T + RM_TB - 1) / RM_TB);
     const long cus = k3k_cu_count() > 0 ? k3k_cu_count() : 1;
@@ -1622,11 +1621,7 @@ extern "C" int k3k_router_chunk(int T, int hidden, int n_experts, long *load_out
         ks = (ks + K3_NXCD - 1) / K3_NXCD * K3_NXCD;
         while (ks > K3_NXCD && hidden / ks < 224) ks -= K3_NXCD;
         const long chunk = ((hidden + ks - 1) / ks + RP_KS - 1) / RP_KS * RP_KS;
-        const long n = (hidden + chunk - 1) / chunk;
-        if (chunk >= 224 && n % K3_NXCD == 0) {
-            if (load_out) *load_out = (tiles * n + cus - 1) / cus * chunk;
-            return (int)chunk;
-        }
+        if (chunk >= 224 && ((hidden + chunk - 1) / chunk) % K3_NXCD == 0) return (int)chunk;
     }
     /* chunks a multiple of 32 columns and at least 256; among those, the split whose
      * busiest CU has the least work (workgroups per CU x columns per workgroup), the most
@@ -1643,7 +1638,6 @@ extern "C" int k3k_router_chunk(int T, int hidden, int n_experts, long *load_out
         const long load = per_cu * chunk;
         if (best_load < 0 || load <= best_load) { best_load = load; best_chunk = chunk; }
     }
-    if (load_out) *load_out = best_load;
     return (int)best_chunk;
 }
 

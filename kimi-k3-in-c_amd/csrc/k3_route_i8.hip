@@ -450,7 +450,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 }  // namespace
 
 /* ---- host side ------------------------------------------------------------------------ */
-constexpr int RI_MIN_T = 128;            /* fewer tokens: the fp64 kernels */
+/* Fewer tokens: the fp64 kernels, whose sums are the more accurate ones of rows that hold outliers: the
+ * digits end 2^-42 below a row chunk's largest value. (Error against 64 bits, root mean square in
+ * 2^-53, 400 tokens x 896 experts: N(0, 1) rows 8.5 there and 28 here, with three values 30 / 100 / 1000
+ * times the rest 10 / 22 / 155 and 1.1e3 / 7.2e3 / 5.9e4; the bounds cover either, and idx and weights are
+ * the same bits.) The int8 kernels would be the faster ones from about 400 tokens (512 tokens x 896
+ * experts 118 us for 160, 1000 x 384 110 for 142). */
+constexpr int RI_MIN_T = 1024;
 constexpr int RI_MAXTT = 128;            /* more token tiles: no choice of chunks */
 
 static int ri_round(int v, int m) { return (v + m - 1) / m * m; }
@@ -458,8 +464,7 @@ static int ri_round(int v, int m) { return (v + m - 1) / m * m; }
 extern "C" int k3k_router_i8_chunk(int T, int hidden, int n_experts)
 {
     if (T < RI_MIN_T || hidden <= 0 || hidden % RI_STEP || n_experts <= 0) return 0;
-    /* (below 1024 tokens and from there on, what follows depends on the token tiles only: workspace
-     * sizes go over those) */
+    /* (what follows depends on the token tiles only: workspace sizes go over those) */
     const int Tp = ri_round(T, RI_TT);
     const long ntt = Tp / RI_TT, nte = ri_round(n_experts, RI_TE) / RI_TE;
     const long cus = k3k_cu_count() >= K3_NXCD ? k3k_cu_count() / K3_NXCD : 1;     /* per XCD */
@@ -484,20 +489,6 @@ extern "C" int k3k_router_i8_chunk(int T, int hidden, int n_experts)
         if (ntt > RI_MAXTT) break;             /* rounds enough: the longest chunks */
     }
     if (!ks) return 0;
-    /* Up to 1023 tokens: against the fp64 kernel, both in us, fitted to 91 shapes of 128 to 1000
-     * tokens and 128 to 1400 experts of 7168 columns (rms 18 us, most of it at the largest). fp64: the
-     * busiest CU's columns; int8: its steps, the digits of both operands, the partials. Whole router,
-     * fp64 / int8: 384 experts, 300 tokens 59 / 59, 400 67 / 71, 1000 141 / 109 us; 896 experts, 200
-     * tokens 86 / 76, 400 149 / 115, 1000 292 / 203; 128 experts, 512 tokens 36 / 54. From 1024 the
-     * int8 ones always. */
-    if (T < 1024) {
-        long load = 0;
-        const int c64 = k3k_router_chunk(Tp, hidden, n_experts, &load);
-        const double tn = 1e-6 * Tp * n_experts;
-        const double f64 = 0.0266 * (double)load - 2.3 * ((hidden + c64 - 1) / c64) * tn + 17.3;
-        const double i8 = 1.55 * (double)best + 1e-6 * hidden * ((double)Tp + n_experts) + 6.4 * ks * tn + 7.7;
-        if (i8 >= f64) return 0;
-    }
     const size_t xbytes = (size_t)Tp * (size_t)hidden * RI_ND;
     const size_t wbytes = (size_t)ri_round(n_experts, RI_TE) * (size_t)hidden * RI_ND;
     if (xbytes >= ((size_t)1 << 31) || wbytes >= ((size_t)1 << 31)) return 0;

@@ -230,8 +230,7 @@ int k3k_gemv_q8(float *y, const float *x, const void *W, int in, int out, int nt
  * fp32 rounding and the logit matters), sigmoid with the host libm's expf, biased
  * first-strict-max top-k, renorm, scale -> idx/wt [T][topk]; nrecomp [T] (may be NULL)
  * receives the number of recomputed logits per token, *used (may be NULL) the chunk width. */
-/* load (may be NULL): the columns of the busiest CU's workgroups */
-int k3k_router_chunk(int T, int hidden, int n_experts, long *load);
+int k3k_router_chunk(int T, int hidden, int n_experts);
 /* 1 when k3k_router_partial scores and certifies the logits itself (a few tokens): its
  * part then holds one 16-byte record per logit, which a selecting decode gate/up reads. */
 int k3k_router_small(int T, int hidden);

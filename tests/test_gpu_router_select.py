@@ -38,11 +38,11 @@ def test_router_select_edges(gpu, orc, k3, T, N, K):
             assert np.array_equal(bits(wt[t]), bits(w2)), t
 
 
-@pytest.mark.parametrize("T,N,K", [(256, 896, 8), (128, 896, 16), (200, 1000, 10), (600, 640, 3)])
+@pytest.mark.parametrize("T,N,K", [(256, 896, 8), (128, 896, 16), (200, 1000, 10), (600, 640, 3), (1024, 384, 2)])
 def test_router_int8_partials_with_gather(gpu, orc, k3, T, N, K):
-    """The routed layer at sizes whose partials come from the int8 kernels (at 128 tokens still
-    from the fp64 ones) and whose gather runs in the final kernel's last workgroup; no expert is in the bank, so the layer
-    is routing and gather alone."""
+    """The routed layer at sizes whose gather runs in the final kernel's last workgroup, with the
+    partials from the fp64 kernels and (1024 tokens) the int8 ones; no expert is in the bank, so the
+    layer is routing and gather alone."""
     from test_gpu_moe_device import stable_gather
     hid, inter = 7168, 512
     say(f"case: routing and gather {N} experts top-{K}, {T} tokens")
