@@ -87,7 +87,9 @@ int k3d_matmul_mxfp4(float *y, const float *x, int ntok, const uint8_t *packed,
                      size_t ws_bytes, void *stream);
 
 /* Y[ntok][out] = X[ntok][in] . W^T for fp32 / bf16 weights (reference k3_ops.c:265-291,
- * 1108-1213). */
+ * 1108-1213), fp32-accurate. One token: bf16 weights give the bits of fp32 weights of the same
+ * values. Two and more run on the matrix cores: there the two agree within rounding, and a token's
+ * result depends in its last bits on the number of tokens. */
 int k3d_matmul_f32(float *y, const float *x, int ntok, const float *W, int in, int out,
                    void *stream);
 int k3d_matmul_bf16(float *y, const float *x, int ntok, const uint16_t *W, int in, int out,
