@@ -553,14 +553,20 @@ __global__ __launch_bounds__(64 * KW) void tok_gemm_kernel(TokArgs a)
         }
 }
 
+/* KB of a stage (MX: beside 2 MT KB of codes in two chunks), and the waves of a workgroup: eight where
+ * two stages of theirs fit 160 KB of LDS, else four */
+constexpr int tok_stage_kb(int wt, int mt, int n8) { return wt == TOK_MX ? n8 : mt * (wt == TOK_F32 ? 2 : 1) + n8; }
+constexpr int tok_waves(int wt, int mt, int n8)
+{
+    return 8 * (2 * tok_stage_kb(wt, mt, n8) + (wt == TOK_MX ? 2 * mt : 0)) <= 160 ? 8 : 4;
+}
+
 template <int WT, int XT, int GLU, int MT, int N8>
 int launch_tok(TokArgs a, hipStream_t st)
 {
-    /* eight waves where two stages of theirs fit 160 KB of LDS, else four; up to four stages (MX: two
-     * or four, beside two chunks of codes) */
+    /* up to four stages (MX: two or four) */
     constexpr int MX = WT == TOK_MX;
-    constexpr int SKB = MX ? N8 : MT * (WT == TOK_F32 ? 2 : 1) + N8, CKB = MX ? 2 * MT : 0;
-    constexpr int KW = 8 * (2 * SKB + CKB) <= 160 ? 8 : 4;
+    constexpr int SKB = tok_stage_kb(WT, MT, N8), CKB = MX ? 2 * MT : 0, KW = tok_waves(WT, MT, N8);
     constexpr int RKB = (KW - 1) * MT * ((N8 + 1) / 2) - KW * SKB;       /* the sums beyond buffer 0 */
     constexpr int S4 = (160 - (RKB > 0 ? RKB : 0) - KW * CKB) / (KW * SKB), ST = XT == 2 ? 2 : S4 >= 4 ? 4 : MX ? 2 : S4;
     const int rows = GLU ? a.rpt : 16 * MT;
@@ -575,63 +581,81 @@ int launch_tok(TokArgs a, hipStream_t st)
 
 /* Cycles for the workgroups that fall to the busiest CU: per workgroup, K columns of cutting x
  * (fp32 activations against bf16 weights), moving the operands (50 bytes per cycle) and
- * multiplying, of which the largest counts whole and the others by 0.4 (measured, how far they
- * overlap), and about 4 us (9600 cycles) to start, fill the stages and add up. */
+ * multiplying, of which the largest counts whole and the others by how far they do not overlap,
+ * and the start, the filling of the stages and the adding up, 3 to 4 us. The overlap is fitted to 18
+ * shapes at 8 matrices (1024 -> 512 to 12288 -> 16384) x 12 token counts (2 to 512): 0.4, and for
+ * fp32 weights 0.2 where eight waves fit the LDS and 1 (none) where four do, one to a SIMD. The
+ * shape taken is then, over those 96 products, on average 0.7 % (bf16; at most 10), 1 % (fp32; 11) and
+ * 0.9 % (MXFP4; 15) slower than the best of the 18; with 0.4 for fp32 weights as well, 11 % (61).
+ * Counting the dequantisation of MXFP4 codes changed no choice for the better. */
 float tok_cost(int wt, int xt, int mt, int n8, int out, int ntok, int in, int cus)
 {
     const long wgs = (long)((out + 16 * mt - 1) / (16 * mt)) * ((ntok + 8 * n8 - 1) / (8 * n8));
     const int nb = (n8 + 1) / 2;
+    const bool f32 = wt == TOK_F32;
     const float cut = xt ? 0.f : wt == TOK_BF16 ? 16.f * nb * 5.5f / 64.f : 0.f;
-    const float bytes = (16.f * mt * (wt == TOK_F32 ? 4.f : wt == TOK_BF16 ? 2.f : 0.6f) + 8.f * n8 * 4) / 50.f;
-    const float mfma = mt * nb * 512.f * (wt == TOK_F32 ? 1.f / 256.f : (xt ? 2.f : 3.f) / 4096.f);
+    const float bytes = (16.f * mt * (f32 ? 4.f : wt == TOK_BF16 ? 2.f : 0.6f) + 8.f * n8 * 4) / 50.f;
+    const float mfma = mt * nb * 512.f * (f32 ? 1.f / 256.f : (xt ? 2.f : 3.f) / 4096.f);
+    const float over = !f32 ? 0.4f : tok_waves(wt, mt, n8) == 8 ? 0.2f : 1.f;
     float c = cut > bytes ? cut : bytes;
     if (mfma > c) c = mfma;
-    c += 0.4f * (cut + bytes + mfma - c);
-    return (c * in + 9600.f) * (float)((wgs + cus - 1) / cus);
+    c += over * (cut + bytes + mfma - c);
+    return (c * in + (f32 ? 7200.f : 9600.f)) * (float)((wgs + cus - 1) / cus);
 }
 
 template <int WT, int XT>
 int dispatch_tok(const TokArgs &a, hipStream_t st)
 {
-    static const int shapes[][2] = {{1, 1}, {1, 2}, {1, 3}, {1, 4}, {1, 5}, {1, 6}, {1, 8},
-                                    {2, 1}, {2, 2}, {2, 4}, {2, 8}, {3, 1}, {3, 2}, {3, 4},
-                                    {4, 1}, {4, 2}, {4, 4}, {4, 8}};
+    /* (row tiles, groups of 8 tokens); the last five are ever the cheapest for fp32 weights only */
+    static const int shapes[][2] = {{1, 1}, {1, 2}, {2, 1}, {2, 2}, {2, 4}, {3, 1}, {3, 2}, {3, 4}, {4, 1},
+                                    {4, 2}, {4, 4}, {4, 8}, {1, 3}, {1, 4}, {1, 5}, {1, 6}, {1, 8}};
     int best = 0;
     float bc = 0;
-    for (int i = 0; i < (int)(sizeof shapes / sizeof shapes[0]); i++) {
+    for (int i = 0; i < (WT == TOK_F32 ? 17 : 12); i++) {
         const float c = tok_cost(WT, XT, shapes[i][0], shapes[i][1], a.out, a.ntok, a.in, k3k_cu_count());
         if (i == 0 || c < bc) {
             best = i;
             bc = c;
         }
     }
+    if constexpr (WT == TOK_F32) {
+        switch (best) {
+        case 12: return launch_tok<WT, XT, 0, 1, 3>(a, st);
+        case 13: return launch_tok<WT, XT, 0, 1, 4>(a, st);
+        case 14: return launch_tok<WT, XT, 0, 1, 5>(a, st);
+        case 15: return launch_tok<WT, XT, 0, 1, 6>(a, st);
+        case 16: return launch_tok<WT, XT, 0, 1, 8>(a, st);
+        }
+    }
     switch (best) {
     case 0: return launch_tok<WT, XT, 0, 1, 1>(a, st);
     case 1: return launch_tok<WT, XT, 0, 1, 2>(a, st);
-    case 2: return launch_tok<WT, XT, 0, 1, 3>(a, st);
-    case 3: return launch_tok<WT, XT, 0, 1, 4>(a, st);
-    case 4: return launch_tok<WT, XT, 0, 1, 5>(a, st);
-    case 5: return launch_tok<WT, XT, 0, 1, 6>(a, st);
-    case 6: return launch_tok<WT, XT, 0, 1, 8>(a, st);
-    case 7: return launch_tok<WT, XT, 0, 2, 1>(a, st);
-    case 8: return launch_tok<WT, XT, 0, 2, 2>(a, st);
-    case 9: return launch_tok<WT, XT, 0, 2, 4>(a, st);
-    case 10: return launch_tok<WT, XT, 0, 2, 8>(a, st);
-    case 11: return launch_tok<WT, XT, 0, 3, 1>(a, st);
-    case 12: return launch_tok<WT, XT, 0, 3, 2>(a, st);
-    case 13: return launch_tok<WT, XT, 0, 3, 4>(a, st);
-    case 14: return launch_tok<WT, XT, 0, 4, 1>(a, st);
-    case 15: return launch_tok<WT, XT, 0, 4, 2>(a, st);
-    case 16: return launch_tok<WT, XT, 0, 4, 4>(a, st);
+    case 2: return launch_tok<WT, XT, 0, 2, 1>(a, st);
+    case 3: return launch_tok<WT, XT, 0, 2, 2>(a, st);
+    case 4: return launch_tok<WT, XT, 0, 2, 4>(a, st);
+    case 5: return launch_tok<WT, XT, 0, 3, 1>(a, st);
+    case 6: return launch_tok<WT, XT, 0, 3, 2>(a, st);
+    case 7: return launch_tok<WT, XT, 0, 3, 4>(a, st);
+    case 8: return launch_tok<WT, XT, 0, 4, 1>(a, st);
+    case 9: return launch_tok<WT, XT, 0, 4, 2>(a, st);
+    case 10: return launch_tok<WT, XT, 0, 4, 4>(a, st);
     default: return launch_tok<WT, XT, 0, 4, 8>(a, st);
     }
 }
 
-/* any K and alignment: fewer shapes */
+/* any K and alignment: fewer shapes. Two row tiles to a workgroup where they make fewer rounds of
+ * workgroups: a round of them takes 1.2-1.3 times a round of one tile with bf16 weights (7169 -> 3584,
+ * 128 tokens: 53.7 us in one round, 85.9 in two of one tile; 64 tokens 52.4 and 46.2, both one round),
+ * and about twice it with fp32 weights, for which they have to halve the rounds (3585 -> 7168: 16 tokens
+ * 21.5 us in one round, 24.5 in two; 200 tokens 253 in four, 225 in seven). Up to 8 tokens, where the
+ * weights' bytes are what counts, two rounds are no slower than one of twice as many (2049 -> 7168, 2
+ * tokens: bf16 7.7 and 8.2, fp32 13.0 and 14.8). */
 template <int WT>
 int dispatch_any(const TokArgs &a, hipStream_t st)
 {
-    const bool two = (a.out + 31) / 32 * ((a.ntok + 63) / 64) >= k3k_cu_count();
+    const long ntt = a.ntok <= 32 ? 1 : (a.ntok + 63) / 64, cus = k3k_cu_count() > 0 ? k3k_cu_count() : 1;
+    const long r1 = ((a.out + 15) / 16 * ntt + cus - 1) / cus, r2 = ((a.out + 31) / 32 * ntt + cus - 1) / cus;
+    const bool two = (a.ntok > 8 || r1 > 2) && (WT == TOK_BF16 ? r2 < r1 : 2 * r2 <= r1);
     if (a.ntok <= 8) return two ? launch_tok<WT, 2, 0, 2, 1>(a, st) : launch_tok<WT, 2, 0, 1, 1>(a, st);
     if (a.ntok <= 16) return two ? launch_tok<WT, 2, 0, 2, 2>(a, st) : launch_tok<WT, 2, 0, 1, 2>(a, st);
     if (a.ntok <= 32) return two ? launch_tok<WT, 2, 0, 2, 4>(a, st) : launch_tok<WT, 2, 0, 1, 4>(a, st);

@@ -39,6 +39,18 @@ def test_tok_matmul_edges(gpu, k3, bf16, T, inn, out):
         assert rel.max() <= 1e-6
 
 
+# (sizes that between them take every tile shape the products are launched with, the K waves with
+# several stages each)
+@pytest.mark.parametrize("bf16", [True, False])
+@pytest.mark.parametrize("T,inn,out", [(20, 1160, 19), (697, 1080, 38), (2, 1072, 4115), (395, 1032, 316), (677, 1064, 275),
+                                       (3, 1056, 8205), (489, 1048, 369), (676, 1032, 372), (389, 1056, 619), (585, 1040, 633),
+                                       (675, 1048, 1109), (686, 1072, 81), (674, 1088, 165), (629, 1048, 194), (680, 1048, 244),
+                                       (618, 1048, 385), (675, 1056, 81), (682, 1056, 331), (691, 1048, 535), (617, 1032, 770),
+                                       (9, 1033, 4200), (17, 1033, 4200), (33, 1033, 4200)])
+def test_tok_matmul_shapes(gpu, k3, bf16, T, inn, out):
+    test_tok_matmul_edges(gpu, k3, bf16, T, inn, out)
+
+
 @pytest.mark.parametrize("inn", [136, 137])
 @pytest.mark.parametrize("bf16", [True, False])
 def test_tok_matmul_nonfinite(gpu, k3, bf16, inn):
@@ -174,6 +186,13 @@ def test_tok_mxfp4_edges(gpu, k3, T, inn, rows):
     finally:
         for b in bufs:
             b.free()
+
+
+@pytest.mark.parametrize("T,inn,rows", [(697, 1088, 38), (700, 1024, 129), (682, 1056, 331), (691, 1088, 65), (683, 1056, 170),
+                                        (618, 1056, 385), (681, 1120, 104), (680, 1056, 244), (691, 1056, 535), (617, 1024, 770)])
+def test_tok_mxfp4_shapes(gpu, k3, T, inn, rows):
+    """Every tile shape the MXFP4 products are launched with."""
+    test_tok_mxfp4_edges(gpu, k3, T, inn, rows)
 
 
 
