@@ -968,8 +968,9 @@ static void moe_latent(float *out, const float *x, const K3MoeW *w, const K3Cfg 
      * side stream and is joined before its sum is added. One token: forked before the router, so
      * that it waits for x alone, but sent after the router and the down-projection, whose few
      * launches are over about when its own arrive: mostly it runs beside the routed experts. More:
-     * forked behind the down-projection, beside the routed experts, which leave the matrix cores
-     * idle (beside the router of 333 tokens it made that and the down-projection 0.23 ms longer). */
+     * forked behind the down-projection, beside the routed experts or, where the two side streams
+     * share a hardware queue, behind their second pass list (beside the router of 333 tokens it made
+     * that and the down-projection 0.23 ms longer). */
     const int shared = SI > 0 && w->sh1 && w->sh3 && w->sh2;
     const int shared_side = shared && k3_dev_lookup(w->sh1) && k3_dev_lookup(w->sh3) &&
                             k3_dev_lookup(w->sh2) && wbytes(w->wdt, E, SI) > 0;

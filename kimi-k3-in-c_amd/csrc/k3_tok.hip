@@ -9,7 +9,7 @@
  * product took, for 7168 -> 3584 in bf16, 13 / 22 / 94 / 153 / 607 us at 4 / 8 / 37 / 64 / 256
  * tokens (fp32: 18 / 33 / - / 222 / 876). Here a weight is read once per block of up to 64
  * tokens and the products run on the matrix cores: 10.5 / 11.2 / 20.8 / 25 / 55 us (fp32: 17.2
- * / 17.6 / - / 38 / 179).
+ * / 17.6 / - / 38 / 144).
  *
  *   bf16 weights: x is cut into three bf16 terms by truncation, x = h + m + l. Each cut
  *     keeps the next 8 significand bits, so the three terms hold all 24 and every product
@@ -40,11 +40,13 @@
  * columns 8g .. 8g+7. No scratch memory: the entry points have none to give, so K cannot be
  * split over workgroups, and every row block reads all of its tokens' x.
  *
- * What bounds it: for few tokens the weight stream; from about 16 tokens the reads of x, which
- * reach about 50 bytes a cycle and CU (64 is the L1's width); past that cutting x (5.5 vector
- * instructions per element: cutting with v_dot2_f32_bf16, 3.5 instructions, changed nothing)
- * and, for fp32 weights, the fp32 matrix rate (1/16 of bf16). The launch rule (tok_cost)
- * weighs these.
+ * What bounds it: for few tokens the weight stream, the fill of the stages and the adding up; from
+ * about 16 tokens no unit by itself (counters: 14-29 bytes a cycle and CU through the L1, whose width is
+ * 64; matrix pipes busy 26-28 % of the cycles in large bf16 and MXFP4 products, vector issue 34-40 %;
+ * 55 and 24 % for fp32 weights, whose matrix rate is 1/16), but the chain of a wave's stage -- its
+ * copies' arrival, the LDS reads, the cut (5.5 vector instructions per element; with v_dot2_f32_bf16,
+ * 3.5, nothing changed) or dequantisation, the products -- since the LDS holds one or two waves to a
+ * SIMD. The launch rule (tok_cost) weighs these.
  *
  * Infinities and NaN: the cut of an infinite x, or a zero term against an infinite weight,
  * gives NaN where the product of the uncut values is infinite. Finite operands give none, so
@@ -580,7 +582,7 @@ int launch_tok(TokArgs a, hipStream_t st)
 }
 
 /* Cycles for the workgroups that fall to the busiest CU: per workgroup, K columns of cutting x
- * (fp32 activations against bf16 weights), moving the operands (50 bytes per cycle) and
+ * (fp32 activations against bf16 weights), moving the operands (50 bytes per cycle, fitted) and
  * multiplying, of which the largest counts whole and the others by how far they do not overlap,
  * and the start, the filling of the stages and the adding up, 3 to 4 us. The overlap is fitted to 18
  * shapes at 8 matrices (1024 -> 512 to 12288 -> 16384) x 12 token counts (2 to 512): 0.4, and for
