@@ -473,7 +473,9 @@ extern "C" int k3k_router_i8_chunk(int T, int hidden, int n_experts)
      * rounds on an XCD, which takes whole (chunk, token tile) pairs, x (steps + 10 for a workgroup's
      * start and end and the partials it adds); the fewest among equals. (The fewest chunks that give
      * every CU two workgroups, before: 2048 tokens of 128 experts 896 workgroups of 8 steps, 166 us
-     * with the final kernel, now 256 of 28, 103.) */
+     * with the final kernel, now 256 of 28, 103. The digits and products of a column are the same in any
+     * chunk; a longer chunk has the larger scale: 1030 tokens of 384 experts, N(0, 1) rows, the sums are
+     * off by 21.5 2^-53 root mean square in 7 chunks and 23.7 in 2.) */
     if (hidden % (RI_STEP * RI_SPS)) return 0;
     const int ngrp = hidden / (RI_STEP * RI_SPS);
     int ks = 0;
