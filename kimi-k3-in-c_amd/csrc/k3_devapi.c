@@ -192,9 +192,9 @@ int k3d_matmul_mxfp4(float *y, const float *x, int ntok, const uint8_t *packed,
     a.scales = scales;
     if (k3k_mx_small_ok(ntok, in, prec == 0 ? 2 : 1, rows, x)) {
         a.xf32 = x;                 /* one or two tokens: the kernel splits x itself */
-    } else if (k3k_tok_mx_ok(w.xhi, w.xlo, packed, in, ntok)) {
-        /* three tokens and more (7168 -> 2048: 13.4 -> 11.2 us at 3, 273 -> 54 at 512, one term
-         * 172 -> 54) */
+    } else if (k3k_tok_mx_ok(w.xhi, w.xlo, packed, in, ntok) && k3k_tok_mx_pays(in, rows, ntok, prec == 0 ? 2 : 1)) {
+        /* three tokens and more (7168 -> 2048: 13.4 us on the streaming kernel and 11.2 here at 3, 273
+         * and 54 at 512, one term 172 and 54) */
         uint16_t *lo = prec == 0 ? w.xlo : NULL;
         if (k3k_split_bf16(w.xhi, lo, x, (size_t)ntok * in, stream)) return fail("split");
         k3k_prof_mark(stream, K3D_STAGE_BEGIN);

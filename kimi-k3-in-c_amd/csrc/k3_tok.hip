@@ -605,21 +605,29 @@ float tok_cost(int wt, int xt, int mt, int n8, int out, int ntok, int in, int cu
     return (c * in + (f32 ? 7200.f : 9600.f)) * (float)((wgs + cus - 1) / cus);
 }
 
+/* (row tiles, groups of 8 tokens); the last five are ever the cheapest for fp32 weights only */
+const int TOK_SHAPES[17][2] = {{1, 1}, {1, 2}, {2, 1}, {2, 2}, {2, 4}, {3, 1}, {3, 2}, {3, 4}, {4, 1},
+                               {4, 2}, {4, 4}, {4, 8}, {1, 3}, {1, 4}, {1, 5}, {1, 6}, {1, 8}};
+
+/* The cheapest shape, and its cycles. */
+int tok_pick(int wt, int xt, int out, int ntok, int in, float *cycles)
+{
+    int best = 0;
+    for (int i = 0; i < (wt == TOK_F32 ? 17 : 12); i++) {
+        const float c = tok_cost(wt, xt, TOK_SHAPES[i][0], TOK_SHAPES[i][1], out, ntok, in, k3k_cu_count());
+        if (i == 0 || c < *cycles) {
+            best = i;
+            *cycles = c;
+        }
+    }
+    return best;
+}
+
 template <int WT, int XT>
 int dispatch_tok(const TokArgs &a, hipStream_t st)
 {
-    /* (row tiles, groups of 8 tokens); the last five are ever the cheapest for fp32 weights only */
-    static const int shapes[][2] = {{1, 1}, {1, 2}, {2, 1}, {2, 2}, {2, 4}, {3, 1}, {3, 2}, {3, 4}, {4, 1},
-                                    {4, 2}, {4, 4}, {4, 8}, {1, 3}, {1, 4}, {1, 5}, {1, 6}, {1, 8}};
-    int best = 0;
-    float bc = 0;
-    for (int i = 0; i < (WT == TOK_F32 ? 17 : 12); i++) {
-        const float c = tok_cost(WT, XT, shapes[i][0], shapes[i][1], a.out, a.ntok, a.in, k3k_cu_count());
-        if (i == 0 || c < bc) {
-            best = i;
-            bc = c;
-        }
-    }
+    float c;
+    const int best = tok_pick(WT, XT, a.out, a.ntok, a.in, &c);
     if constexpr (WT == TOK_F32) {
         switch (best) {
         case 12: return launch_tok<WT, XT, 0, 1, 3>(a, st);
@@ -750,6 +758,24 @@ extern "C" int k3k_tok_mx_ok(const uint16_t *xhi, const uint16_t *xlo, const voi
     uint32_t lo;
     return ntok > 2 && in % 32 == 0 && in < (1 << 22) && ((uintptr_t)packed & 15) == 0 &&
            terms_ok(xhi, xlo, in, ntok, &lo);
+}
+
+/* Whether it is the faster kernel for three tokens and more. The streaming kernel (k3_mx.hip), whose
+ * workgroups are tiles of 16 rows x 16 tokens with a wave per four steps of 128 columns, is it where K is
+ * short, since a wave here takes at least 128 columns of K and the others idle. Two terms: up to 512
+ * columns, and up to 1152 where its tiles are about one to five per CU (168 tokens of 416 -> 630 6.8 us
+ * there and 9.6 here; 11 of 864 -> 7633 7.0 and 9.8; 29 of 768 -> 14889, 7 per CU, 17.1 and 13.0). One
+ * term, for which it does half the work and this kernel the same: wherever its tiles' steps past the
+ * seventh, 330 cycles each on a CU, are cheaper than the launch here (179 tokens of 416 -> 5503 13.3 and
+ * 27.3; 172 of 1728 -> 2790 20.4 and 23.3; 144 of 7424 -> 2943 73.6 and 34.6). Over 900 products the one
+ * taken is on average 0.8 % (two terms, at most 14) and 2.3 % (one, at most 26) slower than the faster one. */
+extern "C" int k3k_tok_mx_pays(int in, int out, int ntok, int terms)
+{
+    const long tiles = (long)((out + 15) / 16) * ((ntok + 15) / 16), cus = k3k_cu_count() > 0 ? k3k_cu_count() : 1;
+    if (terms == 2) return in > 512 && (in > 1152 || 5 * tiles < 4 * cus || tiles > 5 * cus);
+    float c;
+    tok_pick(TOK_MX, 1, out, ntok, in, &c);
+    return 330.f * (float)tiles * (float)((in + 127) / 128 - 7) >= c * (float)cus;
 }
 
 extern "C" int k3k_tok_mx(float *y, const uint16_t *xhi, const uint16_t *xlo, const void *packed, const uint8_t *scales,

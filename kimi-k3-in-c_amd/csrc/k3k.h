@@ -217,6 +217,7 @@ int k3k_tok_terms(float *y, int ldy, int accumulate, const uint16_t *W, const ui
 /* MXFP4 weights (row-major, group 32) times three tokens and more given as two bf16 terms, or one (xlo NULL), where
  * k3k_tok_mx_ok holds (in % 32 == 0, packed 16-byte aligned, the terms within 2 GiB of each other). */
 int k3k_tok_mx_ok(const uint16_t *xhi, const uint16_t *xlo, const void *packed, int in, int ntok);
+int k3k_tok_mx_pays(int in, int out, int ntok, int terms);      /* and is the faster kernel */
 int k3k_tok_mx(float *y, const uint16_t *xhi, const uint16_t *xlo, const void *packed, const uint8_t *scales, int in,
                int out, int ntok, int ldy, void *stream);
 int k3k_gemv_q8(float *y, const float *x, const void *W, int in, int out, int ntok, int ldy,

@@ -42,7 +42,7 @@ def test_tok_matmul_edges(gpu, k3, bf16, T, inn, out):
 # (sizes that between them take every tile shape the products are launched with, the K waves with
 # several stages each)
 @pytest.mark.parametrize("bf16", [True, False])
-@pytest.mark.parametrize("T,inn,out", [(20, 1160, 19), (697, 1080, 38), (2, 1072, 4115), (395, 1032, 316), (677, 1064, 275),
+@pytest.mark.parametrize("T,inn,out", [(382, 1072, 17), (697, 1080, 38), (2, 1072, 4115), (395, 1032, 316), (677, 1064, 275),
                                        (3, 1056, 8205), (489, 1048, 369), (676, 1032, 372), (389, 1056, 619), (585, 1040, 633),
                                        (675, 1048, 1109), (686, 1072, 81), (674, 1088, 165), (629, 1048, 194), (680, 1048, 244),
                                        (618, 1048, 385), (675, 1056, 81), (682, 1056, 331), (691, 1048, 535), (617, 1032, 770),
@@ -51,13 +51,13 @@ def test_tok_matmul_shapes(gpu, k3, bf16, T, inn, out):
     test_tok_matmul_edges(gpu, k3, bf16, T, inn, out)
 
 
-@pytest.mark.parametrize("inn", [136, 137])
+@pytest.mark.parametrize("inn,out", [(136, 40), (137, 40), (136, 2000), (137, 2000)])
 @pytest.mark.parametrize("bf16", [True, False])
-def test_tok_matmul_nonfinite(gpu, k3, bf16, inn):
-    """Infinities and NaN in x and W, the largest finite x, subnormal x: what plain products
+def test_tok_matmul_nonfinite(gpu, k3, bf16, inn, out):
+    """(40 rows: on the vector units; 2000: on the matrix cores.) Infinities and NaN in x and W, the largest finite x, subnormal x: what plain products
     and sums give, element by element."""
-    T, out = 20, 40
-    say(f"case: non-finite operands bf16={bf16} in={inn}")
+    T = 20
+    say(f"case: non-finite operands bf16={bf16} in={inn} out={out}")
     Wb = k3.gen_bf16_normal(inn * out, 91, 0.0, 1.0).reshape(out, inn)
     Wb[3, 7], Wb[4, 9], Wb[5, 100] = 0x7F80, 0xFF80, 0x7FC0          # +inf, -inf, NaN
     Wb[6, :] = 0
@@ -122,7 +122,9 @@ def test_tok_matmul_nan_tokens_cost(gpu, k3, bf16, T, inn, out):
 
 
 @pytest.mark.parametrize("T,inn,out", [(1, 1, 3), (1, 7, 5), (1, 520, 40), (1, 513, 33), (1, 1001, 999), (1, 4099, 70), (1, 7169, 300),
-                                       (2, 520, 65), (5, 512, 40), (33, 1024, 129), (64, 264, 300)])
+                                       (2, 520, 65), (5, 512, 40), (33, 1024, 129), (64, 264, 300), (2, 1001, 9), (2, 1, 3), (3, 512, 7),
+                                       (4, 9, 8), (5, 7, 8), (5, 2056, 1), (7, 1030, 33), (2, 7168, 1000), (8, 7169, 530),
+                                       (9, 520, 680), (9, 520, 690), (2, 1000, 4096), (2, 1000, 4097)])
 def test_matmul_any_alignment(gpu, k3, T, inn, out):
     """Any row length, and x, W at any element: against fp64, and for one token bf16 weights give
     the bits of fp32 weights of the same values (the reference's invariant), at every alignment."""
