@@ -226,9 +226,11 @@ struct SelSmem {
  *    16, the final kernel of a workgroup per token took 225 us with them and 192 with the threshold, one
  *    token's 10.0 and 7.5 (up to 512 experts and 8 groups the two chains are as fast: 11.6 / 12.3 us
  *    for 64 tokens of 384, top 8, so they keep them);
- *  - else wave 0 alone: lane l holds the keys of experts l + 64 i (SW of them) and the
- *    largest of its keys; after each extraction the lane that held it drops the key and
- *    takes its next largest.
+ *  - else wave 0 alone: lane l holds the keys of experts l + 64 i (SW of them; of 32 their choices
+ *    only: 64 registers of keys spilled, and beside the spills the compiler kept a live register
+ *    in a copy made under a partial execution mask, which lost it for the other lanes) and the
+ *    largest of its keys; after each extraction the lane that held it drops the key and takes its
+ *    next largest.
  * Lane j of wave 0 keeps the j-th selected key. Uncertified logits that matter (selected,
  * i.e. a key at least the last selected one, or able to reach the selection) are listed in
  * expert order by ballots, recomputed by the whole workgroup with the reference's chain
@@ -399,16 +401,30 @@ __device__ uint64_t select_rounds(SelSmem<SW> &sm, const float *x, const float *
             if (need && slot < RF_LIST) sm.list[slot] = 64 * wv + lane;
             if (tid == 0) sm.nlist = min(total, RF_LIST);
         } else if (wv == 0) {
-            uint64_t key[SW];
+            constexpr bool FULL = SW <= 16;         /* whole keys in registers, else their choices */
+            uint64_t key[FULL ? SW : 1];
+            uint32_t kc[FULL ? 1 : SW];
             uint64_t head = 0ull;
+            /* the largest of kc, the lowest expert among equals */
+            auto largest = [&]() {
+                uint32_t h = 0u, at = 0u;
 #pragma unroll
-            for (int i = 0; i < SW; i++) {
-                const int e = lane + 64 * i;
-                const float c = sm.c[e];
-                key[i] = (e < n_experts && c > -INFINITY)
-                             ? ((uint64_t)choice_order(c) << 32) | (uint64_t)(0xffffffffu - (uint32_t)e)
-                             : 0ull;
-                head = head > key[i] ? head : key[i];
+                for (int i = 0; i < SW; i++) {
+                    at = kc[i] > h ? (uint32_t)i : at;
+                    h = kc[i] > h ? kc[i] : h;
+                }
+                return h ? ((uint64_t)h << 32) | (uint64_t)(0xffffffffu - (uint32_t)(lane + 64 * (int)at)) : 0ull;
+            };
+            if constexpr (FULL) {
+#pragma unroll
+                for (int i = 0; i < SW; i++) {
+                    key[i] = key_of(lane + 64 * i);
+                    head = head > key[i] ? head : key[i];
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < SW; i++) kc[i] = (uint32_t)(key_of(lane + 64 * i) >> 32);
+                head = largest();
             }
             uint32_t taken = 0u;                    /* bit i: key i was selected */
             int nsel = 0;
@@ -421,16 +437,24 @@ __device__ uint64_t select_rounds(SelSmem<SW> &sm, const float *x, const float *
                 last = m;
                 if (lane == j) mysel = m;
                 if (head == m) {
-                    uint64_t h2 = 0ull;
+                    if constexpr (FULL) {
+                        uint64_t h2 = 0ull;
 #pragma unroll
-                    for (int i = 0; i < SW; i++) {
-                        if (key[i] == m) {
-                            key[i] = 0ull;
-                            taken |= 1u << i;
+                        for (int i = 0; i < SW; i++) {
+                            if (key[i] == m) {
+                                key[i] = 0ull;
+                                taken |= 1u << i;
+                            }
+                            h2 = h2 > key[i] ? h2 : key[i];
                         }
-                        h2 = h2 > key[i] ? h2 : key[i];
+                        head = h2;
+                    } else {
+                        const uint32_t at = (0xffffffffu - (uint32_t)m) >> 6;
+                        taken |= 1u << at;
+#pragma unroll
+                        for (int i = 0; i < SW; i++) kc[i] = (uint32_t)i == at ? 0u : kc[i];
+                        head = largest();
                     }
-                    head = h2;
                 }
             }
             const float ckth = nsel > 0 ? key_choice(last) : -INFINITY;
