@@ -240,8 +240,8 @@ int k3d_matmul_bf16(float *y, const float *x, int ntok, const uint16_t *W, int i
 typedef struct {
     double *part;
     float *rbound;
-    int *nrecomp;
-    int *ctr;                   /* the final kernel's arrival counter, when it gathers, and the chunk it summed */
+    int *nrecomp;               /* recomputed logits per token, then the chunk that was summed */
+    int *ctr;                   /* the final kernel's arrival counter, when it gathers */
     int chunk;
     void *i8;                   /* scratch of the int8 partials (NULL: the fp64 ones) */
 } RtWs;
@@ -250,8 +250,8 @@ static void router_layout(Carve *c, RtWs *w, int T, int hidden, int n_experts, i
 {
     const size_t ks = (size_t)((hidden + chunk - 1) / chunk);
     w->chunk = chunk;
-    w->nrecomp = (int *)take(c, (size_t)T * 4);
-    w->ctr = (int *)take(c, 8);
+    w->nrecomp = (int *)take(c, ((size_t)T + 1) * 4);
+    w->ctr = (int *)take(c, 4);
     /* chunk partials, or (a few tokens) one 16-byte scored record per logit */
     w->part = (double *)take(c, (ks < 2 ? 2 : ks) * T * n_experts * 8);
     w->rbound = (float *)take(c, ks * T * n_experts * 4);
@@ -339,7 +339,7 @@ static int router_run(int *idx, float *wt, const float *x, int T, const float *W
                                   exc, stream)) {
         return fail("router_partial");
     }
-    if (k3k_router_final(idx, wt, w->nrecomp, w->ctr + 1, w->part, w->rbound, w->chunk, x, W, bias, T, hidden,
+    if (k3k_router_final(idx, wt, w->nrecomp, w->part, w->rbound, w->chunk, x, W, bias, T, hidden,
                          n_experts, topk, renorm, routed_scale, exc, gather ? &g : NULL, stream))
         return fail("router_final");
     return 0;
@@ -363,7 +363,7 @@ int k3d_router_partials(double *h_part, float *h_rbound, int *h_chunk, size_t ca
     RtWs w;
     int chunk = 0;
     router_layout(&c, &w, T, hidden, n_experts, hidden, 0);
-    if (k3k_d2h(&chunk, w.ctr + 1, 4, NULL) || k3k_sync(NULL)) return fail("router_partials");
+    if (k3k_d2h(&chunk, w.nrecomp + T, 4, NULL) || k3k_sync(NULL)) return fail("router_partials");
     if (chunk <= 0) return bad("k3d_router_partials: no router call has used the workspace");
     c.off = 0;
     router_layout(&c, &w, T, hidden, n_experts, chunk, 0);

@@ -739,10 +739,10 @@ __device__ void gather_block(const GatherDev &g);
  * from router_small_kernel's scored records (PRE) or from the chunk partials, summed in
  * k order and certified here (certify_score) -- into LDS; then select_rounds (wave 0
  * selects, the workgroup recomputes what matters) and select_weight; renormalise and
- * scale (k3_ops.c:459-475). nrecomp[t] (optional) counts recomputes, *used (optional) is the chunk
+ * scale (k3_ops.c:459-475). nrecomp[t] (optional) counts recomputes, nrecomp[T] is the chunk
  * width. KB: chunk partials loaded per batch. */
 template <int SL, int SW, int KB, bool PRE, bool GATHER = false>
-__global__ __launch_bounds__(KB > 32 ? 512 : 1024) void router_final_kernel(int *idx, float *wt, int *nrecomp, int *used,
+__global__ __launch_bounds__(KB > 32 ? 512 : 1024) void router_final_kernel(int *idx, float *wt, int *nrecomp,
                                                             const double *part,
                                                             const float *rbound, int ksplit,
                                                             int chunk, const float *x,
@@ -756,7 +756,6 @@ __global__ __launch_bounds__(KB > 32 ? 512 : 1024) void router_final_kernel(int 
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int nthr = blockDim.x;
     const int t = blockIdx.x;
-    if (used && t == 0 && tid == 0) *used = chunk;
 #pragma unroll
     for (int i = 0; i < SL; i++) {
         const int e = tid + nthr * i;
@@ -813,7 +812,10 @@ __global__ __launch_bounds__(KB > 32 ? 512 : 1024) void router_final_kernel(int 
                 idx[(size_t)t * topk + lane] = id >= 0 ? id : 0;
             wt[(size_t)t * topk + lane] = w;
         }
-        if (nrecomp && lane == 0) nrecomp[t] = nre;
+        if (nrecomp && lane == 0) {
+            nrecomp[t] = nre;
+            if (!PRE && t == 0) nrecomp[T] = chunk;
+        }
     }
     if constexpr (GATHER) {
         /* The workgroup that finishes last runs the gather over every token's idx. Each
@@ -899,7 +901,7 @@ __device__ double chain_wave(double (*ring)[RF_BLK], const float *w, const float
  * 896: 23.6 us here, 19.6 there). What bounds it: the partials (12 bytes per chunk and logit) for
  * many tokens, the chain of loads, certification and selection of one wave for few. */
 template <int SL>
-__global__ __launch_bounds__(256) void router_final_wave_kernel(int *idx, float *wt, int *nrecomp, int *used, const double *part,
+__global__ __launch_bounds__(256) void router_final_wave_kernel(int *idx, float *wt, int *nrecomp, const double *part,
                                                                 const float *rbound, int ksplit, int chunk,
                                                                 const float *x, const float *W, const float *bias, int T,
                                                                 int hidden, int n_experts, int topk, int renorm,
@@ -911,7 +913,6 @@ __global__ __launch_bounds__(256) void router_final_wave_kernel(int *idx, float 
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int t = (int)blockIdx.x * 4 + wv;
     if (t >= T) return;
-    if (used && t == 0 && lane == 0) *used = chunk;
     int en[SL];                                        /* the lane's experts, the last one past the end */
     double Q[SL], bs[SL];
 #pragma unroll
@@ -1096,7 +1097,10 @@ __global__ __launch_bounds__(256) void router_final_wave_kernel(int *idx, float 
         idx[(size_t)t * topk + lane] = id >= 0 ? id : 0;
         wt[(size_t)t * topk + lane] = w;
     }
-    if (nrecomp && lane == 0) nrecomp[t] = nre;
+    if (nrecomp && lane == 0) {
+        nrecomp[t] = nre;
+        if (t == 0) nrecomp[T] = chunk;
+    }
 }
 
 /* ---- expert-major gather -----------------------------------------------------------
@@ -1762,7 +1766,7 @@ static GatherDev gather_dev(const K3kGatherArgs *g, const int *idx, int N, int n
     return d;
 }
 
-extern "C" int k3k_router_final(int *idx, float *wt, int *nrecomp, int *used, const double *part,
+extern "C" int k3k_router_final(int *idx, float *wt, int *nrecomp, const double *part,
                                 const float *rbound, int chunk, const float *x, const float *W,
                                 const float *bias, int T, int hidden, int n_experts, int topk,
                                 int renorm, float routed_scale, const K3kExc *exc,
@@ -1785,7 +1789,7 @@ extern "C" int k3k_router_final(int *idx, float *wt, int *nrecomp, int *used, co
             return k3k_fail("router_final: the gather cannot run here", hipErrorInvalidValue);
 #define K3_RFG(SL, SW, KB)                                                                           \
     hipLaunchKernelGGL((router_final_kernel<SL, SW, KB, false, true>), dim3(T), dim3(1024), 0, st, idx, wt, \
-                       nrecomp, used, part, rbound, ks, chunk, x, W, bias, T, hidden, n_experts, topk, renorm, \
+                       nrecomp, part, rbound, ks, chunk, x, W, bias, T, hidden, n_experts, topk, renorm, \
                        routed_scale, e, gd)
         if (n_experts <= 512 && ks <= 16) K3_RFG(1, 8, 16);
         else if (n_experts <= 512) K3_RFG(1, 8, RF_KB);
@@ -1804,12 +1808,12 @@ extern "C" int k3k_router_final(int *idx, float *wt, int *nrecomp, int *used, co
      * over SW keys per lane: 8 up to 512 experts, 16 up to 1024, else 32 (each pick rescans
      * the picking lane's SW keys). */
 #define K3_RF(SL, SW, KB, PRE, NT)                                                                  \
-    hipLaunchKernelGGL((router_final_kernel<SL, SW, KB, PRE>), dim3(T), dim3(NT), 0, st, idx, wt, nrecomp, used, \
+    hipLaunchKernelGGL((router_final_kernel<SL, SW, KB, PRE>), dim3(T), dim3(NT), 0, st, idx, wt, nrecomp, \
                        part, rbound, ks, chunk, x, W, bias, T, hidden, n_experts, topk, renorm,        \
                        routed_scale, e, gd)
 #define K3_RFW(SL)                                                                                   \
     hipLaunchKernelGGL((router_final_wave_kernel<SL>), dim3((unsigned)((T + 3) / 4)), dim3(256), 0, st, idx, wt, \
-                       nrecomp, used, part, rbound, ks, chunk, x, W, bias, T, hidden, n_experts, topk, renorm, \
+                       nrecomp, part, rbound, ks, chunk, x, W, bias, T, hidden, n_experts, topk, renorm, \
                        routed_scale, e)
     /* many tokens: a wave each (router_final_wave_kernel) */
     if (!pre && T >= 3 * k3k_cu_count() && n_experts <= 1024) {

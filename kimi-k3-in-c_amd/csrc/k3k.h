@@ -229,8 +229,8 @@ int k3k_gemv_q8(float *y, const float *x, const void *W, int in, int out, int nt
  * rbound[k][t][e] on its intermediate magnitudes. k3k_router_final: the certified logit
  * (the reference's sequential fp64 chain recomputed where the bound cannot decide the
  * fp32 rounding and the logit matters), sigmoid with the host libm's expf, biased
- * first-strict-max top-k, renorm, scale -> idx/wt [T][topk]; nrecomp [T] (may be NULL)
- * receives the number of recomputed logits per token, *used (may be NULL) the chunk width. */
+ * first-strict-max top-k, renorm, scale -> idx/wt [T][topk]; nrecomp [T + 1] (may be
+ * NULL) receives the number of recomputed logits per token, then the chunk width. */
 int k3k_router_chunk(int T, int hidden, int n_experts);
 /* 1 when k3k_router_partial scores and certifies the logits itself (a few tokens): its
  * part then holds one 16-byte record per logit, which a selecting decode gate/up reads. */
@@ -265,7 +265,7 @@ int k3k_router_partial_i8(double *part, float *rbound, void *scratch, const floa
                           const float *W, int hidden, int n_experts, int chunk, int *ctr, int *idx,
                           int n_idx, void *stream);
 /* gather (may be NULL): also run the gather of idx, as k3k_gather would. */
-int k3k_router_final(int *idx, float *wt, int *nrecomp, int *used, const double *part, const float *rbound,
+int k3k_router_final(int *idx, float *wt, int *nrecomp, const double *part, const float *rbound,
                      int chunk, const float *x, const float *W, const float *bias, int T,
                      int hidden, int n_experts, int topk, int renorm, float routed_scale,
                      const K3kExc *exc, const K3kGatherArgs *gather, void *stream);
