@@ -209,7 +209,7 @@ struct SelSmem {
  * above -inf, none left: idx 0, weight 0; k3_ops.c:459-467) over the scored experts in sm.
  * Keys are unique (the expert's index in the low word), so the selection is the topk
  * largest keys in order, however they are found:
- *  - by threshold, past 512 experts, when the ng = ceil(n_experts / 64) groups of 64 experts fit
+ *  - by threshold, past 512 experts and for more than 4, when the ng = ceil(n_experts / 64) groups of 64 experts fit
  *    the workgroup's waves and there are at least topk rows of 16 experts: wave g
  *    reduces its rows to their largest choices; wave 0 takes the topk-th largest of the (at
  *    most 64) row maxima, each lane counting the maxima above its own; at least topk keys lie
@@ -217,7 +217,8 @@ struct SelSmem {
  *    order they are few (about 1.3 topk). They are packed into LDS, and wave 0 ranks them by
  *    counting, a lane per candidate;
  *  - two levels, when that leaves more than 64 candidates (many equal choices, or choices in
- *    order of their expert) or there are too few rows, and ng * topk <= 256: wave g takes the
+ *    order of their expert) or there are too few rows, or for up to 4 (14 tokens of 823 experts, top 1:
+ *    26.8 us, 28.2 with the threshold; top 4 27.9 and 28.5, top 6 28.9 and 28.5), and ng * topk <= 256: wave g takes the
  *    topk largest keys of group g (one key per lane, each extraction one wave maximum,
  *    wave_max_key_fast), then wave 0
  *    the topk largest of those ng * topk candidates (one to four per lane: a lane holds
@@ -252,7 +253,7 @@ __device__ uint64_t select_rounds(SelSmem<SW> &sm, const float *x, const float *
                                                 : 0ull;
     };
     const int nrow = ng * 4;                        /* rows of 16 experts, at most 64 */
-    const bool thr = SW == 16 && two && ng > 8 && nrow >= topk;
+    const bool thr = SW == 16 && two && ng > 8 && nrow >= topk && topk > 4;
     nre = 0;
     uint64_t mysel = 0ull;
     for (int round = 0; round <= n_experts; round++) {
